@@ -234,6 +234,46 @@ __device__ __forceinline__ void left_shift_sv(uint32_t v[8], uint32_t shift)
 
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 
+// n / d and n % d for a divisor d >= 1 with m = 0xFFFFFFFF / d from the host:
+// mulhi(n, m) is q or q - 1, one correction makes it exact (a handful of
+// instructions instead of a full division)
+struct UDiv {
+  uint32_t d, m;
+  __device__ __forceinline__ uint32_t div(uint32_t n, uint32_t& r) const
+  {
+    uint32_t q = __umulhi(n, m);
+    r = n - q * d;
+    if (r >= d) {
+      ++q;
+      r -= d;
+    }
+    return q;
+  }
+};
+static inline UDiv udiv(uint32_t d) { return UDiv{d, 0xFFFFFFFFu / d}; }
+
+// Bit 7 of each byte set where that byte of x >= the byte of t (unsigned; t holds
+// one value in all four bytes).  Where the high bits differ they decide; where they
+// agree, (x | 0x80) - (t & 0x7F) carries the comparison of the low 7 bits into
+// bit 7 without borrowing from the next byte.
+__device__ __forceinline__ uint32_t bytes_ge(uint32_t x, uint32_t t)
+{
+  const uint32_t H = 0x80808080u;
+  const uint32_t d = (x | H) - (t & ~H);
+  return ((x & ~t) | (~(x ^ t) & d)) & H;
+}
+
+// Pass flags (bit 7 of each byte) of 16 int8 log-odds against thr: signed bytes
+// compare as unsigned ones once their sign bits are flipped.
+__device__ __forceinline__ void prob_pass(const uint4& v, int thr, uint32_t f[4])
+{
+  const uint32_t t = ((uint32_t)(uint8_t)thr ^ 0x80u) * 0x01010101u, s = 0x80808080u;
+  f[0] = bytes_ge(v.x ^ s, t);
+  f[1] = bytes_ge(v.y ^ s, t);
+  f[2] = bytes_ge(v.z ^ s, t);
+  f[3] = bytes_ge(v.w ^ s, t);
+}
+
 // Runs of consecutive lanes with in set and equal (idx, meaning): returns the run
 // length for the first lane of each run and 0 for every other lane.  Neighbouring
 // points of an image often share a voxel; one shuffle and one ballot find the runs

@@ -152,28 +152,6 @@ __global__ void __launch_bounds__(256) k_collide(uint8_t* __restrict__ a, const 
 
 constexpr int kLoadsInFlight = 4;  // per lane, in the kernels that stream a ProbVoxelMap
 
-// Bit 7 of each byte set where that byte of x >= the byte of t (unsigned; t holds
-// one value in all four bytes).  Where the high bits differ they decide; where they
-// agree, (x | 0x80) - (t & 0x7F) carries the comparison of the low 7 bits into
-// bit 7 without borrowing from the next byte.
-__device__ __forceinline__ uint32_t bytes_ge(uint32_t x, uint32_t t)
-{
-  const uint32_t H = 0x80808080u;
-  const uint32_t d = (x | H) - (t & ~H);
-  return ((x & ~t) | (~(x ^ t) & d)) & H;
-}
-
-// Pass flags (bit 7 of each byte) of 16 int8 log-odds against thr: signed bytes
-// compare as unsigned ones once their sign bits are flipped.
-__device__ __forceinline__ void prob_pass(const uint4& v, int thr, uint32_t f[4])
-{
-  const uint32_t t = ((uint32_t)(uint8_t)thr ^ 0x80u) * 0x01010101u, s = 0x80808080u;
-  f[0] = bytes_ge(v.x ^ s, t);
-  f[1] = bytes_ge(v.y ^ s, t);
-  f[2] = bytes_ge(v.z ^ s, t);
-  f[3] = bytes_ge(v.w ^ s, t);
-}
-
 // The passing voxels of a wave's 64 lanes x 16 voxels, spread over its lanes: each
 // lane lists its own (offset lane * 16 + voxel) in the wave's LDS list at its prefix
 // position, then lane t visits entries t, t + 64, ...  A lane whose 16 voxels all

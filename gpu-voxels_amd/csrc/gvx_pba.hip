@@ -497,24 +497,6 @@ constexpr int YS = YT + 1;             // LDS words per staged line (odd: transp
 constexpr int YW_WAVES = 8;
 static_assert(32 % YW_WAVES == 0, "a wave's staged rows r = w + YW_WAVES i share word (YW_WAVES i) / 32");
 constexpr int YW_RPS = YB / YW_WAVES;  // output rows searched per wave (lanes = the 64 lines)
-// n / d and n % d for a wave-uniform divisor d >= 1 with m = 0xFFFFFFFF / d from the
-// host: mulhi(n, m) is q or q - 1, one correction makes it exact (a handful of
-// scalar instructions instead of a full division)
-struct UDiv {
-  uint32_t d, m;
-  __device__ __forceinline__ uint32_t div(uint32_t n, uint32_t& r) const
-  {
-    uint32_t q = __umulhi(n, m);
-    r = n - q * d;
-    if (r >= d) {
-      ++q;
-      r -= d;
-    }
-    return q;
-  }
-};
-static inline UDiv udiv(uint32_t d) { return UDiv{d, 0xFFFFFFFFu / d}; }
-
 // The windowed y pass writes each voxel's site relative to the voxel, 2 bytes:
 // (y_site - y + 64) | (z_site - z + 64) << 7.  A resolved window search finds its
 // site within WIN_R rows and at a cost below (WIN_R + 1)^2, so both offsets lie in
@@ -1227,31 +1209,86 @@ __global__ void k_dist_sq(const uint32_t* __restrict__ map, const uint32_t* __re
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const uint64_t id = idx ? idx[i] : i;
+    const uint64_t id = idx[i];
     out[i] = dist_sq(map[id], id, dx, dy, uninit);
   }
 }
 
-__global__ void k_dist_metric(const uint32_t* __restrict__ map, uint64_t n, uint32_t dx, uint32_t dy, uint32_t uninit,
-                              float side, float* __restrict__ out)
+// The read-out of every voxel in index order: squared distances (int32) or metric
+// ones (float).  A thread takes 4 consecutive voxels with one 16-byte load; the
+// coordinates of the first come from two reciprocal divisions, the others step (the
+// index fits 32 bits: a map has at most 2^32 voxels).  HBM bound: 8 bytes a voxel;
+// one voxel per thread with two 64-bit divisions was VALU bound (1.5 instructions
+// per byte moved).  vec: out is 16-byte aligned.
+template <bool METRIC>
+__global__ void __launch_bounds__(256) k_dist_all(const uint32_t* __restrict__ map, uint64_t n, UDiv dxd, UDiv dyd,
+                                                  uint32_t uninit, float side, void* __restrict__ out, bool vec)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const int32_t d = dist_sq(map[i], i, dx, dy, uninit);
-    out[i] = d == INT32_MAX ? 3.402823466e+38f : sqrtf((float)d) * side;
+  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; 4 * q < n; q += stride) {
+    uint32_t x, y;
+    uint32_t z = dyd.div(dxd.div((uint32_t)(4 * q), x), y);
+    const uint4 v = reinterpret_cast<const uint4*>(map)[q];  // allocations are padded to 256 bytes
+    const uint32_t raw[4] = {v.x, v.y, v.z, v.w};
+    uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int32_t ex = (int32_t)x - (int32_t)(raw[k] & 0x3FF), ey = (int32_t)y - (int32_t)((raw[k] >> 10) & 0x3FF),
+                    ez = (int32_t)z - (int32_t)(raw[k] >> 20);
+      const int32_t d = raw[k] == uninit ? INT32_MAX : ex * ex + ey * ey + ez * ez;
+      if (METRIC) r[k] = __float_as_uint(d == INT32_MAX ? 3.402823466e+38f : sqrtf((float)d) * side);
+      else r[k] = (uint32_t)d;
+      if (++x == dxd.d) {
+        x = 0;
+        if (++y == dyd.d) {
+          y = 0;
+          ++z;
+        }
+      }
+    }
+    uint32_t* o = reinterpret_cast<uint32_t*>(out) + 4 * q;
+    if (vec && 4 * q + 4 <= n) {
+      *reinterpret_cast<uint4*>(o) = make_uint4(r[0], r[1], r[2], r[3]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (4 * q + k < n) o[k] = r[k];
+    }
   }
 }
 
-// mergeOccupied (DistanceVoxelMap.hpp:109-136 / DistanceVoxelMap.h:92-134)
-__global__ void k_merge_occupied(uint32_t* __restrict__ dist, const int8_t* __restrict__ prob, uint64_t n, uint32_t dx,
-                                 uint32_t dy, uint32_t ox, uint32_t oy, uint32_t oz, int thr)
+// mergeOccupied (DistanceVoxelMap.hpp:109-136 / DistanceVoxelMap.h:92-134): log-odds
+// at or above thr write their coordinates.  A lane tests 16 log-odds of one 16-byte
+// load 4 bytes at a time and visits only the passing ones; the HBM bytes it needs are
+// 1 per voxel and the written ones.  One voxel per thread with two 64-bit divisions
+// was issue bound.
+__global__ void __launch_bounds__(256) k_merge_occupied(uint32_t* __restrict__ dist, const uint8_t* __restrict__ prob,
+                                                        uint64_t n, UDiv dxd, UDiv dyd, uint32_t ox, uint32_t oy,
+                                                        uint32_t oz, int thr)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    if ((int)prob[i] > thr) {
-      const uint32_t x = (uint32_t)(i % dx), y = (uint32_t)((i / dx) % dy), z = (uint32_t)(i / ((uint64_t)dx * dy));
-      dist[i] = (x + ox) | ((y + oy) << 10) | ((z + oz) << 20);
-    }
+  for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; 16 * c < n; c += stride) {
+    uint32_t f[4];
+    prob_pass(reinterpret_cast<const uint4*>(prob)[c], thr, f);  // allocations are padded to 256 bytes
+    if ((f[0] | f[1] | f[2] | f[3]) == 0u) continue;
+    uint32_t x0, y0;
+    const uint32_t z0 = dyd.div(dxd.div((uint32_t)(16 * c), x0), y0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      for (uint32_t m = f[q]; m != 0u; m &= m - 1u) {
+        const uint32_t o = (uint32_t)q * 4 + ((uint32_t)__builtin_ctz(m) >> 3);
+        const uint64_t i = 16 * c + o;
+        if (i >= n) break;
+        uint32_t x = x0 + o, y = y0, z = z0;
+        while (x >= dxd.d) {
+          x -= dxd.d;
+          if (++y == dyd.d) {
+            y = 0;
+            ++z;
+          }
+        }
+        dist[i] = (x + ox) | ((y + oy) << 10) | ((z + oz) << 20);
+      }
   }
 }
 
@@ -1295,6 +1332,8 @@ __global__ void __launch_bounds__(EX_BLOCK) k_exact(uint32_t* __restrict__ map, 
   }
   if (active && found && best < cur) map[id] = (uint32_t)bo[0] | ((uint32_t)bo[1] << 10) | ((uint32_t)bo[2] << 20);
 }
+
+static unsigned dist_all_grid(uint64_t n) { return grid_for((n + 3) / 4, 256, 32768); }
 
 struct PbaScratch {
   void* zs = nullptr;     // z pass output, uint16 per voxel
@@ -1593,11 +1632,14 @@ int gvx_dist_merge_occupied(gvx_map dist, gvx_map prob, const uint32_t offset[3]
     return fail(GVX_ERR_DIM_MISMATCH, "mergeOccupied: map dimensions differ");
   std::unique_lock<std::recursive_mutex> g1(dist->mu, std::defer_lock), g2(prob->mu, std::defer_lock);
   std::lock(g1, g2);
-  hipLaunchKernelGGL(k_merge_occupied, dim3(grid_for(dist->n, 256, 8192)), dim3(256), 0, rt().stream,
-                     (uint32_t*)dist->data, (const int8_t*)prob->data, dist->n, dist->dims[0], dist->dims[1],
-                     offset ? offset[0] : 0u, offset ? offset[1] : 0u, offset ? offset[2] : 0u,
-                     (int)float_to_probability(threshold));
-  GVX_HIP(hipGetLastError());
+  const int thr = (int)float_to_probability(threshold) + 1;  // strictly above the threshold
+  if (thr <= PROB_MAX) {
+    hipLaunchKernelGGL(k_merge_occupied, dim3(grid_for((dist->n + 15) / 16, 256, 16384)), dim3(256), 0, rt().stream,
+                       (uint32_t*)dist->data, (const uint8_t*)prob->data, dist->n, udiv(dist->dims[0]),
+                       udiv(dist->dims[1]), offset ? offset[0] : 0u, offset ? offset[1] : 0u, offset ? offset[2] : 0u,
+                       thr);
+    GVX_HIP(hipGetLastError());
+  }
   return sync();
 }
 
@@ -1649,8 +1691,13 @@ int gvx_dist_squared(gvx_map m, const uint32_t* idx, uint64_t n, int32_t* out, i
     for (uint64_t i = 0; i < n; ++i)
       if (hp[i] >= m->n) return fail(GVX_ERR_BAD_ARG, "voxel index out of range");
   }
-  hipLaunchKernelGGL(k_dist_sq, dim3(grid_for(n, 256, 8192)), dim3(256), 0, rt().stream, (const uint32_t*)m->data,
-                     didx, n, m->dims[0], m->dims[1], m->uninit, dout);
+  if (didx)
+    hipLaunchKernelGGL(k_dist_sq, dim3(grid_for(n, 256, 8192)), dim3(256), 0, rt().stream, (const uint32_t*)m->data,
+                       didx, n, m->dims[0], m->dims[1], m->uninit, dout);
+  else
+    hipLaunchKernelGGL(k_dist_all<false>, dim3(dist_all_grid(n)), dim3(256), 0, rt().stream,
+                       (const uint32_t*)m->data, n, udiv(m->dims[0]), udiv(m->dims[1]), m->uninit, m->side,
+                       (void*)dout, ((uintptr_t)dout & 15) == 0);
   GVX_HIP(hipGetLastError());
   if (mem == GVX_MEM_HOST) GVX_HIP(hipMemcpyAsync(out, dout, n * 4, hipMemcpyDeviceToHost, rt().stream));
   return sync();
@@ -1668,8 +1715,9 @@ int gvx_dist_metric(gvx_map m, float* out, int mem)
     GVX_CHECK(stage_reserve(m->n * 4, &st));
     dout = (float*)st;
   }
-  hipLaunchKernelGGL(k_dist_metric, dim3(grid_for(m->n, 256, 8192)), dim3(256), 0, rt().stream,
-                     (const uint32_t*)m->data, m->n, m->dims[0], m->dims[1], m->uninit, m->side, dout);
+  hipLaunchKernelGGL(k_dist_all<true>, dim3(dist_all_grid(m->n)), dim3(256), 0, rt().stream,
+                     (const uint32_t*)m->data, m->n, udiv(m->dims[0]), udiv(m->dims[1]), m->uninit, m->side,
+                     (void*)dout, ((uintptr_t)dout & 15) == 0);
   GVX_HIP(hipGetLastError());
   if (mem == GVX_MEM_HOST) GVX_HIP(hipMemcpyAsync(out, dout, m->n * 4, hipMemcpyDeviceToHost, rt().stream));
   return sync();
