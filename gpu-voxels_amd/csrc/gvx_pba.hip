@@ -27,33 +27,38 @@ namespace gvx {
 constexpr uint16_t ZNONE = 0xFFFF;
 
 // ---------------------------------------------------------------- z pass
-// Block = 64 columns (lanes = consecutive (x, y) columns) x ZP waves; wave w takes
-// the z range [128 w, 128 w + 128) of every column: its occupancy as 4 register
-// words (all 128 loads issued before any is used).  The words of all waves meet in
+// Block = 64 columns (x range xr, row y; lanes = consecutive x) x W / ZWP waves; wave w
+// takes the z range [32 ZWP w, 32 ZWP (w + 1)) of every column: its occupancy as ZWP
+// register words (all loads issued before any is used).  The words of all waves meet in
 // LDS, so each wave also knows the nearest obstacle below and above its range,
 // and writes the nearest obstacle z (ties to the lower z) of its range as uint16.
+// ZWP = 4 keeps 128 loads a lane in flight; small maps, whose few columns would leave
+// most of the chip idle, take ZWP = 1 (four times the waves: 128^3 ZTIME).
 // FULL: dz == 32 * W, every load unconditional so the compiler keeps many in flight.
-// With dx % 64 == 0, colm[(y / 32) * (dx / 64) + x / 64] gets bit y % 32 when the
-// 64 columns (x, y) of that row segment were stored (one of them holds an obstacle);
-// the other segments are not stored.  Other widths store every column.
-// tflags[x / 64] gets bit y / tile_rows for every column (x, y) holding an
-// obstacle: the y pass skips (x range, row tile) blocks without one.
-// xcnt[x / 64] counts the obstacles of each 64-column x range (the y pass's density test).
-constexpr int ZWP = 4;  // occupancy words (of 32 z) per wave
-template <int W, bool FULL>
+// flags (null: every column is stored and nothing is flagged):
+// colm[(y / 32) * nxr + xr] gets bit y % 32 when the 64 columns of that row segment
+// were stored (one of them holds an obstacle); the other segments are not stored.
+// tflags[xr] gets bit y / tile_rows for every row holding an obstacle: the y pass skips
+// (x range, row tile) blocks without one.  xcnt[xr] counts the obstacles of each x
+// range and xcnt[16 + xr] its (row, 128 z) cells of 64 columns without one: few empty
+// cells tell an evenly filled range from one whose obstacles sit on a few surfaces.
+constexpr int ZCELL = 4;  // words (of 32 z) per cell
+template <int W, bool FULL, int ZWP>
 __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __restrict__ map,
                                                           uint16_t* __restrict__ zs, uint32_t* __restrict__ tflags,
                                                           uint32_t* __restrict__ colm, uint32_t* __restrict__ xcnt,
                                                           uint32_t tile_rows, uint32_t dx, uint32_t dy, uint32_t dz,
-                                                          uint32_t uninit)
+                                                          UDiv nxrd, uint32_t uninit)
 {
   static_assert(W % ZWP == 0, "whole parts");
   __shared__ uint32_t sb[W][64];  // occupancy word w of the 64 columns
   const uint32_t lane = threadIdx.x & 63, part = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint64_t col = (uint64_t)blockIdx.x * 64 + lane;
-  const bool cin = col < (uint64_t)dx * dy;
+  uint32_t xr;
+  const uint32_t cy = nxrd.div(blockIdx.x, xr), cx = xr * 64 + lane;
+  const bool cin = cx < dx;
+  const uint64_t col = (uint64_t)cy * dx + (cin ? cx : dx - 1);
   const uint64_t layer = (uint64_t)dx * dy;
-  const uint32_t* __restrict__ p = map + (cin ? col : 0);
+  const uint32_t* __restrict__ p = map + col;
   uint32_t bits[ZWP];
 #pragma unroll
   for (int i = 0; i < ZWP; ++i) {
@@ -90,12 +95,11 @@ __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __rest
   uint32_t any = last != 0xFFFFu || after != 0xFFFFu ? 1u : 0u;
 #pragma unroll
   for (int i = 0; i < ZWP; ++i) any |= bits[i];
-  // with dx % 64 == 0 a block is 64 columns of one row: when none of them holds an
-  // obstacle nothing is stored (its segment's bit in colm stays clear and the y
-  // pass never reads it); with one, all 64 are, so stores stay whole rows
-  const bool seg = dx % 64 == 0;
+  // when none of the 64 columns holds an obstacle nothing is stored (the segment's bit
+  // in colm stays clear and the y pass never reads it); with one, all 64 are, so stores
+  // stay whole rows
   const bool wave_any = wave_ballot(any != 0u) != 0ull;
-  if (cin && (!seg || wave_any)) {
+  if (cin && (!tflags || wave_any)) {
     uint16_t* __restrict__ o = zs + col;
 #pragma unroll
     for (int i = 0; i < ZWP; ++i) {
@@ -120,21 +124,26 @@ __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __rest
       }
     }
   }
-  if (part != 0 || !cin) return;
-  uint32_t nob = 0;
-  for (int w = 0; w < W; ++w) nob += (uint32_t)__popc(sb[w][lane]);
-  const uint32_t c32 = (uint32_t)col, cx = c32 % dx, cy = c32 / dx;  // col < 2^20
-  const uint32_t fw = cx / 64, fb = 1u << (cy / tile_rows);
-  if (seg) {  // the block's 64 columns share one flag bit and one segment bit: one atomic each
-    for (int o = 32; o > 0; o >>= 1) nob += (uint32_t)__shfl_xor((int)nob, o, 64);
-    if (lane == 0 && wave_any) {
-      atomicOr(tflags + fw, fb);
-      atomicOr(colm + (uint64_t)(cy >> 5) * (dx / 64) + cx / 64, 1u << (cy & 31));
-      atomicAdd(xcnt + fw, nob);
+  if (part != 0 || !tflags) return;
+  uint32_t nob = 0, empty = 0;
+  for (int c = 0; c < W / ZCELL; ++c) {
+    uint32_t m = 0;
+    for (int i = 0; i < ZCELL; ++i) {
+      const uint32_t v = sb[c * ZCELL + i][lane];
+      nob += (uint32_t)__popc(v);
+      m |= v;
     }
-  } else if (any) {
-    atomicOr(tflags + fw, fb);
-    atomicAdd(xcnt + fw, nob);
+    if ((uint32_t)(c * ZCELL * 32) < dz && wave_ballot(m != 0u) == 0ull) ++empty;
+  }
+  // the block's 64 columns share one flag bit and one segment bit: one atomic each
+  for (int o = 32; o > 0; o >>= 1) nob += (uint32_t)__shfl_xor((int)nob, o, 64);
+  if (lane == 0) {
+    if (wave_any) {
+      atomicOr(tflags + xr, 1u << (cy / tile_rows));
+      atomicOr(colm + (uint64_t)(cy >> 5) * nxrd.d + xr, 1u << (cy & 31));
+      atomicAdd(xcnt + xr, nob);
+    }
+    if (empty) atomicAdd(xcnt + 16 + xr, empty);
   }
 }
 
@@ -195,6 +204,12 @@ constexpr int TX = GVX_PBA_TX;    // x pass: positions per tile (4 TX-byte row s
 constexpr int RK = GVX_PBA_RK;    // stack entries per line held in LDS
 static_assert(RK >= 4 && (RK & (RK - 1)) == 0 && TX >= 4 && 64 % TX == 0 && TYR <= 32, "tile shape");
 
+__device__ __forceinline__ void wave_lds_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 __device__ __forceinline__ int32_t sq24(int32_t v) { return __mul24(v, v); }
 
 // raw buffer loads over one z slice of a map or of the z-pass output (below
@@ -277,24 +292,24 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
                                               const uint32_t* __restrict__ colm,
                                               unsigned long long* __restrict__ xflags,
                                               uint32_t* __restrict__ yfs, uint32_t dx, uint32_t dy,
-                                              uint32_t dz, uint32_t uninit)
+                                              uint32_t dz, uint32_t uninit, bool redo)
 {
   static_assert(TYR == 32, "one column-mask word per row tile");
   __shared__ uint16_t ztile[TYR][TB];
   __shared__ uint32_t ring[RK][TB];
   const uint32_t ngroups = (dx + TB - 1) / TB * dz;
-  if (blockIdx.x < dz) {
+  if (!redo && blockIdx.x < dz) {
     // the format of slice z's y output for the x pass (yfs[dz + ngroups + z]): 0 =
-    // relative sites, 1 = packed (the slice, or each of its groups, is redone here),
-    // 2 = both
+    // relative sites, 1 = packed (each of its groups is done here), 2 = both
     const uint32_t zz = blockIdx.x, nxr = (dx + TB - 1) / TB, l = threadIdx.x;
     const uint64_t fm = wave_ballot(l < nxr && yfs[dz + l * dz + zz] != 0u);
     const uint64_t allc = nxr >= 64 ? ~0ull : (1ull << nxr) - 1ull;
-    if (l == 0) yfs[dz + ngroups + zz] = yfs[zz] != 0u || fm == allc ? 1u : fm == 0ull ? 0u : 2u;
+    if (l == 0) yfs[dz + ngroups + zz] = fm == allc ? 1u : fm == 0ull ? 0u : 2u;
   }
-  // the windowed kernel resolved this group: neither its slice (yfs[z]) nor the group
-  // itself (yfs[dz + group]) was left to this kernel
-  if (yfs[blockIdx.x % dz] == 0u && yfs[dz + blockIdx.x] == 0u) return;
+  // first run: the groups that the window left to this kernel; second run (redo): the
+  // others of slices whose cut-off window outputs the x pass could not use (yfs[z])
+  const bool own = yfs[dz + blockIdx.x] != 0u;
+  if (redo ? own || yfs[blockIdx.x % dz] == 0u : !own) return;
   // consecutive blocks take consecutive z with the same x range: workgroups are
   // dealt round-robin over the XCDs, so every XCD gets every x range (obstacles
   // clustered in a few x ranges would otherwise load a few XCDs only)
@@ -332,8 +347,8 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
   uint32_t todo = tflags[x0 / 64] & (ntiles >= 32 ? 0xFFFFFFFFu : (1u << ntiles) - 1u);
   uint32_t pre[TYR], pre_cm = 0;
   auto load_rows = [&](uint32_t t) {  // past the end of the line: harmless reloads of the last row
-    // rows of this tile whose 64-column segment was stored (TYR == 32; all for other widths)
-    pre_cm = dx % 64 == 0 ? colm[(uint64_t)t * (dx / 64) + x0 / 64] : 0xFFFFFFFFu;
+    // rows of this tile whose 64-column segment was stored (TYR == 32)
+    pre_cm = colm[(uint64_t)t * ((dx + 63) / 64) + x0 / 64];
 #pragma unroll
     for (int r = 0; r < TYR; ++r) {
       const uint32_t yr = t * TYR + r;
@@ -396,7 +411,8 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
   }
   // a line whose x tile kept no site is never read again: the x pass skips the tile
   // and the colouring writes every voxel of every row, so its rows are not stored
-  if (((kept >> ((lane / TX) * TX)) & ((1ull << TX) - 1ull)) == 0) return;
+  // (in a second run the window has announced every tile)
+  if (!redo && ((kept >> ((lane / TX) * TX)) & ((1ull << TX) - 1ull)) == 0) return;
   // output rows through a descriptor over this z slice: lane offset x, row offset uniform
   const __amdgpu_buffer_rsrc_t orr = slice_rsrc(out + (uint64_t)z * dx * dy, dx * dy * 4);
   if (st.n == 0) {
@@ -475,37 +491,81 @@ __device__ __forceinline__ uint32_t win_search(const uint32_t* kp, bool active, 
   return best;
 }
 
-// y pass, windowed: a block takes 64 lines x0 .. x0+63 at one z and two row blocks
-// of 64 output rows, y0 .. y0+63 and y0+64 .. y0+127.  For each row block the z-pass
-// rows y0 - H .. y0 + 63 + H of the 64 columns are loaded with coalesced row loads
-// (the second row block's while the first is searched) and stored transposed (one
-// LDS row of keys per line, key position = y, payload = the site's z); each wave
-// searches 8 output rows with lanes = the 64 lines (lane l reads line l's keys, the
-// odd line stride keeps them on distinct banks), so its winners, whose keys hold
-// their sites, are whole rows and are stored directly.  The halo H follows the
-// x range's obstacle density rho (counted by the z pass): H = 2.5 / sqrt(rho),
-// rounded up to WIN_CHECK, at most WIN_R (28 at 1 %, where 8 of the 32768 row blocks
-// of a uniform 512^3 field need more, 8 at 10 %, where 3 do); a row block that does
-// not resolve is staged again with H = WIN_R, and only one that fails then sends its
-// z slice to the stack kernel.  Below rho = 1/256 (or with an obstacle-free row tile)
-// the x range's groups go to the stack kernel.
+// Growing windows of YG neighbouring outputs per lane: output i sits at row r0 + i of a
+// column of keys (read(r): the key at row r, KEY_NONE outside the line) and starts with
+// b[i] = its own key, or 0 when it is not wanted.  Step k looks at the rows r0 + i - k
+// and r0 + i + k of every output; neighbouring outputs share all but one of them per
+// side, so the two rows of YG keys live in registers that shift by one per step (the
+// loop is unrolled by YG, so every register index is static) and a step costs two LDS
+// reads, not 2 YG, beside its subtraction and v_min3 per output (see win_search for
+// the relative minima).  Returns the radius K reached: kmax (a multiple of WIN_CHECK,
+// at least the value passed) or the first multiple of WIN_CHECK at which the whole wave
+// has resolved; output i is exact when b[i] + (K^2 << SH) < (K + 1)^2 << SH.
+// One output at a time reads 2 keys per v_min3 and tests the wave's radius per output:
+// at 512^3 with 1 % obstacles YWINTIME.
+constexpr int YG = 8;
+template <int SH, typename Read>
+__device__ __forceinline__ int grow_windows(Read&& read, int r0, int kmax, int32_t (&b)[YG])
+{
+  int32_t t[YG], u[YG];
+#pragma unroll
+  for (int i = 0; i < YG; ++i) t[i] = u[i] = (int32_t)read(r0 + i);
+  for (int k = 0;; k += YG) {
+#pragma unroll
+    for (int s = 1; s <= YG; ++s) {
+      t[(YG - s) % YG] = (int32_t)read(r0 - (k + s));          // output 0's row, the others' move on
+      u[(YG - 1 + s) % YG] = (int32_t)read(r0 + YG - 1 + k + s);  // output YG - 1's
+      const int32_t w = (2 * (k + s) - 1) << SH;
+#pragma unroll
+      for (int i = 0; i < YG; ++i) b[i] = min(min(b[i] - w, t[(i - s + YG) % YG]), u[(i + s) % YG]);
+      if (s % WIN_CHECK == 0) {
+        if (k + s >= kmax) return k + s;
+        int32_t m = b[0];
+#pragma unroll
+        for (int i = 1; i < YG; ++i) m = max(m, b[i]);
+        if (wave_ballot(m >= ((2 * (k + s) + 1) << SH)) == 0ull) return k + s;
+      }
+    }
+  }
+}
+static_assert(YG % WIN_CHECK == 0, "the radius is tested inside the unrolled steps");
+
+// y pass, windowed: a block takes 64 lines x0 .. x0+63 at one z and YBR output rows.
+// The z-pass rows y0 - R .. y0 + YBR - 1 + R of the 64 columns are loaded with coalesced
+// row loads into LDS keys (row-major: lane l reads line l's, one bank each); each wave
+// searches YBR / YW_WAVES rows, YG at a time, with lanes = the 64 lines, so its winners,
+// whose keys hold their sites, are whole rows and are stored directly.
+//
+// The window is cut off at a radius R that holds for the distances of the final result,
+// not of this pass: a voxel at distance d from its nearest obstacle o takes it in the x
+// pass from position (o.x, y, z), where o is at most d away in the (y, z) plane.  So a
+// position with no site within R is marked (YREL_FAR: a cost above every window's) and
+// the x pass checks that its winners cost at most R^2; then no marked position, whose
+// true cost is above R^2, could have won or tied.  With obstacles spread evenly at
+// density rho the largest distance over 10^8 voxels is 1.9 rho^(-1/3) inside the map and
+// 2.6 rho^(-1/3) in its corners (P(r) = exp(-4/3 pi r^3 rho), an eighth of the ball in a
+// corner): R = 2.6 rho^(-1/3), 12 at 1 %, 28 at 0.1 %.  (The whole-plane radius this
+// pass would need is 2.5 rho^(-1/2): 28 at 1 %, 79 at 0.1 %.)  A z slice holding marked
+// positions that the x pass could not do with is redone by the stack kernel.
+//
+// x ranges that are not evenly filled, judged by their density (below 1/2048, where R
+// would pass WIN_R) and by their share of empty 64 x 128 cells against the
+// exp(-cell rho) of an even spread, go to the stack kernel at once.
 // Blocks are dealt to the XCDs so that the blocks of one (x range, z) group run one
 // after another on one XCD, where the overlapping halo rows are still in its L2.
-constexpr int YB = 64;                 // output rows per row block
-constexpr int YT = YB + 2 * WIN_R;     // rows staged per block, at most
-constexpr int YS = YT + 1;             // LDS words per staged line (odd: transposed writes spread over the banks)
+constexpr int YBR = 128;               // output rows per block
+constexpr int YNR = YBR + 2 * WIN_R;   // rows staged per block, at most
 constexpr int YW_WAVES = 8;
-static_assert(32 % YW_WAVES == 0, "a wave's staged rows r = w + YW_WAVES i share word (YW_WAVES i) / 32");
-constexpr int YW_RPS = YB / YW_WAVES;  // output rows searched per wave (lanes = the 64 lines)
+constexpr uint32_t YREL_FAR = 0x3FFFu;  // relative site (63, 63): costs 7938
+static_assert(YBR % (YW_WAVES * YG) == 0, "whole groups per wave");
+
 // The windowed y pass writes each voxel's site relative to the voxel, 2 bytes:
-// (y_site - y + 64) | (z_site - z + 64) << 7.  A resolved window search finds its
-// site within WIN_R rows and at a cost below (WIN_R + 1)^2, so both offsets lie in
-// [-WIN_R, WIN_R].  The stack kernel redoes every z slice with a group the window
-// left unresolved, and the groups of x ranges too sparse for the window, and writes
-// packed DistanceVoxels to the 4-byte buffer; the x pass reads a slice's rows in its
-// one format, or leaves rows whose slice has both to the x stack kernels.
-static_assert(WIN_R < 64, "relative sites hold offsets in [-64, 63]");
-// For a resolved window winner (key low bits y_site << 10 | z_site) neither field
+// (y_site - y + 64) | (z_site - z + 64) << 7.  A window winner lies within WIN_R rows and
+// at a cost below (WIN_R + 1)^2, so both offsets lie in [-WIN_R, WIN_R].  The stack
+// kernel writes packed DistanceVoxels to the 4-byte buffer; the x pass reads a slice's
+// rows in its one format, or leaves rows whose slice has both to the x stack kernels.
+static_assert(WIN_R < 63, "relative sites hold offsets in [-64, 63], the last for YREL_FAR");
+// For a window winner (key low bits y_site << 10 | z_site) neither field
 // wraps, so the relative site is a sum: c = yrel_base(y, z)
 __device__ __forceinline__ uint32_t yrel_base(uint32_t y, uint32_t z) { return (64u - y) + ((64u - z) << 7); }
 __device__ __forceinline__ uint32_t yrel_win(uint32_t key, uint32_t c)
@@ -518,231 +578,269 @@ __device__ __forceinline__ uint32_t yrel_site(uint32_t rel, uint32_t x, uint32_t
   return x | ((y + (rel & 127u) - 64u) << 10) | ((z + (rel >> 7) - 64u) << 20);
 }
 
-// Row block stages of the y window (halo H, a multiple of WIN_CHECK): wave w stages
-// rows y = y0 - H + w + YW_WAVES i.  ywin_load issues the row loads (clamped into the
-// slice, so unconditional); ywin_stage works out the rows' segment masks and stores
-// the keys transposed into kt[line][WIN_R - H + r]; ywin_find lets the lanes search
-// their lines, returns whether some voxel did not resolve and ends with a barrier, so
-// kt may be reused.
-template <int H>
-struct YRows {
-  static constexpr int NR = YB + 2 * H;
-  static constexpr int RPW = NR / YW_WAVES;
-  static_assert(NR % YW_WAVES == 0 && H <= WIN_R, "whole rows per wave");
-  uint32_t v[RPW];
-};
-
-template <int H>
-__device__ __forceinline__ void ywin_load(YRows<H>& rows, const __amdgpu_buffer_rsrc_t zr, uint32_t xl, uint32_t y0,
-                                          uint32_t dx, uint32_t dy, uint32_t w)
-{
-  constexpr int RPW = YRows<H>::RPW;
-  const int32_t ybase = (int32_t)y0 - H + (int32_t)w;
-  if ((int32_t)y0 >= H && y0 + YB + H <= dy) {  // every staged row inside the map (block-uniform)
-    const uint32_t off0 = (uint32_t)ybase * dx * 2, step = YW_WAVES * dx * 2;
-#pragma unroll
-    for (int i = 0; i < RPW; ++i)
-      rows.v[i] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)(xl * 2), (int)(off0 + (uint32_t)i * step), 0);
-  } else {  // rows outside the map read a row inside it (their keys are KEY_NONE)
-#pragma unroll
-    for (int i = 0; i < RPW; ++i) {
-      const int32_t yc = min(max(ybase + YW_WAVES * i, 0), (int32_t)dy - 1);
-      rows.v[i] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)(xl * 2), (int)((uint32_t)yc * dx * 2), 0);
-    }
-  }
-}
-
-template <int H>
-__device__ __forceinline__ void ywin_stage(uint32_t* kt, const YRows<H>& rows, const uint32_t* __restrict__ colm,
+// one block's rows with window radius R (a multiple of WIN_CHECK); returns whether this
+// wave marked a position
+template <int R>
+__device__ __forceinline__ bool ywin_block(int32_t* kt, const __amdgpu_buffer_rsrc_t zr,
+                                           const uint32_t* __restrict__ colm, const __amdgpu_buffer_rsrc_t orr,
                                            uint32_t x0, uint32_t y0, uint32_t z, uint32_t dx, uint32_t dy,
-                                           uint32_t lane, uint32_t w)
+                                           uint32_t nxr, uint32_t lane, uint32_t w)
 {
-  constexpr int NR = YRows<H>::NR, RPW = YRows<H>::RPW;
-  const int32_t ybase = (int32_t)y0 - H + (int32_t)w;
-  const int32_t zc = (int32_t)(z & 1023u);  // z < 1024: tells the compiler dz fits a 24-bit product
-  // segment bits of the staged rows (y0 is a multiple of 32): rm[k] bit b = row 32 k + b
-  constexpr int S = (32 - H % 32) % 32;  // (y0 - H) mod 32
-  constexpr int NW = (NR + 31) / 32;
-  const int32_t base = ((int32_t)y0 - H) >> 5;  // floor((y0 - H) / 32)
-  const int32_t nyw = (int32_t)((dy + 31) / 32);
-  uint32_t cw[NW + 1], ok[NW];
-#pragma unroll
-  for (int j = 0; j <= NW; ++j) {
-    const int32_t wi = base + j;
-    cw[j] = dx % 64 != 0 ? 0xFFFFFFFFu : wi >= 0 && wi < nyw ? colm[(uint32_t)wi * (dx / 64) + x0 / 64] : 0u;
-  }
-  // staged rows that hold sites: r in [rlo, rhi) (y inside the map) with a stored
-  // segment; ok[k] bit b = row 32 k + b + w, i.e. shifted by the wave's row offset so
-  // that row w + YW_WAVES i is bit (YW_WAVES i) % 32 of word (YW_WAVES i) / 32
-  const int32_t rlo = H - (int32_t)y0, rhi = (int32_t)dy - (int32_t)y0 + H;
-#pragma unroll
-  for (int k = 0; k < NW; ++k) {
-    const uint32_t seg = S == 0 ? cw[k] : (cw[k] >> S) | (cw[k + 1] << ((32 - S) % 32));
-    const int32_t a = min(max(rlo - 32 * k, 0), 32), b = min(max(rhi - 32 * k, 0), 32);
-    const uint32_t below_b = b >= 32 ? 0xFFFFFFFFu : (1u << b) - 1u, below_a = a >= 32 ? 0xFFFFFFFFu : (1u << a) - 1u;
-    ok[k] = (seg & below_b & ~below_a) >> w;
-  }
+  constexpr int NR = YBR + 2 * R, RPW = NR / YW_WAVES;
+  static_assert(NR % YW_WAVES == 0 && R <= WIN_R && R % WIN_CHECK == 0, "whole rows per wave");
+  const uint32_t x = x0 + lane, xl = x < dx ? x : dx - 1;
+  const bool xin = x < dx;
+  const int32_t ybase = (int32_t)y0 - R + (int32_t)w;
+  uint32_t v[RPW];
+  // rows outside the map read a row inside it (their keys are KEY_NONE)
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
-    const uint32_t r = w + YW_WAVES * i;
+    const int32_t yc = min(max(ybase + YW_WAVES * i, 0), (int32_t)dy - 1);
+    v[i] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)(xl * 2), (int)((uint32_t)yc * dx * 2), 0);
+  }
+  const int32_t zc = (int32_t)(z & 1023u);  // z < 1024: tells the compiler dz fits a 24-bit product
+#pragma unroll
+  for (int i = 0; i < RPW; ++i) {
     const int32_t y = ybase + YW_WAVES * i;
-    const bool rowok = (ok[(YW_WAVES * i) / 32] >> ((YW_WAVES * i) % 32)) & 1u;  // block-uniform
-    const uint32_t vi = rows.v[i];
-    // y key (SH = 20): min((z_site - z)^2, 2047) << 20 | y << 10 | z_site
-    const int32_t dzv = (int32_t)vi - zc;
+    // rows inside the map whose 64-column segment was stored (uniform over the wave)
+    const int32_t yc = min(max(y, 0), (int32_t)dy - 1);
+    const bool rowok = y == yc && ((colm[(uint32_t)(yc >> 5) * nxr + x0 / 64] >> (yc & 31)) & 1u);
+    // key (SH = 20): min((z_site - z)^2, 2047) << 20 | y << 10 | z_site.  A column
+    // without a site (ZNONE) costs 2047, above every cost that a window resolves.
+    const int32_t dzv = (int32_t)v[i] - zc;
     const uint32_t c = min((uint32_t)__mul24(dzv, dzv), 2047u);
-    // rows above the map (y < 0, KEY_NONE rows) keep only 10 bits of y, so every key
-    // stays below 2^31
-    const uint32_t key = (c << 20) | (((uint32_t)y << 10) & 0xFFC00u) | vi;
-    // a row without sites (uniform) ORs KEY_NONE (bits 0-30) in, with no branch: every
-    // such row reads KEY_NONE, every other key is unchanged.  A column without a site
-    // (ZNONE) keeps its key: its cost saturates at 2047, above the cost of any site
-    // that resolves a voxel (below (WIN_R + 1)^2), so it never decides one.  Lanes past
-    // dx stage lines that no active lane searches.
-    const uint32_t none_row = rowok ? 0u : KEY_NONE;
-    kt[lane * YS + (WIN_R - H) + r] = key | none_row;
+    const uint32_t key = (c << 20) | (((uint32_t)y << 10) & 0xFFC00u) | v[i];
+    kt[(w + YW_WAVES * i) * TB + lane] = (int32_t)(key | (rowok ? 0u : KEY_NONE));
   }
-}
-
-template <int H>
-__device__ __forceinline__ bool ywin_find(uint32_t* kt, uint32_t x0, uint32_t y0, uint32_t dx, uint32_t dy,
-                                          uint32_t lane, uint32_t w, uint32_t* res)
-{
-  __syncthreads();  // every row staged
-  const bool xin = x0 + lane < dx;
-  bool fail = false;
+  __syncthreads();
+  bool cut = false;
+#pragma unroll 1
+  for (uint32_t g = 0; g < (uint32_t)(YBR / (YW_WAVES * YG)); ++g) {
+    const uint32_t j = (g * YW_WAVES + w) * YG, yw = y0 + j;  // output rows yw .. yw + YG - 1
+    if (yw >= dy) break;
+    const int32_t* kl = kt + lane;
+    int32_t b[YG];
 #pragma unroll
-  for (int i = 0; i < YW_RPS; ++i) {
-    const uint32_t j = w * YW_RPS + (uint32_t)i;  // output row y0 + j (uniform over the wave)
-    bool okl = true;
-    res[i] = win_search<20>(kt + lane * YS + j, xin && y0 + j < dy, okl, H);
-    fail = fail || !okl;
-  }
-  return __syncthreads_or(fail) != 0;  // also: every search is done before kt is reused
-}
-
-// the row block's winners (keys holding their sites) as relative sites (yrel_win):
-// a wave's lanes hold whole rows, so each row is one coalesced store
-__device__ __forceinline__ void ywin_store(const uint32_t* res, uint16_t* __restrict__ outl, uint32_t x0,
-                                           uint32_t y0, uint32_t z, uint32_t dx, uint32_t dy, uint32_t lane,
-                                           uint32_t w)
-{
-  const uint32_t x = x0 + lane, yw = y0 + w * YW_RPS;
-  const __amdgpu_buffer_rsrc_t orr = slice_rsrc(outl, dx * dy * 2);
-  const uint32_t c = yrel_base(yw, z), so = yw * dx * 2;  // row i: c - i, so + i * dx * 2
-  if (y0 + YB <= dy && x0 + TB <= dx) {  // block-uniform: every row and lane inside the map
+    for (int i = 0; i < YG; ++i) {
+      b[i] = kl[(R + j + i) * TB];
+      if (!xin || yw + (uint32_t)i >= dy) b[i] = 0;
+    }
+    const int k = grow_windows<20>([&](int r) { return kl[r * TB]; }, R + (int)j, R, b);
+    const uint32_t lim = (uint32_t)((k + 1) * (k + 1)) << 20, add = (uint32_t)(k * k) << 20;
+    const uint32_t c = yrel_base(yw, z);
 #pragma unroll
-    for (int i = 0; i < YW_RPS; ++i)
-      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)yrel_win(res[i], c - (uint32_t)i), orr, (int)(x * 2),
-                                            (int)(so + (uint32_t)i * dx * 2), 0);
-  } else {
-#pragma unroll
-    for (int i = 0; i < YW_RPS; ++i)
-      if (yw + (uint32_t)i < dy && x < dx)
-        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)yrel_win(res[i], c - (uint32_t)i), orr, (int)(x * 2),
-                                              (int)(so + (uint32_t)i * dx * 2), 0);
+    for (int i = 0; i < YG; ++i) {
+      if (!xin || yw + (uint32_t)i >= dy) continue;
+      const uint32_t res = (uint32_t)b[i] + add;
+      const bool ok = res < lim;
+      cut = cut || !ok;
+      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(ok ? yrel_win(res, c - (uint32_t)i) : YREL_FAR), orr,
+                                            (int)(x * 2), (int)((yw + (uint32_t)i) * dx * 2), 0);
+    }
   }
+  return wave_ballot(cut) != 0ull;
 }
 
-// one block's row blocks y0 and y0 + YB (when inside the map) with halo H: the second
-// block's rows are loaded while the first one is searched.  A row block that does not
-// resolve is staged again with halo WIN_R; one that fails then leaves the group to the
-// stack kernel.  Returns whether the group was left to it.
-template <int H>
-__device__ __forceinline__ bool ywin_pair(uint32_t* kt, const __amdgpu_buffer_rsrc_t zr,
-                                          const uint32_t* __restrict__ colm, uint16_t* __restrict__ outl,
-                                          uint32_t x0, uint32_t y0, uint32_t z, uint32_t dx, uint32_t dy,
-                                          uint32_t lane, uint32_t w)
-{
-  const uint32_t xl = x0 + lane < dx ? x0 + lane : dx - 1;
-  const bool two = y0 + YB < dy;  // block-uniform
-  uint32_t res[YW_RPS];
-  YRows<H> a, b;
-  ywin_load<H>(a, zr, xl, y0, dx, dy, w);
-  ywin_stage<H>(kt, a, colm, x0, y0, z, dx, dy, lane, w);
-  if (two) ywin_load<H>(b, zr, xl, y0 + YB, dx, dy, w);  // in flight during the first search
-  const bool fa = ywin_find<H>(kt, x0, y0, dx, dy, lane, w, res);
-  if (!fa) ywin_store(res, outl, x0, y0, z, dx, dy, lane, w);
-  bool fb = false;
-  if (two) {
-    ywin_stage<H>(kt, b, colm, x0, y0 + YB, z, dx, dy, lane, w);
-    fb = ywin_find<H>(kt, x0, y0 + YB, dx, dy, lane, w, res);
-    if (!fb) ywin_store(res, outl, x0, y0 + YB, z, dx, dy, lane, w);
-  }
-  // a row block that did not resolve is staged again with halo WIN_R, after both
-  // (so the rare retry does not add to the registers live above)
-  for (int k = 0; k < 2; ++k) {
-    if (!(k == 0 ? fa : fb)) continue;
-    if (H == WIN_R) return true;
-    const uint32_t yk = y0 + (uint32_t)k * YB;
-    YRows<WIN_R> full;
-    ywin_load<WIN_R>(full, zr, xl, yk, dx, dy, w);
-    ywin_stage<WIN_R>(kt, full, colm, x0, yk, z, dx, dy, lane, w);
-    if (ywin_find<WIN_R>(kt, x0, yk, dx, dy, lane, w, res)) return true;
-    ywin_store(res, outl, x0, yk, z, dx, dy, lane, w);
-  }
-  return false;
-}
-
-__global__ void __launch_bounds__(TB * YW_WAVES, 8) k_pba_y_win(const uint16_t* __restrict__ zs,
+__global__ void __launch_bounds__(TB * YW_WAVES, 6) k_pba_y_win(const uint16_t* __restrict__ zs,
                                                              uint16_t* __restrict__ out,
                                                              const uint32_t* __restrict__ tflags,
                                                              const uint32_t* __restrict__ colm,
                                                              unsigned long long* __restrict__ xflags,
-                                                             uint32_t* __restrict__ yfs,
-                                                             const uint32_t* __restrict__ xcnt, uint32_t dx,
+                                                             uint32_t* __restrict__ yfs, uint32_t* __restrict__ ycut,
+                                                             uint32_t* __restrict__ xcnt, uint32_t dx,
                                                              uint32_t dy, UDiv dzd, UDiv nybd, uint32_t ngroups)
 {
-  __shared__ uint32_t kt[TB * YS];
+  __shared__ int32_t kt[YNR * TB];
   const uint32_t xcd = blockIdx.x % 8, seq = blockIdx.x / 8;
   uint32_t jb, z;
   const uint32_t g = nybd.div(seq, jb) * 8 + xcd;
   if (g >= ngroups) return;  // uniform over the block
-  const uint32_t dz = dzd.d, x0 = dzd.div(g, z) * TB, y0 = jb * 2 * YB;  // g = the stack kernel's block index
+  const uint32_t dz = dzd.d, xr = dzd.div(g, z), x0 = xr * TB, y0 = jb * YBR;  // g = the stack kernel's block index
   const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
-  const uint32_t ntl = (dy + TYR - 1) / TYR;
-  const uint32_t all = ntl >= 32 ? 0xFFFFFFFFu : (1u << ntl) - 1u;
-  const uint32_t tf = tflags[x0 / 64] & all;
+  const uint32_t ntl = (dy + TYR - 1) / TYR, nxr = (dx + TB - 1) / TB;
+  const uint32_t tf = tflags[xr] & (ntl >= 32 ? 0xFFFFFFFFu : (1u << ntl) - 1u);
   if (tf == 0) return;  // no obstacle in these columns: no line keeps a site, nothing is read later
-  // halo from the density (see above): the smallest multiple of WIN_CHECK with
-  // H^2 rho >= 2.5^2, at most WIN_R (in float: it only picks the halo tried first)
-  const uint64_t cols = (uint64_t)(dx - x0 < (uint32_t)TB ? dx - x0 : (uint32_t)TB) * dy * dz;
-  const uint32_t nob = xcnt[x0 / 64];
-  const float colsf = (float)(dx - x0 < (uint32_t)TB ? dx - x0 : (uint32_t)TB) * (float)dy * (float)dz;
-  const float hf = __builtin_amdgcn_sqrtf(6.25f * colsf * __builtin_amdgcn_rcpf((float)(nob ? nob : 1u)));
-  int hh = (int)__builtin_ceilf(hf * (1.0f / WIN_CHECK)) * WIN_CHECK;
-  hh = __builtin_amdgcn_readfirstlane(hh < WIN_CHECK ? WIN_CHECK : hh > WIN_R ? WIN_R : hh);
-  // row tiles without an obstacle (far voxels), or too few obstacles: left to the stack kernel
-  if (tf != all || (uint64_t)nob * 256 < cols) {  // the same for every z of the x range
+  // density and evenness of the x range (in float: they only pick the path)
+  const float ncol = (float)(dx - x0 < (uint32_t)TB ? dx - x0 : (uint32_t)TB), nob = (float)xcnt[xr];
+  const float rho = nob / (ncol * (float)dy * (float)dz);
+  const uint32_t cz = 32 * ZCELL;
+  const float cells = (float)dy * (float)((dz + cz - 1) / cz), zdepth = (float)(dz < cz ? dz : cz);
+  const float even = __builtin_amdgcn_exp2f(-1.4427f * rho * ncol * zdepth);
+  const float tail = dz > cz && dz % cz ? (float)dy : 0.0f;  // the last cells are shorter
+  const bool sparse = rho * 2048.0f < 1.0f || (float)xcnt[16 + xr] > cells * fminf(1.0f, 1.5f * even + 0.03f) + tail;
+  const float rf = 2.6f * __builtin_amdgcn_exp2f(-__builtin_amdgcn_logf(rho) * (1.0f / 3.0f));
+  const int rr = (int)__builtin_ceilf(rf * (1.0f / WIN_CHECK)) * WIN_CHECK;
+  const int r = __builtin_amdgcn_readfirstlane(rr < WIN_CHECK ? WIN_CHECK : rr > WIN_R ? WIN_R : rr);
+  if (__builtin_amdgcn_readfirstlane((int)sparse)) {  // the same for every block of the x range
     if (threadIdx.x == 0) yfs[dz + g] = 1u;
     return;
   }
-  // (a block of a slice that another block has already flagged still runs: the stack
-  // kernel rewrites the whole slice after this kernel, and checking first would cost
-  // every block a barrier and a load round)
   const __amdgpu_buffer_rsrc_t zr = slice_rsrc(zs + (uint64_t)z * dx * dy, dx * dy * 2);
-  uint16_t* __restrict__ outl = out + (uint64_t)z * dx * dy;
-  bool left;
-  switch (hh) {  // block-uniform
-#define GVX_YWIN_CASE(HV) \
-  case HV: left = ywin_pair<HV>(kt, zr, colm, outl, x0, y0, z, dx, dy, lane, w); break;
+  const __amdgpu_buffer_rsrc_t orr = slice_rsrc(out + (uint64_t)z * dx * dy, dx * dy * 2);
+  bool cut;
+  switch (r) {  // block-uniform
+#define GVX_YWIN_CASE(RV) \
+  case RV: cut = ywin_block<RV>(kt, zr, colm, orr, x0, y0, z, dx, dy, nxr, lane, w); break;
     GVX_YWIN_CASE(4) GVX_YWIN_CASE(8) GVX_YWIN_CASE(12) GVX_YWIN_CASE(16)
     GVX_YWIN_CASE(20) GVX_YWIN_CASE(24) GVX_YWIN_CASE(28)
 #undef GVX_YWIN_CASE
-    default: left = ywin_pair<WIN_R>(kt, zr, colm, outl, x0, y0, z, dx, dy, lane, w);
+    default: cut = ywin_block<WIN_R>(kt, zr, colm, orr, x0, y0, z, dx, dy, nxr, lane, w);
   }
-  if (left) {
-    if (threadIdx.x == 0) yfs[z] = 1u;
-    return;
-  }
-  // every line of the range kept a site (this row block resolved with a site in every
-  // line): its x tiles are read by the x pass
-  if (threadIdx.x == 0) {
+  if (cut && lane == 0) ycut[z] = 1u;
+  if (threadIdx.x == 0 && jb == 0) {
+    if (z == 0) atomicMax(xcnt + 32, 64u - (uint32_t)r);  // the smallest radius used, as 64 - R
+    // the x tiles of the range are read by the x pass
     unsigned long long f = 0;
 #pragma unroll
     for (int k = 0; k < TB / TX; ++k)
       if (x0 + k * TX < dx) f |= 1ull << (x0 / TX + k);
     atomicOr(xflags + z, f);
+  }
+}
+
+// ---------------------------------------------------------------- small maps
+// The stack kernels walk a line per lane: a small map has too few lines to fill the chip
+// and one walk's latency sets the pace (128^3: 256 waves, SMALLSTACK).  The windows of
+// grow_windows have every voxel of a line to work on at once, so maps of up to
+// PBA_SCAN_MAX voxels grow them as far as the line goes (an exact result whatever the
+// field, no flags and no second path): 2 instructions per voxel and radius, early exit
+// when a wave has resolved.
+// The line lies between PBASCANLINE
+constexpr uint64_t PBA_SCAN_MAX = 1ull << 24;
+constexpr uint32_t PBA_SCAN_EDGE = 512;  // longest y line (LDS: 256 bytes a row) and x line (64 lanes x YG)
+static inline bool pba_scan_suits(const uint32_t d[3])
+{
+  return (uint64_t)d[0] * d[1] * d[2] <= PBA_SCAN_MAX && d[0] <= PBA_SCAN_EDGE && d[1] <= PBA_SCAN_EDGE && d[2] <= 1024;
+}
+
+// y pass: a block takes 64 lines (x range, z) with every row in LDS between two rows of
+// KEY_NONE; keys (SH = 10) are cost << 10 | y, and the winner's z is read again from the
+// z pass (a 21-bit cost and two 10-bit coordinates do not fit one word).  Output:
+// packed DistanceVoxels.
+constexpr int YSC_WAVES = 16;
+__global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* __restrict__ zs,
+                                                               uint32_t* __restrict__ out, uint32_t dx, uint32_t dy,
+                                                               UDiv dzd, uint32_t uninit)
+{
+  extern __shared__ int32_t ysc_lds[];  // (dy + 2) x 64
+  uint32_t z;
+  const uint32_t x0 = dzd.div(blockIdx.x, z) * TB;
+  const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
+  const uint32_t x = x0 + lane, xl = x < dx ? x : dx - 1;
+  const uint16_t* __restrict__ zsl = zs + (uint64_t)z * dx * dy;
+  constexpr int LD = 8;  // row loads in flight
+  for (uint32_t y0 = w; y0 < dy; y0 += YSC_WAVES * LD) {
+    uint32_t v[LD];
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+      const uint32_t y = y0 + YSC_WAVES * i;
+      v[i] = zsl[(y < dy ? y : dy - 1) * dx + xl];
+    }
+#pragma unroll
+    for (int i = 0; i < LD; ++i) {
+      const uint32_t y = y0 + YSC_WAVES * i;
+      const uint32_t c = (uint32_t)sq24((int32_t)v[i] - (int32_t)z);
+      if (y < dy) ysc_lds[(y + 1) * TB + lane] = (int32_t)(v[i] == ZNONE ? KEY_NONE : c << 10 | y);
+    }
+  }
+  if (w == 0) {
+    ysc_lds[lane] = (int32_t)KEY_NONE;
+    ysc_lds[(dy + 1) * TB + lane] = (int32_t)KEY_NONE;
+  }
+  __syncthreads();
+  const int32_t* kl = ysc_lds + lane;
+  const int last = (int)dy + 1;
+  for (uint32_t y0 = w * YG; y0 < dy; y0 += YSC_WAVES * YG) {
+    auto read = [&](int r) { return kl[min(max(r, 0), last) * TB]; };
+    int32_t b[YG];
+#pragma unroll
+    for (int i = 0; i < YG; ++i) {
+      b[i] = read((int)y0 + 1 + i);
+      if (x >= dx || y0 + (uint32_t)i >= dy) b[i] = 0;
+    }
+    const uint32_t far = max(y0 + YG - 1, dy - 1 - y0);  // the line's farther end from any of the outputs
+    const int k = grow_windows<10>(read, (int)y0 + 1, (int)(far + WIN_CHECK - 1) / WIN_CHECK * WIN_CHECK, b);
+    uint32_t ys[YG], zv[YG];
+#pragma unroll
+    for (int i = 0; i < YG; ++i) {
+      const uint32_t res = (uint32_t)b[i] + ((uint32_t)(k * k) << 10);
+      ys[i] = res == KEY_NONE ? 0xFFFFFFFFu : res & 1023u;
+      zv[i] = zsl[(ys[i] < dy ? ys[i] : dy - 1) * dx + xl];
+    }
+#pragma unroll
+    for (int i = 0; i < YG; ++i)
+      if (x < dx && y0 + (uint32_t)i < dy)
+        out[((uint64_t)z * dy + y0 + (uint32_t)i) * dx + x] =
+            ys[i] == 0xFFFFFFFFu ? uninit : x | (ys[i] << 10) | (zv[i] << 20);
+  }
+}
+
+// x pass: a wave takes 64 / LPR rows (y, z) with LPR lanes each (a power of two), every
+// lane YG consecutive positions.  Keys (SH = 10: cost << 10 | x) sit in LDS with one word
+// after every 8, so the lanes' stride of 9 words is free of bank conflicts, and a
+// KEY_NONE word at either end of the row, where reads past it are clamped; the entries
+// lie beside them for the winners.
+constexpr int XSC_WAVES = 4;
+constexpr uint32_t XSC_W = TB * YG;                         // positions a wave holds
+constexpr uint32_t XSC_KEYS = XSC_W + XSC_W / 8 + 2 * 8;    // key words of a wave: up to 8 rows of two ends
+__global__ void __launch_bounds__(TB * XSC_WAVES) k_pba_x_scan(const uint32_t* __restrict__ yb,
+                                                               uint32_t* __restrict__ map, uint32_t dx, UDiv dyd,
+                                                               uint32_t dz, uint32_t llog, uint32_t uninit)
+{
+  __shared__ int32_t xsc_keys[XSC_WAVES][XSC_KEYS];
+  __shared__ uint32_t xsc_ent[XSC_WAVES][XSC_W];
+  const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
+  const uint32_t lpr = 1u << llog, pw = lpr * YG, rs = pw + pw / 8 + 2;  // lanes, positions, key words per row
+  const uint32_t nlines = dyd.d * dz, rows = TB >> llog;
+  const uint32_t line0 = (blockIdx.x * XSC_WAVES + w) * rows;
+  if (line0 >= nlines) return;  // no block-wide barrier in here
+  int32_t* keys = xsc_keys[w];
+  uint32_t* ent = xsc_ent[w];
+  uint32_t v[YG];
+#pragma unroll
+  for (int j = 0; j < YG; ++j) {
+    const uint32_t e = lane + TB * j, line = line0 + (e >> (llog + 3)), p = e & (pw - 1);
+    v[j] = line < nlines && p < dx ? yb[(uint64_t)line * dx + p] : uninit;
+  }
+#pragma unroll
+  for (int j = 0; j < YG; ++j) {
+    const uint32_t e = lane + TB * j, r = e >> (llog + 3), p = e & (pw - 1);
+    uint32_t y;
+    const uint32_t z = dyd.div(line0 + r, y);
+    const uint32_t c = (uint32_t)(sq24((int32_t)((v[j] >> 10) & 0x3FFu) - (int32_t)y) +
+                                  sq24((int32_t)((v[j] >> 20) & 0x3FFu) - (int32_t)z));
+    keys[r * rs + 1 + p + (p >> 3)] = (int32_t)(v[j] == uninit ? KEY_NONE : c << 10 | p);
+    ent[e] = v[j];
+  }
+  if (lane < 2 * rows) keys[(lane >> 1) * rs + (lane & 1 ? rs - 1 : 0)] = (int32_t)KEY_NONE;
+  wave_lds_sync();
+  const uint32_t row = lane >> llog, l = lane & (lpr - 1), line = line0 + row;
+  const bool act = line < nlines;
+  const int lo = (int)(row * rs), hi = lo + (int)rs - 1, at = lo + 1 + 9 * (int)l;
+  // position 8 l + m of the lane's row; the spare word after every 8 is never addressed
+  auto read = [&](int m) { return keys[min(max(at + m + (m >> 3), lo), hi)]; };
+  int32_t b[YG];
+#pragma unroll
+  for (int i = 0; i < YG; ++i) {
+    b[i] = read(i);
+    if (!act || YG * l + (uint32_t)i >= dx) b[i] = 0;
+  }
+  const int k = grow_windows<10>(read, 0, (int)(dx + WIN_CHECK - 2) / WIN_CHECK * WIN_CHECK, b);
+  uint32_t o[YG];
+#pragma unroll
+  for (int i = 0; i < YG; ++i) {
+    const uint32_t res = (uint32_t)b[i] + ((uint32_t)(k * k) << 10), p = res & (pw - 1);
+    o[i] = res == KEY_NONE ? uninit : ent[row * pw + p];
+  }
+  if (!act) return;
+  uint32_t* __restrict__ dst = map + (uint64_t)line * dx + YG * l;
+  if ((dx & 3u) == 0) {  // rows of whole 16-byte quads
+    if (YG * l < dx) *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
+    if (YG * l + 4 < dx) *reinterpret_cast<uint4*>(dst + 4) = make_uint4(o[4], o[5], o[6], o[7]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < YG; ++i)
+      if (YG * l + (uint32_t)i < dx) dst[i] = o[i];
   }
 }
 
@@ -926,12 +1024,6 @@ __device__ __forceinline__ uint32_t wave_prefix_max(uint32_t v, uint32_t lane)
 constexpr int XC_LINES = 4;
 constexpr int XC_LPW = 4;
 __host__ __device__ constexpr uint32_t xc_pad(uint32_t dx) { return (dx + 255u) & ~255u; }
-__device__ __forceinline__ void wave_lds_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __global__ void __launch_bounds__(TB * XC_LINES) k_pba_x_colour(uint32_t* __restrict__ map,
                                                                 const uint32_t* __restrict__ stk,
                                                                 const uint32_t* __restrict__ cnt,
@@ -1039,11 +1131,13 @@ constexpr int XW_RPW = 8;  // rows per wave, one after another
 template <int NJ>
 __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __restrict__ yb,
                                                              const uint16_t* __restrict__ yr,
-                                                             const uint32_t* __restrict__ yfs,
+                                                             const uint32_t* __restrict__ yfmt,
                                                              uint32_t* __restrict__ map,
                                                              const unsigned long long* __restrict__ xflags,
-                                                             uint32_t* __restrict__ xfb, uint32_t dx, UDiv dyd,
-                                                             uint32_t dz, uint32_t uninit)
+                                                             const uint32_t* __restrict__ ycut,
+                                                             const uint32_t* __restrict__ rinv,
+                                                             uint32_t* __restrict__ xfb, uint32_t* __restrict__ yredo,
+                                                             uint32_t dx, UDiv dyd, uint32_t dz, uint32_t uninit)
 {
   extern __shared__ uint32_t xw_lds[];
   const uint32_t dy = dyd.d;
@@ -1068,11 +1162,28 @@ __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __r
   // entry, so that no later wait for them also waits for a prefetch
   const unsigned long long tf = line0 < nlines ? xflags[zf] & allt : 0ull, tl = line0 < nlines ? xflags[zl] & allt : 0ull;
   // format of the y output of the wave's (at most two) slices, set by the y stack
-  // kernel: 0 = relative sites in yr, 1 = packed sites in yb (the slice, or every
-  // 64-column group of it, went to the y stack kernel), 2 = both (its rows are left to
-  // the x stack kernels, which read each tile in its own format)
-  const uint32_t* __restrict__ yfmt = yfs + dz + (dx + TB - 1) / TB * dz;
+  // kernel: 0 = relative sites in yr, 1 = packed sites in yb (every 64-column group of
+  // the slice went to the y stack kernel), 2 = both (its rows are left to the x stack
+  // kernels, which read each tile in its own format)
   const uint32_t fmtf = line0 < nlines ? yfmt[zf] : 0u, fmtl = line0 < nlines ? yfmt[zl] : 0u;
+  // slices whose windowed y pass marked positions beyond its radius R: a winner counts
+  // only up to R^2 (see the y pass); a group left over there has its slice's windowed y
+  // lines redone by the stack kernel
+  const uint32_t cutf = line0 < nlines ? ycut[zf] : 0u, cutl = line0 < nlines ? ycut[zl] : 0u;
+  const uint32_t rcut = 64u - *rinv, lim = (rcut + 1u) * (rcut + 1u) << 11;
+  if (line0 >= nlines) return;
+  if (dy >= (uint32_t)XW_RPW && tf != 0 && tl != 0 && (tf != allt || fmtf == 2u) && (tl != allt || fmtl == 2u)) {
+    // no row of this wave can be searched: leave them all (on a 512^3 depth-camera scene
+    // every row; walking them one by one took XWSKIP)
+    const uint32_t line = line0 + lane;
+    if (lane < (uint32_t)XW_RPW && line < nlines) {
+      uint32_t yy;
+      const uint32_t zz = dyd.div(line, yy);
+      xfb[(uint64_t)(yy / TB) * dz + zz] = 1u;
+      if ((zz == zf ? cutf : cutl) != 0u) yredo[zz] = 1u;
+    }
+    return;
+  }
   // the next row's entries are loaded while the current one is searched (relative
   // sites are expanded once they have arrived); only rows that will be searched
   // (every x tile of their slice kept a site) are read: the others' loads get a
@@ -1106,7 +1217,7 @@ __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __r
       z = wrap ? z + 1 : z;
     }
     const uint32_t fmt = z == zf ? fmtf : fmtl;
-    const bool pk = fmt == 1u;
+    const bool pk = fmt == 1u, cut = (z == zf ? cutf : cutl) != 0u;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)  // (waits for the prefetch) then the next row's
       e[j] = pk ? en[j] : yrel_site(en[j], lane + TB * j, y, z);
@@ -1118,7 +1229,10 @@ __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __r
     if (tiles == 0) {  // no line of the slice kept a site
       for (uint32_t p = lane; p < dx; p += TB) row[p] = uninit;
     } else if (tiles != allt || fmt == 2u) {  // x ranges without a site (far voxels), or mixed formats
-      if (lane == 0) xfb[grp] = 1u;
+      if (lane == 0) {
+        xfb[grp] = 1u;
+        if (cut) yredo[z] = 1u;
+      }
     } else {
       search = true;
     }
@@ -1173,12 +1287,15 @@ __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __r
             const uint32_t p = lane + TB * j;
             bool ok = true;
             const uint32_t b = win_search<11>(key + (p < dx ? p : 0), p < dx, ok);
-            fail = fail || !ok;
+            fail = fail || !ok || (cut && p < dx && b >= lim);
             res[j] = (b >> 1) & 1023u;
           }
         }
         if (wave_ballot(fail)) {
-          if (lane == 0) xfb[grp] = 1u;
+          if (lane == 0) {
+            xfb[grp] = 1u;
+            if (cut) yredo[z] = 1u;
+          }
         } else {
           if (full) {
 #pragma unroll
@@ -1389,7 +1506,7 @@ static uint64_t pba_flag_words(uint32_t dx, uint32_t dy, uint32_t dz)
   const uint64_t cwords = (uint64_t)((dy + 31) / 32) * ((dx + 63) / 64);
   const uint64_t xgroups = (uint64_t)((dy + TB - 1) / TB) * dz;
   const uint64_t ygroups = (uint64_t)((dx + TB - 1) / TB) * dz;
-  return 64 + 2 * (uint64_t)dz + cwords + dz + ygroups + dz + xgroups + 64;
+  return 64 + 2 * (uint64_t)dz + cwords + dz + ygroups + dz + dz + xgroups + 64;
 }
 
 static int pba_launch(MapS* m, const PbaBufs& sc, bool timed);
@@ -1463,47 +1580,75 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
   uint32_t* tflags = (uint32_t*)sc.flags;
   unsigned long long* xflags = (unsigned long long*)((uint32_t*)sc.flags + 64);
   uint32_t* colm = (uint32_t*)sc.flags + 64 + 2 * (uint64_t)dz;
-  // y lines left to the stack kernel: yfs[z] per slice (a window search that did not
-  // resolve), then yfs[dz + group] per 64-column group (ranges too sparse for the window),
-  // then per slice the format of its y output (set by the stack kernel for the x pass)
+  // y lines of the stack kernel: yfs[z] per slice (second run, see k_pba_y), then
+  // yfs[dz + group] per 64-column group (ranges too sparse for the window), then per
+  // slice the format of its y output (set by the first run for the x pass)
   uint32_t* yfs = colm + cwords;
-  uint32_t* xfb = yfs + dz + ygroups + dz;  // x groups left to the stack kernels
-  uint32_t* xcnt = xfb + xgroups;  // obstacles per 64-column x range
+  uint32_t* yfmt = yfs + dz + ygroups;
+  uint32_t* ycut = yfmt + dz;  // slices with positions beyond the y window
+  uint32_t* xfb = ycut + dz;   // x groups left to the stack kernels
+  uint32_t* xcnt = xfb + xgroups;  // per x range: obstacles, empty cells (+ 16); smallest window radius (+ 32)
+  const bool scan = pba_scan_suits(m->dims);
+  const uint32_t nxr = (dx + TB - 1) / TB;
   const uint64_t cols = (uint64_t)dx * dy;
+  const uint32_t u = m->uninit;
   {
     ProfScope ps(timed ? "pba_z" : nullptr);
-    GVX_CHECK(fill_u32(sc.flags, 0u, fwords));
-    GVX_CHECK(pba_launched("fill of the flags"));
-    dim3 g((unsigned)((cols + 63) / 64));
-    const uint32_t u = m->uninit;
-#define ZL(W)                                                                                               \
-  if (dz == 32 * W)                                                                                         \
-    hipLaunchKernelGGL((k_pba_z<W, true>), g, dim3(64 * (W / ZWP)), 0, s, map, zs, tflags, colm, xcnt,       \
-                       (uint32_t)TYR, dx, dy, dz, u);                                                       \
-  else hipLaunchKernelGGL((k_pba_z<W, false>), g, dim3(64 * (W / ZWP)), 0, s, map, zs, tflags, colm, xcnt,  \
-                          (uint32_t)TYR, dx, dy, dz, u)
-    if (dz <= 128) { ZL(4); }
-    else if (dz <= 256) { ZL(8); }
-    else if (dz <= 512) { ZL(16); }
-    else if (dz <= 1024) { ZL(32); }
-    else {
-      hipLaunchKernelGGL(k_pba_z_long, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, map, zs, dx, dy, dz, u);
-      GVX_CHECK(fill_u32(tflags, 0xFFFFFFFFu, 64));  // no block flags: every tile is walked
-      GVX_CHECK(fill_u32(colm, 0xFFFFFFFFu, cwords));  // and every segment was stored
+    if (!scan) {
+      GVX_CHECK(fill_u32(sc.flags, 0u, fwords));
+      GVX_CHECK(pba_launched("fill of the flags"));
+    }
+    const dim3 g(nxr * dy);
+#define ZL(W, P)                                                                                               \
+  if (dz == 32 * W)                                                                                            \
+    hipLaunchKernelGGL((k_pba_z<W, true, P>), g, dim3(64 * (W / P)), 0, s, map, zs, scan ? nullptr : tflags,    \
+                       colm, xcnt, (uint32_t)TYR, dx, dy, dz, udiv(nxr), u);                                   \
+  else hipLaunchKernelGGL((k_pba_z<W, false, P>), g, dim3(64 * (W / P)), 0, s, map, zs, scan ? nullptr : tflags, \
+                          colm, xcnt, (uint32_t)TYR, dx, dy, dz, udiv(nxr), u)
+    if (scan && dz <= 512) {
+      if (dz <= 128) { ZL(4, 1); }
+      else if (dz <= 256) { ZL(8, 1); }
+      else { ZL(16, 1); }
+    } else {
+      if (dz <= 128) { ZL(4, 4); }
+      else if (dz <= 256) { ZL(8, 4); }
+      else if (dz <= 512) { ZL(16, 4); }
+      else if (dz <= 1024) { ZL(32, 4); }
+      else {
+        hipLaunchKernelGGL(k_pba_z_long, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, map, zs, dx, dy, dz, u);
+        GVX_CHECK(fill_u32(tflags, 0xFFFFFFFFu, 64));  // no block flags: every tile is walked
+        GVX_CHECK(fill_u32(colm, 0xFFFFFFFFu, cwords));  // and every segment was stored
+      }
     }
 #undef ZL
     GVX_CHECK(pba_launched("k_pba_z"));
   }
+  if (scan) {
+    {
+      ProfScope ps(timed ? "pba_y" : nullptr);
+      hipLaunchKernelGGL(k_pba_y_scan, dim3(nxr * dz), dim3(TB * YSC_WAVES), (size_t)(dy + 2) * TB * 4, s, zs, yb, dx,
+                         dy, udiv(dz), u);
+      GVX_CHECK(pba_launched("k_pba_y_scan"));
+    }
+    ProfScope ps(timed ? "pba_x" : nullptr);
+    const uint32_t llog = dx <= 64 ? 3 : dx <= 128 ? 4 : dx <= 256 ? 5 : 6, rows = XSC_WAVES * (TB >> llog);
+    hipLaunchKernelGGL(k_pba_x_scan, dim3((unsigned)((lines + rows - 1) / rows)), dim3(TB * XSC_WAVES), 0, s, yb, map,
+                       dx, udiv(dy), dz, llog, u);
+    return pba_launched("k_pba_x_scan");
+  }
+  auto y_stack = [&](bool redo) {
+    hipLaunchKernelGGL(k_pba_y, dim3((unsigned)ygroups), dim3(TB), 0, s, zs, yb, st, tflags, colm, xflags, yfs, dx, dy,
+                       dz, u, redo);
+    return pba_launched("k_pba_y");
+  };
   {
     ProfScope ps(timed ? "pba_y" : nullptr);
-    const uint32_t nyb = (dy + 2 * YB - 1) / (2 * YB);  // blocks per group: two row blocks each
+    const uint32_t nyb = (dy + YBR - 1) / YBR;             // blocks per group
     const uint64_t wblocks = (ygroups + 7) / 8 * 8 * nyb;  // blocks of 8 groups per XCD slot
     hipLaunchKernelGGL(k_pba_y_win, dim3((unsigned)wblocks), dim3(TB * YW_WAVES), 0, s, zs, yr, tflags, colm, xflags,
-                       yfs, xcnt, dx, dy, udiv(dz), udiv(nyb), (uint32_t)ygroups);
+                       yfs, ycut, xcnt, dx, dy, udiv(dz), udiv(nyb), (uint32_t)ygroups);
     GVX_CHECK(pba_launched("k_pba_y_win"));
-    hipLaunchKernelGGL(k_pba_y, dim3((unsigned)ygroups), dim3(TB), 0, s, zs, yb, st, tflags, colm, xflags, yfs, dx, dy,
-                       dz, m->uninit);
-    GVX_CHECK(pba_launched("k_pba_y"));
+    GVX_CHECK(y_stack(false));
   }
   {
     ProfScope ps(timed ? "pba_x" : nullptr);
@@ -1511,20 +1656,22 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
     const uint64_t xrows = (uint64_t)XW_WAVES * XW_RPW;
     const dim3 xg((unsigned)((lines + xrows - 1) / xrows));
     const size_t xl = (size_t)(2 * dx + 2 * WIN_R) * 4 * XW_WAVES;
-    if (dx <= 256)
-      hipLaunchKernelGGL(k_pba_x_win<4>, xg, dim3(TB * XW_WAVES), xl, s, yb, yr, yfs, map, xflags, xfb, dx, udiv(dy), dz, m->uninit);
-    else if (dx <= 512)
-      hipLaunchKernelGGL(k_pba_x_win<8>, xg, dim3(TB * XW_WAVES), xl, s, yb, yr, yfs, map, xflags, xfb, dx, udiv(dy), dz, m->uninit);
-    else
-      hipLaunchKernelGGL(k_pba_x_win<16>, xg, dim3(TB * XW_WAVES), xl, s, yb, yr, yfs, map, xflags, xfb, dx, udiv(dy), dz, m->uninit);
+#define XL(NJ)                                                                                                  \
+  hipLaunchKernelGGL(k_pba_x_win<NJ>, xg, dim3(TB * XW_WAVES), xl, s, yb, yr, yfmt, map, xflags, ycut, xcnt + 32, \
+                     xfb, yfs, dx, udiv(dy), dz, u)
+    if (dx <= 256) XL(4);
+    else if (dx <= 512) XL(8);
+    else XL(16);
+#undef XL
     GVX_CHECK(pba_launched("k_pba_x_win"));
+    GVX_CHECK(y_stack(true));
     hipLaunchKernelGGL(k_pba_x, dim3((unsigned)xgroups), dim3(TB), 0, s, yb, yr, yfs, st, cnt, xflags, xfb, dx, dy, dz,
-                       m->uninit);
+                       u);
     GVX_CHECK(pba_launched("k_pba_x"));
     const uint64_t clines = (uint64_t)XC_LINES * XC_LPW, units = (lines + clines - 1) / clines;
     const uint64_t cgrid = std::max<uint64_t>((units + 63) / 64, std::min<uint64_t>(units, 4096));
     hipLaunchKernelGGL(k_pba_x_colour, dim3((unsigned)cgrid), dim3(TB * XC_LINES),
-                       (size_t)xc_pad(dx) * 8 * XC_LINES, s, map, st, cnt, xfb, dx, udiv(dy), dz, m->uninit);
+                       (size_t)xc_pad(dx) * 8 * XC_LINES, s, map, st, cnt, xfb, dx, udiv(dy), dz, u);
     GVX_CHECK(pba_launched("k_pba_x_colour"));
   }
   return GVX_OK;
