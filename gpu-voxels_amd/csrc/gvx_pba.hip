@@ -540,13 +540,14 @@ static_assert(YG % WIN_CHECK == 0, "the radius is tested inside the unrolled ste
 // not of this pass: a voxel at distance d from its nearest obstacle o takes it in the x
 // pass from position (o.x, y, z), where o is at most d away in the (y, z) plane.  So a
 // position with no site within R is marked (YREL_FAR: a cost above every window's) and
-// the x pass checks that its winners cost at most R^2; then no marked position, whose
-// true cost is above R^2, could have won or tied.  With obstacles spread evenly at
-// density rho the largest distance over 10^8 voxels is 1.9 rho^(-1/3) inside the map and
-// 2.6 rho^(-1/3) in its corners (P(r) = exp(-4/3 pi r^3 rho), an eighth of the ball in a
-// corner): R = 2.6 rho^(-1/3), 12 at 1 %, 28 at 0.1 %.  (The whole-plane radius this
-// pass would need is 2.5 rho^(-1/2): 28 at 1 %, 79 at 0.1 %.)  A z slice holding marked
-// positions that the x pass could not do with is redone by the stack kernel.
+// the x pass checks that its winners cost less than (R + 1)^2; then no marked position,
+// whose true cost is at least that, could have won or tied.  With obstacles spread
+// evenly at density rho, P(no obstacle within r) = exp(-4/3 pi r^3 rho), an eighth of
+// that ball in a corner of the map: R + 1 = 2.78 rho^(-1/3) (R = 12 at 1 %, 28 at 0.1 %,
+// in steps of WIN_CHECK) leaves about 1 map of 512^3 in 1000 with a corner voxel beyond
+// it and 10^-10 of the others.  (The whole-plane radius this pass would need is 2.5
+// rho^(-1/2): 28 at 1 %, 79 at 0.1 %.)  A z slice holding marked positions that the x
+// pass could not do with is redone by the stack kernel.
 //
 // x ranges that are not evenly filled, judged by their density (below 1/2048, where R
 // would pass WIN_R) and by their share of empty 64 x 128 cells against the
@@ -581,36 +582,40 @@ __device__ __forceinline__ uint32_t yrel_site(uint32_t rel, uint32_t x, uint32_t
 // one block's rows with window radius R (a multiple of WIN_CHECK); returns whether this
 // wave marked a position
 template <int R>
-__device__ __forceinline__ bool ywin_block(int32_t* kt, const __amdgpu_buffer_rsrc_t zr,
+__device__ __forceinline__ bool ywin_block(int32_t* kt, const uint16_t* __restrict__ zsl,
                                            const uint32_t* __restrict__ colm, const __amdgpu_buffer_rsrc_t orr,
                                            uint32_t x0, uint32_t y0, uint32_t z, uint32_t dx, uint32_t dy,
                                            uint32_t nxr, uint32_t lane, uint32_t w)
 {
   constexpr int NR = YBR + 2 * R, RPW = NR / YW_WAVES;
-  static_assert(NR % YW_WAVES == 0 && R <= WIN_R && R % WIN_CHECK == 0, "whole rows per wave");
+  static_assert(NR % YW_WAVES == 0 && RPW <= 32 && R <= WIN_R && R % WIN_CHECK == 0, "whole rows per wave");
   const uint32_t x = x0 + lane, xl = x < dx ? x : dx - 1;
   const bool xin = x < dx;
+  const int xoff = xin ? (int)(x * 2) : 0x7FFFFFF0;
   const int32_t ybase = (int32_t)y0 - R + (int32_t)w;
+  // lane i looks up whether the wave's row i is inside the map and its 64-column segment
+  // was stored: one load for all rows (a scalar load per row waits for each in turn)
+  const int32_t yl = ybase + YW_WAVES * (int32_t)lane;
+  uint32_t seg = 0;
+  if (lane < (uint32_t)RPW && yl >= 0 && yl < (int32_t)dy) seg = colm[(uint32_t)(yl >> 5) * nxr + x0 / 64] >> (yl & 31);
   uint32_t v[RPW];
   // rows outside the map read a row inside it (their keys are KEY_NONE)
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
     const int32_t yc = min(max(ybase + YW_WAVES * i, 0), (int32_t)dy - 1);
-    v[i] = __builtin_amdgcn_raw_buffer_load_b16(zr, (int)(xl * 2), (int)((uint32_t)yc * dx * 2), 0);
+    v[i] = (zsl + (size_t)((uint32_t)yc * dx))[xl];  // uniform row, 32-bit lane offset
   }
+  const uint32_t rows = (uint32_t)wave_ballot((seg & 1u) != 0u);
   const int32_t zc = (int32_t)(z & 1023u);  // z < 1024: tells the compiler dz fits a 24-bit product
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
     const int32_t y = ybase + YW_WAVES * i;
-    // rows inside the map whose 64-column segment was stored (uniform over the wave)
-    const int32_t yc = min(max(y, 0), (int32_t)dy - 1);
-    const bool rowok = y == yc && ((colm[(uint32_t)(yc >> 5) * nxr + x0 / 64] >> (yc & 31)) & 1u);
     // key (SH = 20): min((z_site - z)^2, 2047) << 20 | y << 10 | z_site.  A column
     // without a site (ZNONE) costs 2047, above every cost that a window resolves.
     const int32_t dzv = (int32_t)v[i] - zc;
     const uint32_t c = min((uint32_t)__mul24(dzv, dzv), 2047u);
     const uint32_t key = (c << 20) | (((uint32_t)y << 10) & 0xFFC00u) | v[i];
-    kt[(w + YW_WAVES * i) * TB + lane] = (int32_t)(key | (rowok ? 0u : KEY_NONE));
+    kt[(w + YW_WAVES * i) * TB + lane] = (int32_t)(key | ((rows >> i) & 1u ? 0u : KEY_NONE));
   }
   __syncthreads();
   bool cut = false;
@@ -628,14 +633,16 @@ __device__ __forceinline__ bool ywin_block(int32_t* kt, const __amdgpu_buffer_rs
     const int k = grow_windows<20>([&](int r) { return kl[r * TB]; }, R + (int)j, R, b);
     const uint32_t lim = (uint32_t)((k + 1) * (k + 1)) << 20, add = (uint32_t)(k * k) << 20;
     const uint32_t c = yrel_base(yw, z);
+    // lanes and rows outside the map count as exact; the lanes' offset is beyond the
+    // buffer, so nothing is stored for them
 #pragma unroll
     for (int i = 0; i < YG; ++i) {
-      if (!xin || yw + (uint32_t)i >= dy) continue;
       const uint32_t res = (uint32_t)b[i] + add;
       const bool ok = res < lim;
       cut = cut || !ok;
-      __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(ok ? yrel_win(res, c - (uint32_t)i) : YREL_FAR), orr,
-                                            (int)(x * 2), (int)((yw + (uint32_t)i) * dx * 2), 0);
+      if (yw + (uint32_t)i < dy)  // uniform
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(ok ? yrel_win(res, c - (uint32_t)i) : YREL_FAR), orr, xoff,
+                                              (int)((yw + (uint32_t)i) * dx * 2), 0);
     }
   }
   return wave_ballot(cut) != 0ull;
@@ -668,23 +675,23 @@ __global__ void __launch_bounds__(TB * YW_WAVES, 6) k_pba_y_win(const uint16_t* 
   const float even = __builtin_amdgcn_exp2f(-1.4427f * rho * ncol * zdepth);
   const float tail = dz > cz && dz % cz ? (float)dy : 0.0f;  // the last cells are shorter
   const bool sparse = rho * 2048.0f < 1.0f || (float)xcnt[16 + xr] > cells * fminf(1.0f, 1.5f * even + 0.03f) + tail;
-  const float rf = 2.6f * __builtin_amdgcn_exp2f(-__builtin_amdgcn_logf(rho) * (1.0f / 3.0f));
+  const float rf = 2.78f * __builtin_amdgcn_exp2f(-__builtin_amdgcn_logf(rho) * (1.0f / 3.0f)) - 1.0f;
   const int rr = (int)__builtin_ceilf(rf * (1.0f / WIN_CHECK)) * WIN_CHECK;
   const int r = __builtin_amdgcn_readfirstlane(rr < WIN_CHECK ? WIN_CHECK : rr > WIN_R ? WIN_R : rr);
   if (__builtin_amdgcn_readfirstlane((int)sparse)) {  // the same for every block of the x range
     if (threadIdx.x == 0) yfs[dz + g] = 1u;
     return;
   }
-  const __amdgpu_buffer_rsrc_t zr = slice_rsrc(zs + (uint64_t)z * dx * dy, dx * dy * 2);
+  const uint16_t* __restrict__ zsl = zs + (uint64_t)z * dx * dy;
   const __amdgpu_buffer_rsrc_t orr = slice_rsrc(out + (uint64_t)z * dx * dy, dx * dy * 2);
   bool cut;
   switch (r) {  // block-uniform
 #define GVX_YWIN_CASE(RV) \
-  case RV: cut = ywin_block<RV>(kt, zr, colm, orr, x0, y0, z, dx, dy, nxr, lane, w); break;
+  case RV: cut = ywin_block<RV>(kt, zsl, colm, orr, x0, y0, z, dx, dy, nxr, lane, w); break;
     GVX_YWIN_CASE(4) GVX_YWIN_CASE(8) GVX_YWIN_CASE(12) GVX_YWIN_CASE(16)
     GVX_YWIN_CASE(20) GVX_YWIN_CASE(24) GVX_YWIN_CASE(28)
 #undef GVX_YWIN_CASE
-    default: cut = ywin_block<WIN_R>(kt, zr, colm, orr, x0, y0, z, dx, dy, nxr, lane, w);
+    default: cut = ywin_block<WIN_R>(kt, zsl, colm, orr, x0, y0, z, dx, dy, nxr, lane, w);
   }
   if (cut && lane == 0) ycut[z] = 1u;
   if (threadIdx.x == 0 && jb == 0) {
@@ -723,12 +730,20 @@ __global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* _
                                                                UDiv dzd, uint32_t uninit)
 {
   extern __shared__ int32_t ysc_lds[];  // (dy + 2) x 64
+  __shared__ uint32_t ysc_site[TB];  // the line holds a site
   uint32_t z;
   const uint32_t x0 = dzd.div(blockIdx.x, z) * TB;
   const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
   const uint32_t x = x0 + lane, xl = x < dx ? x : dx - 1;
   const uint16_t* __restrict__ zsl = zs + (uint64_t)z * dx * dy;
   constexpr int LD = 8;  // row loads in flight
+  if (w == 0) {
+    ysc_site[lane] = 0u;
+    ysc_lds[lane] = (int32_t)KEY_NONE;
+    ysc_lds[(dy + 1) * TB + lane] = (int32_t)KEY_NONE;
+  }
+  __syncthreads();
+  bool site = false;
   for (uint32_t y0 = w; y0 < dy; y0 += YSC_WAVES * LD) {
     uint32_t v[LD];
 #pragma unroll
@@ -741,13 +756,13 @@ __global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* _
       const uint32_t y = y0 + YSC_WAVES * i;
       const uint32_t c = (uint32_t)sq24((int32_t)v[i] - (int32_t)z);
       if (y < dy) ysc_lds[(y + 1) * TB + lane] = (int32_t)(v[i] == ZNONE ? KEY_NONE : c << 10 | y);
+      site = site || v[i] != ZNONE;
     }
   }
-  if (w == 0) {
-    ysc_lds[lane] = (int32_t)KEY_NONE;
-    ysc_lds[(dy + 1) * TB + lane] = (int32_t)KEY_NONE;
-  }
+  if (site) ysc_site[lane] = 1u;
   __syncthreads();
+  // a line without a site would keep its wave's windows growing to the end
+  const bool want = x < dx && ysc_site[lane] != 0u;
   const int32_t* kl = ysc_lds + lane;
   const int last = (int)dy + 1;
   for (uint32_t y0 = w * YG; y0 < dy; y0 += YSC_WAVES * YG) {
@@ -756,7 +771,7 @@ __global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* _
 #pragma unroll
     for (int i = 0; i < YG; ++i) {
       b[i] = read((int)y0 + 1 + i);
-      if (x >= dx || y0 + (uint32_t)i >= dy) b[i] = 0;
+      if (!want || y0 + (uint32_t)i >= dy) b[i] = 0;
     }
     const uint32_t far = max(y0 + YG - 1, dy - 1 - y0);  // the line's farther end from any of the outputs
     const int k = grow_windows<10>(read, (int)y0 + 1, (int)(far + WIN_CHECK - 1) / WIN_CHECK * WIN_CHECK, b);
@@ -764,7 +779,7 @@ __global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* _
 #pragma unroll
     for (int i = 0; i < YG; ++i) {
       const uint32_t res = (uint32_t)b[i] + ((uint32_t)(k * k) << 10);
-      ys[i] = res == KEY_NONE ? 0xFFFFFFFFu : res & 1023u;
+      ys[i] = want ? res & 1023u : 0xFFFFFFFFu;
       zv[i] = zsl[(ys[i] < dy ? ys[i] : dy - 1) * dx + xl];
     }
 #pragma unroll
