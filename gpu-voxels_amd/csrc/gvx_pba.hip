@@ -6,19 +6,21 @@
 //           register bitmask (all loads issued before any use), so each voxel is
 //           read once and the nearest obstacle z (ties to the lower z) is written
 //           as uint16.
-//   y pass  on dense fields a windowed search (k_pba_y_win): every voxel takes the
-//           lowest key cost + k^2 within a radius that grows until the whole wave
-//           has resolved, and stores its site relative to itself in 2 bytes.  Z
-//           slices it cannot resolve (far voxels, sparse fields) go to the
+//   y pass  on evenly filled x ranges a windowed search (k_pba_y_win): every voxel
+//           takes the lowest key cost + k^2 within a radius that grows until the whole
+//           wave has resolved, cut off where no result can need more, and stores its
+//           site relative to itself in 2 bytes.  Other x ranges go to the
 //           proximate-point stack kernel (k_pba_y: PBA phase 2 and phase 3 with
 //           the stack's top entries in an LDS ring per line, spilled to a per-line
 //           global array only when deeper), which writes packed DistanceVoxels.
-//   x pass  the same windowed search along x (k_pba_x_win), reading each slice's
+//   x pass  a windowed search along x (k_pba_x_win), reading each slice's
 //           y output in its format; rows it cannot resolve go to the stack kernel
 //           (k_pba_x, 64 x 16 LDS tiles turning the per-lane walk into row loads,
 //           final stacks to a global array) and the colouring kernel
 //           (k_pba_x_colour: each position's owner as a prefix maximum of the
 //           entries' first positions, whole row segments written).
+// Small maps take one kernel each for y and x (k_pba_y_chunk, k_pba_x_chunk), which
+// search outwards over chunks of a line whatever the field.
 // All bisector tests are exact integer comparisons.
 #include "gvx_internal.hpp"
 
@@ -33,7 +35,7 @@ constexpr uint16_t ZNONE = 0xFFFF;
 // LDS, so each wave also knows the nearest obstacle below and above its range,
 // and writes the nearest obstacle z (ties to the lower z) of its range as uint16.
 // ZWP = 4 keeps 128 loads a lane in flight; small maps, whose few columns would leave
-// most of the chip idle, take ZWP = 1 (four times the waves: 128^3 ZTIME).
+// most of the chip idle, take ZWP = 1 (four times the waves: 128^3 18 -> 7 us).
 // FULL: dz == 32 * W, every load unconditional so the compiler keeps many in flight.
 // flags (null: every column is stored and nothing is flagged):
 // colm[(y / 32) * nxr + xr] gets bit y % 32 when the 64 columns of that row segment
@@ -56,27 +58,25 @@ __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __rest
   uint32_t xr;
   const uint32_t cy = nxrd.div(blockIdx.x, xr), cx = xr * 64 + lane;
   const bool cin = cx < dx;
-  const uint64_t col = (uint64_t)cy * dx + (cin ? cx : dx - 1);
+  const uint32_t col = cy * dx + (cin ? cx : dx - 1);  // dx dy <= 2^20: a lane offset from the layer's base
   const uint64_t layer = (uint64_t)dx * dy;
-  const uint32_t* __restrict__ p = map + col;
   uint32_t bits[ZWP];
 #pragma unroll
   for (int i = 0; i < ZWP; ++i) {
     const int w = (int)part * ZWP + i;
-    uint32_t v[32];
-    if (FULL) {
-#pragma unroll
-      for (int b = 0; b < 32; ++b) v[b] = p[(uint64_t)(w * 32 + b) * layer];
-    } else {
-#pragma unroll
-      for (int b = 0; b < 32; ++b) {
-        const uint32_t z = (uint32_t)(w * 32 + b);
-        v[b] = z < dz ? p[(uint64_t)z * layer] : uninit;
-      }
-    }
+    // layers past the map read the last one and are masked off, so that no load waits
+    // behind a test (a test per load: 2.5 times the time on a 320^3 map)
+    const uint32_t zn = FULL ? 32u : (uint32_t)(w * 32) < dz ? min(dz - (uint32_t)(w * 32), 32u) : 0u;  // uniform
     uint32_t word = 0;
+    if (zn != 0u) {
+      uint32_t v[32];
 #pragma unroll
-    for (int b = 0; b < 32; ++b) word |= (v[b] != uninit ? 1u : 0u) << b;
+      for (int b = 0; b < 32; ++b)
+        v[b] = (map + (uint64_t)((uint32_t)(w * 32) + (FULL ? (uint32_t)b : min((uint32_t)b, zn - 1u))) * layer)[col];
+#pragma unroll
+      for (int b = 0; b < 32; ++b) word |= (v[b] != uninit ? 1u : 0u) << b;
+      if (zn < 32u) word &= (1u << zn) - 1u;
+    }
     bits[i] = cin ? word : 0u;
     sb[w][lane] = bits[i];
   }
@@ -100,7 +100,6 @@ __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __rest
   // stay whole rows
   const bool wave_any = wave_ballot(any != 0u) != 0ull;
   if (cin && (!tflags || wave_any)) {
-    uint16_t* __restrict__ o = zs + col;
 #pragma unroll
     for (int i = 0; i < ZWP; ++i) {
       const int w = (int)part * ZWP + i;
@@ -119,7 +118,7 @@ __global__ void __launch_bounds__(64 * (W / ZWP)) k_pba_z(const uint32_t* __rest
           if (last == 0xFFFFu) pick = hi;
           else if (hi == 0xFFFFu) pick = last;
           else pick = (z - last <= hi - z) ? last : hi;
-          o[(uint64_t)z * layer] = (uint16_t)pick;
+          (zs + (uint64_t)z * layer)[col] = (uint16_t)pick;
         }
       }
     }
@@ -448,10 +447,8 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
 // never resolves a voxel.  Lanes take consecutive
 // positions of a line held in LDS and grow the radius together, one ds_read2 and
 // one min3 per step, until every lane has resolved (or the radius reaches
-// WIN_R).  A group with a voxel that does not resolve within WIN_R (or whose
-// block obviously holds far voxels: part of it has no obstacle) is flagged, and
-// the proximate-point kernels redo the whole group (in the y pass: its whole z
-// slice).  The output is the same either way.
+// WIN_R).  An x-pass group with a voxel that does not resolve is flagged, and
+// the proximate-point kernels redo it.  The output is the same either way.
 constexpr int WIN_R = 32;                    // largest window radius
 constexpr uint32_t KEY_NONE = 0x7FFFFFFFu;   // no site: at or above every real key, below 2^31
 constexpr int WIN_CHECK = 4;                 // radius steps between the wave's all-resolved tests
@@ -502,7 +499,7 @@ __device__ __forceinline__ uint32_t win_search(const uint32_t* kp, bool active, 
 // at least the value passed) or the first multiple of WIN_CHECK at which the whole wave
 // has resolved; output i is exact when b[i] + (K^2 << SH) < (K + 1)^2 << SH.
 // One output at a time reads 2 keys per v_min3 and tests the wave's radius per output:
-// at 512^3 with 1 % obstacles YWINTIME.
+// the y window took 281 us at 512^3 with 1 % obstacles, this way 225 us (VALU bound).
 constexpr int YG = 8;
 template <int SH, typename Read>
 __device__ __forceinline__ int grow_windows(Read&& read, int r0, int kmax, int32_t (&b)[YG])
@@ -705,157 +702,236 @@ __global__ void __launch_bounds__(TB * YW_WAVES, 6) k_pba_y_win(const uint16_t* 
   }
 }
 
-// ---------------------------------------------------------------- small maps
-// The stack kernels walk a line per lane: a small map has too few lines to fill the chip
-// and one walk's latency sets the pace (128^3: 256 waves, SMALLSTACK).  The windows of
-// grow_windows have every voxel of a line to work on at once, so maps of up to
-// PBA_SCAN_MAX voxels grow them as far as the line goes (an exact result whatever the
-// field, no flags and no second path): 2 instructions per voxel and radius, early exit
-// when a wave has resolved.
-// The line lies between PBASCANLINE
-constexpr uint64_t PBA_SCAN_MAX = 1ull << 24;
-constexpr uint32_t PBA_SCAN_EDGE = 512;  // longest y line (LDS: 256 bytes a row) and x line (64 lanes x YG)
-static inline bool pba_scan_suits(const uint32_t d[3])
+// ---------------------------------------------------------------- chunked search
+// Where distances are large, windows that grow voxel by voxel look at many positions in
+// vain.  A line's keys (SH = 10: cost << 10 | position, unsigned, NKEY_NONE without a
+// site) are therefore kept in chunks of YG with each chunk's lowest key: YG outputs of
+// one chunk take the sites of their own chunk, then look outwards chunk by chunk; a
+// chunk whose lowest key plus the squared distance to it is no better than the worst of
+// the outputs is passed over (one LDS read, an addition and a comparison for YG x YG
+// pairs), and the search ends when the distance alone is no better.  The lower bound
+// holds the tie rule too (key order: cost, then position).  On surface scenes (128^3 and
+// 256^3) an x-pass wave visits 4 to 5 chunks of 8 and tests 7 to 15, a y-pass wave visits
+// 6 to 9 (its 64 lines differ more) and tests 15 to 28.
+// Dimensions up to 1024: costs stay below 3 * 1023^2, so keys stay below NKEY_NONE, and
+// NKEY_NONE plus a squared distance inside the line below 2^32.
+constexpr uint32_t NKEY_NONE = 0xC0000000u;
+// the sites k[0 .. YG) of the chunk D positions after the outputs' (D: a multiple of YG,
+// wave-uniform): output i takes the lowest of k[j] + ((D + j - i)^2 << 10)
+__device__ __forceinline__ void chunk_visit(const uint32_t (&k)[YG], int D, uint32_t (&b)[YG])
 {
-  return (uint64_t)d[0] * d[1] * d[2] <= PBA_SCAN_MAX && d[0] <= PBA_SCAN_EDGE && d[1] <= PBA_SCAN_EDGE && d[2] <= 1024;
+  uint32_t c[2 * YG - 1];
+#pragma unroll
+  for (int m = 0; m < 2 * YG - 1; ++m) c[m] = (uint32_t)((D + m - (YG - 1)) * (D + m - (YG - 1))) << 10;
+#pragma unroll
+  for (int i = 0; i < YG; ++i)
+#pragma unroll
+    for (int j = 0; j < YG; j += 2)
+      b[i] = min(min(b[i], k[j] + c[j - i + YG - 1]), k[j + 1] + c[j + 1 - i + YG - 1]);
+}
+__device__ __forceinline__ uint32_t chunk_max(const uint32_t (&b)[YG])
+{
+  uint32_t m = b[0];
+#pragma unroll
+  for (int i = 1; i < YG; ++i) m = max(m, b[i]);
+  return m;
+}
+// squared distance (as a key) from any output to the nearest position of a chunk d >= 1 away
+__device__ __forceinline__ uint32_t chunk_gap(int d) { return (uint32_t)((YG * (d - 1) + 1) * (YG * (d - 1) + 1)) << 10; }
+
+// The y stack kernel walks a line per lane: a map with few lines leaves the chip idle and
+// one walk's latency sets the pace (surface scenes: 60-130 us at 128^3, 80-250 us at
+// 256^3, as at 512^3).  Maps of up to
+// PBA_CHUNK_MAX voxels (and lines that fit LDS) search chunks instead.
+// Both sides measured, whole EDT, box and depth-camera scenes / 1 % and 0.1 % uniform:
+// 128^3 67, 68 / 59, 68 us against 202, 131 / 83, 88; 256^3 208, 199 / 146, 190 against
+// 372, 264 / 144, 172; 320^3 488, 481 / 343, 420 against 563, 489 / 295, 358.
+constexpr uint64_t PBA_CHUNK_MAX = 1ull << 24;
+constexpr uint32_t PBA_CHUNK_EDGE = 512;  // longest y line: 64 x 4 bytes of LDS per row, and per chunk
+static inline bool pba_chunk_suits(const uint32_t d[3])
+{
+  return (uint64_t)d[0] * d[1] * d[2] <= PBA_CHUNK_MAX && d[0] <= 1024 && d[1] <= PBA_CHUNK_EDGE && d[2] <= 1024;
 }
 
-// y pass: a block takes 64 lines (x range, z) with every row in LDS between two rows of
-// KEY_NONE; keys (SH = 10) are cost << 10 | y, and the winner's z is read again from the
-// z pass (a 21-bit cost and two 10-bit coordinates do not fit one word).  Output:
-// packed DistanceVoxels.
-constexpr int YSC_WAVES = 16;
-__global__ void __launch_bounds__(TB * YSC_WAVES) k_pba_y_scan(const uint16_t* __restrict__ zs,
+// y pass: a block takes 64 lines (x range, z), lanes = the lines, a wave YG rows at a
+// time; the winner's z is read again from the z pass (a 22-bit cost and two 10-bit
+// coordinates do not fit one word).  Output: packed DistanceVoxels.
+constexpr int YC_WAVES = 16;
+static inline size_t yc_lds(uint32_t dy) { return (size_t)((dy + YG - 1) / YG) * (YG + 1) * TB * 4; }
+__global__ void __launch_bounds__(TB * YC_WAVES) k_pba_y_chunk(const uint16_t* __restrict__ zs,
                                                                uint32_t* __restrict__ out, uint32_t dx, uint32_t dy,
                                                                UDiv dzd, uint32_t uninit)
 {
-  extern __shared__ int32_t ysc_lds[];  // (dy + 2) x 64
-  __shared__ uint32_t ysc_site[TB];  // the line holds a site
+  extern __shared__ uint32_t yc_keys[];  // rows up to a whole chunk x 64, then the chunks' lowest keys x 64
+  __shared__ uint32_t yc_site[TB];       // the line holds a site
   uint32_t z;
   const uint32_t x0 = dzd.div(blockIdx.x, z) * TB;
   const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
   const uint32_t x = x0 + lane, xl = x < dx ? x : dx - 1;
+  const uint32_t nch = (dy + YG - 1) / YG;
+  uint32_t* low = yc_keys + nch * YG * TB;
   const uint16_t* __restrict__ zsl = zs + (uint64_t)z * dx * dy;
-  constexpr int LD = 8;  // row loads in flight
-  if (w == 0) {
-    ysc_site[lane] = 0u;
-    ysc_lds[lane] = (int32_t)KEY_NONE;
-    ysc_lds[(dy + 1) * TB + lane] = (int32_t)KEY_NONE;
-  }
+  if (w == 0) yc_site[lane] = 0u;
   __syncthreads();
-  bool site = false;
-  for (uint32_t y0 = w; y0 < dy; y0 += YSC_WAVES * LD) {
-    uint32_t v[LD];
-#pragma unroll
-    for (int i = 0; i < LD; ++i) {
-      const uint32_t y = y0 + YSC_WAVES * i;
-      v[i] = zsl[(y < dy ? y : dy - 1) * dx + xl];
-    }
-#pragma unroll
-    for (int i = 0; i < LD; ++i) {
-      const uint32_t y = y0 + YSC_WAVES * i;
-      const uint32_t c = (uint32_t)sq24((int32_t)v[i] - (int32_t)z);
-      if (y < dy) ysc_lds[(y + 1) * TB + lane] = (int32_t)(v[i] == ZNONE ? KEY_NONE : c << 10 | y);
-      site = site || v[i] != ZNONE;
-    }
-  }
-  if (site) ysc_site[lane] = 1u;
-  __syncthreads();
-  // a line without a site would keep its wave's windows growing to the end
-  const bool want = x < dx && ysc_site[lane] != 0u;
-  const int32_t* kl = ysc_lds + lane;
-  const int last = (int)dy + 1;
-  for (uint32_t y0 = w * YG; y0 < dy; y0 += YSC_WAVES * YG) {
-    auto read = [&](int r) { return kl[min(max(r, 0), last) * TB]; };
-    int32_t b[YG];
+  for (uint32_t g = w; g < nch; g += YC_WAVES) {  // a wave stages whole chunks
+    uint32_t v[YG], lo = NKEY_NONE;
 #pragma unroll
     for (int i = 0; i < YG; ++i) {
-      b[i] = read((int)y0 + 1 + i);
-      if (!want || y0 + (uint32_t)i >= dy) b[i] = 0;
+      const uint32_t y = g * YG + i;
+      v[i] = (zsl + (size_t)((y < dy ? y : dy - 1) * dx))[xl];
     }
-    const uint32_t far = max(y0 + YG - 1, dy - 1 - y0);  // the line's farther end from any of the outputs
-    const int k = grow_windows<10>(read, (int)y0 + 1, (int)(far + WIN_CHECK - 1) / WIN_CHECK * WIN_CHECK, b);
+#pragma unroll
+    for (int i = 0; i < YG; ++i) {
+      const uint32_t y = g * YG + i;
+      const uint32_t c = (uint32_t)sq24((int32_t)v[i] - (int32_t)z);
+      const uint32_t key = v[i] == ZNONE || y >= dy ? NKEY_NONE : c << 10 | y;
+      yc_keys[y * TB + lane] = key;
+      lo = min(lo, key);
+    }
+    low[g * TB + lane] = lo;
+    if (lo != NKEY_NONE) yc_site[lane] = 1u;
+  }
+  __syncthreads();
+  // a line without a site would keep its wave searching to the end
+  const bool want = x < dx && yc_site[lane] != 0u;
+  for (uint32_t g = w; g < nch; g += YC_WAVES) {
+    uint32_t b[YG], k[YG];
+#pragma unroll
+    for (int i = 0; i < YG; ++i) {
+      b[i] = want && g * YG + i < dy ? 0xFFFFFFFFu : 0u;
+      k[i] = yc_keys[(g * YG + i) * TB + lane];
+    }
+    chunk_visit(k, 0, b);
+    uint32_t m = chunk_max(b);
+    const int last = (int)max(g, nch - 1 - g);
+    for (int d = 1; d <= last; ++d) {
+      const uint32_t gap = chunk_gap(d);
+      if (wave_ballot(m > gap) == 0ull) break;
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {  // uniform
+        const int gc = side ? (int)g + d : (int)g - d;
+        if (gc < 0 || gc >= (int)nch || wave_ballot(low[gc * TB + lane] + gap < m) == 0ull) continue;
+#pragma unroll
+        for (int i = 0; i < YG; ++i) k[i] = yc_keys[(gc * YG + i) * TB + lane];
+        chunk_visit(k, side ? d * YG : -d * YG, b);
+        m = chunk_max(b);
+      }
+    }
     uint32_t ys[YG], zv[YG];
 #pragma unroll
     for (int i = 0; i < YG; ++i) {
-      const uint32_t res = (uint32_t)b[i] + ((uint32_t)(k * k) << 10);
-      ys[i] = want ? res & 1023u : 0xFFFFFFFFu;
+      ys[i] = b[i] & 1023u;
       zv[i] = zsl[(ys[i] < dy ? ys[i] : dy - 1) * dx + xl];
     }
 #pragma unroll
     for (int i = 0; i < YG; ++i)
-      if (x < dx && y0 + (uint32_t)i < dy)
-        out[((uint64_t)z * dy + y0 + (uint32_t)i) * dx + x] =
-            ys[i] == 0xFFFFFFFFu ? uninit : x | (ys[i] << 10) | (zv[i] << 20);
+      if (x < dx && g * YG + i < dy)
+        out[((uint64_t)z * dy + g * YG + i) * dx + x] = want ? x | (ys[i] << 10) | (zv[i] << 20) : uninit;
   }
 }
 
-// x pass: a wave takes 64 / LPR rows (y, z) with LPR lanes each (a power of two), every
-// lane YG consecutive positions.  Keys (SH = 10: cost << 10 | x) sit in LDS with one word
-// after every 8, so the lanes' stride of 9 words is free of bank conflicts, and a
-// KEY_NONE word at either end of the row, where reads past it are clamped; the entries
-// lie beside them for the winners.
-constexpr int XSC_WAVES = 4;
-constexpr uint32_t XSC_W = TB * YG;                         // positions a wave holds
-constexpr uint32_t XSC_KEYS = XSC_W + XSC_W / 8 + 2 * 8;    // key words of a wave: up to 8 rows of two ends
-__global__ void __launch_bounds__(TB * XSC_WAVES) k_pba_x_scan(const uint32_t* __restrict__ yb,
-                                                               uint32_t* __restrict__ map, uint32_t dx, UDiv dyd,
-                                                               uint32_t dz, uint32_t llog, uint32_t uninit)
+// x pass: a block takes XN_ROWS rows (y, z), every wave XN_CH neighbouring chunks of all
+// of them (lane = row + XN_ROWS * chunk), so the distances are wave-uniform; a chunk is
+// read with two 16-byte LDS reads (row strides of 4 x odd words keep both arrays free of
+// bank conflicts).  The winner's entry is read again from the y pass.
+constexpr int XN_ROWS = 32, XN_CH = TB / XN_ROWS, XN_WAVES = 8;
+static inline __host__ __device__ uint32_t xn_stride(uint32_t nch) { return nch * YG + 4; }            // 4 x odd
+static inline __host__ __device__ uint32_t xn_lows(uint32_t nch) { return ((nch + 3) / 4 | 1u) * 4; }  // 4 x odd
+static inline size_t xn_lds(uint32_t dx)
 {
-  __shared__ int32_t xsc_keys[XSC_WAVES][XSC_KEYS];
-  __shared__ uint32_t xsc_ent[XSC_WAVES][XSC_W];
+  const uint32_t nch = (dx + YG - 1) / YG;
+  return (size_t)XN_ROWS * (xn_stride(nch) + xn_lows(nch)) * 4;
+}
+__global__ void __launch_bounds__(TB * XN_WAVES) k_pba_x_chunk(const uint32_t* __restrict__ yb,
+                                                               uint32_t* __restrict__ map, uint32_t dx, UDiv dyd,
+                                                               uint32_t dz, uint32_t uninit)
+{
+  extern __shared__ uint4 xn_lds4[];
+  uint32_t* keys = reinterpret_cast<uint32_t*>(xn_lds4);
   const uint32_t lane = threadIdx.x % TB, w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / TB));
-  const uint32_t lpr = 1u << llog, pw = lpr * YG, rs = pw + pw / 8 + 2;  // lanes, positions, key words per row
-  const uint32_t nlines = dyd.d * dz, rows = TB >> llog;
-  const uint32_t line0 = (blockIdx.x * XSC_WAVES + w) * rows;
-  if (line0 >= nlines) return;  // no block-wide barrier in here
-  int32_t* keys = xsc_keys[w];
-  uint32_t* ent = xsc_ent[w];
-  uint32_t v[YG];
-#pragma unroll
-  for (int j = 0; j < YG; ++j) {
-    const uint32_t e = lane + TB * j, line = line0 + (e >> (llog + 3)), p = e & (pw - 1);
-    v[j] = line < nlines && p < dx ? yb[(uint64_t)line * dx + p] : uninit;
-  }
-#pragma unroll
-  for (int j = 0; j < YG; ++j) {
-    const uint32_t e = lane + TB * j, r = e >> (llog + 3), p = e & (pw - 1);
+  const uint32_t nch = (dx + YG - 1) / YG, ks = xn_stride(nch), ls = xn_lows(nch);
+  uint32_t* low = keys + XN_ROWS * ks;
+  const uint32_t nlines = dyd.d * dz, line0 = blockIdx.x * XN_ROWS;
+  constexpr int LD = 4;  // loads in flight
+  for (uint32_t r = w; r < (uint32_t)XN_ROWS; r += XN_WAVES) {
+    if (line0 + r >= nlines) break;
     uint32_t y;
     const uint32_t z = dyd.div(line0 + r, y);
-    const uint32_t c = (uint32_t)(sq24((int32_t)((v[j] >> 10) & 0x3FFu) - (int32_t)y) +
-                                  sq24((int32_t)((v[j] >> 20) & 0x3FFu) - (int32_t)z));
-    keys[r * rs + 1 + p + (p >> 3)] = (int32_t)(v[j] == uninit ? KEY_NONE : c << 10 | p);
-    ent[e] = v[j];
+    const uint32_t* __restrict__ prow = yb + (uint64_t)(line0 + r) * dx;
+    for (uint32_t p0 = lane; p0 < nch * YG; p0 += TB * LD) {
+      uint32_t v[LD];
+#pragma unroll
+      for (int j = 0; j < LD; ++j) {
+        const uint32_t p = p0 + TB * j;
+        v[j] = prow[p < dx ? p : dx - 1];
+      }
+#pragma unroll
+      for (int j = 0; j < LD; ++j) {
+        const uint32_t p = p0 + TB * j;
+        const uint32_t c = (uint32_t)(sq24((int32_t)((v[j] >> 10) & 0x3FFu) - (int32_t)y) +
+                                      sq24((int32_t)(v[j] >> 20) - (int32_t)z));
+        if (p < nch * YG) keys[r * ks + p] = v[j] == uninit || p >= dx ? NKEY_NONE : c << 10 | p;
+      }
+    }
   }
-  if (lane < 2 * rows) keys[(lane >> 1) * rs + (lane & 1 ? rs - 1 : 0)] = (int32_t)KEY_NONE;
-  wave_lds_sync();
-  const uint32_t row = lane >> llog, l = lane & (lpr - 1), line = line0 + row;
+  __syncthreads();
+  auto chunk = [&](uint32_t r, uint32_t g, uint32_t (&k)[YG]) {
+    const uint4* q = reinterpret_cast<const uint4*>(keys + r * ks + g * YG);
+    const uint4 a = q[0], c = q[1];
+    k[0] = a.x; k[1] = a.y; k[2] = a.z; k[3] = a.w;
+    k[4] = c.x; k[5] = c.y; k[6] = c.z; k[7] = c.w;
+  };
+  for (uint32_t e = threadIdx.x; e < XN_ROWS * nch; e += TB * XN_WAVES) {
+    const uint32_t r = e % XN_ROWS, g = e / XN_ROWS;
+    uint32_t k[YG];
+    chunk(r, g, k);  // rows past the map hold anything and are not used
+    uint32_t lo = k[0];
+#pragma unroll
+    for (int i = 1; i < YG; ++i) lo = min(lo, k[i]);
+    low[r * ls + g] = lo;
+  }
+  __syncthreads();
+  const uint32_t row = lane % XN_ROWS, line = line0 + row;
   const bool act = line < nlines;
-  const int lo = (int)(row * rs), hi = lo + (int)rs - 1, at = lo + 1 + 9 * (int)l;
-  // position 8 l + m of the lane's row; the spare word after every 8 is never addressed
-  auto read = [&](int m) { return keys[min(max(at + m + (m >> 3), lo), hi)]; };
-  int32_t b[YG];
+  for (uint32_t g0 = w * XN_CH; g0 < nch; g0 += XN_WAVES * XN_CH) {
+    const int g = (int)(g0 + lane / XN_ROWS);
+    const bool in = act && g < (int)nch;
+    uint32_t b[YG], k[YG];
 #pragma unroll
-  for (int i = 0; i < YG; ++i) {
-    b[i] = read(i);
-    if (!act || YG * l + (uint32_t)i >= dx) b[i] = 0;
-  }
-  const int k = grow_windows<10>(read, 0, (int)(dx + WIN_CHECK - 2) / WIN_CHECK * WIN_CHECK, b);
-  uint32_t o[YG];
+    for (int i = 0; i < YG; ++i) b[i] = in && (uint32_t)g * YG + i < dx ? 0xFFFFFFFFu : 0u;
+    chunk(row, in ? (uint32_t)g : 0u, k);
+    chunk_visit(k, 0, b);
+    uint32_t m = chunk_max(b);
+    const int last = max((int)g0 + XN_CH - 1, (int)nch - 1 - (int)g0);
+    for (int d = 1; d <= last; ++d) {
+      const uint32_t gap = chunk_gap(d);
+      if (wave_ballot(m > gap) == 0ull) break;
 #pragma unroll
-  for (int i = 0; i < YG; ++i) {
-    const uint32_t res = (uint32_t)b[i] + ((uint32_t)(k * k) << 10), p = res & (pw - 1);
-    o[i] = res == KEY_NONE ? uninit : ent[row * pw + p];
-  }
-  if (!act) return;
-  uint32_t* __restrict__ dst = map + (uint64_t)line * dx + YG * l;
-  if ((dx & 3u) == 0) {  // rows of whole 16-byte quads
-    if (YG * l < dx) *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
-    if (YG * l + 4 < dx) *reinterpret_cast<uint4*>(dst + 4) = make_uint4(o[4], o[5], o[6], o[7]);
-  } else {
+      for (int side = 0; side < 2; ++side) {
+        const int gc = side ? g + d : g - d;
+        const bool there = gc >= 0 && gc < (int)nch;
+        const bool better = there && low[row * ls + (there ? (uint32_t)gc : 0u)] + gap < m;
+        if (wave_ballot(better) == 0ull) continue;
+        if (there) {  // lanes whose line ends before: no sites (and squares beyond a key)
+          chunk(row, (uint32_t)gc, k);
+          chunk_visit(k, side ? d * YG : -d * YG, b);
+        }
+        m = chunk_max(b);
+      }
+    }
+    if (!in) continue;
+    uint32_t o[YG];
 #pragma unroll
-    for (int i = 0; i < YG; ++i)
-      if (YG * l + (uint32_t)i < dx) dst[i] = o[i];
+    for (int i = 0; i < YG; ++i) o[i] = b[i] >= NKEY_NONE ? uninit : yb[(uint64_t)line * dx + min(b[i] & 1023u, dx - 1)];
+    uint32_t* __restrict__ dst = map + (uint64_t)line * dx + (uint32_t)g * YG;
+    if ((dx & 3u) == 0) {  // rows of whole 16-byte quads
+      *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
+      if ((uint32_t)g * YG + 4 < dx) *reinterpret_cast<uint4*>(dst + 4) = make_uint4(o[4], o[5], o[6], o[7]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < YG; ++i)
+        if ((uint32_t)g * YG + i < dx) dst[i] = o[i];
+    }
   }
 }
 
@@ -873,7 +949,7 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
                                               uint32_t dy, uint32_t dz, uint32_t uninit)
 {
   constexpr int LPR = 64 / TX;  // loader: rows covered by one pass of the wave
-  if (xfb && xfb[blockIdx.x] == 0u) return;  // the windowed kernel resolved this group
+  if (xfb[blockIdx.x] == 0u) return;  // the windowed kernel resolved this group
   constexpr int NLD = TB / LPR;   // loader passes per tile
   __shared__ uint32_t tile[TB][TX + 1];
   __shared__ uint32_t ring[RK][TB];
@@ -1064,7 +1140,7 @@ __global__ void __launch_bounds__(TB * XC_LINES) k_pba_x_colour(uint32_t* __rest
     if (u < units) {
       uint32_t y0;
       const uint32_t z0 = dyd.div((uint32_t)u * UL, y0);
-      f = !xfb || dy % UL != 0 || xfb[(uint64_t)(y0 / TB) * dz + z0] != 0u;
+      f = dy % UL != 0 || xfb[(uint64_t)(y0 / TB) * dz + z0] != 0u;
     }
     todo = wave_ballot(f);  // the same in every wave of the block
   }
@@ -1076,7 +1152,7 @@ __global__ void __launch_bounds__(TB * XC_LINES) k_pba_x_colour(uint32_t* __rest
       if (ln >= nlines) return;
       uint32_t ly;
       const uint32_t lz = dyd.div(ln, ly);
-      if (xfb && xfb[(uint64_t)(ly / TB) * dz + lz] == 0u) continue;
+      if (xfb[(uint64_t)(ly / TB) * dz + lz] == 0u) continue;
       const uint32_t* __restrict__ s = stk + (uint64_t)ln * dx;
       // the first 64 entries are loaded together with the count (slots past the
       // count hold stale values and are not used)
@@ -1189,7 +1265,7 @@ __global__ void __launch_bounds__(TB * XW_WAVES) k_pba_x_win(const uint32_t* __r
   if (line0 >= nlines) return;
   if (dy >= (uint32_t)XW_RPW && tf != 0 && tl != 0 && (tf != allt || fmtf == 2u) && (tl != allt || fmtl == 2u)) {
     // no row of this wave can be searched: leave them all (on a 512^3 depth-camera scene
-    // every row; walking them one by one took XWSKIP)
+    // every row; walking them one by one took 61 us, leaving them 10 us)
     const uint32_t line = line0 + lane;
     if (lane < (uint32_t)XW_RPW && line < nlines) {
       uint32_t yy;
@@ -1603,24 +1679,24 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
   uint32_t* ycut = yfmt + dz;  // slices with positions beyond the y window
   uint32_t* xfb = ycut + dz;   // x groups left to the stack kernels
   uint32_t* xcnt = xfb + xgroups;  // per x range: obstacles, empty cells (+ 16); smallest window radius (+ 32)
-  const bool scan = pba_scan_suits(m->dims);
+  const bool chunks = pba_chunk_suits(m->dims);
   const uint32_t nxr = (dx + TB - 1) / TB;
   const uint64_t cols = (uint64_t)dx * dy;
   const uint32_t u = m->uninit;
   {
     ProfScope ps(timed ? "pba_z" : nullptr);
-    if (!scan) {
+    if (!chunks) {
       GVX_CHECK(fill_u32(sc.flags, 0u, fwords));
       GVX_CHECK(pba_launched("fill of the flags"));
     }
     const dim3 g(nxr * dy);
 #define ZL(W, P)                                                                                               \
   if (dz == 32 * W)                                                                                            \
-    hipLaunchKernelGGL((k_pba_z<W, true, P>), g, dim3(64 * (W / P)), 0, s, map, zs, scan ? nullptr : tflags,    \
+    hipLaunchKernelGGL((k_pba_z<W, true, P>), g, dim3(64 * (W / P)), 0, s, map, zs, chunks ? nullptr : tflags,    \
                        colm, xcnt, (uint32_t)TYR, dx, dy, dz, udiv(nxr), u);                                   \
-  else hipLaunchKernelGGL((k_pba_z<W, false, P>), g, dim3(64 * (W / P)), 0, s, map, zs, scan ? nullptr : tflags, \
+  else hipLaunchKernelGGL((k_pba_z<W, false, P>), g, dim3(64 * (W / P)), 0, s, map, zs, chunks ? nullptr : tflags, \
                           colm, xcnt, (uint32_t)TYR, dx, dy, dz, udiv(nxr), u)
-    if (scan && dz <= 512) {
+    if (chunks && dz <= 512) {
       if (dz <= 128) { ZL(4, 1); }
       else if (dz <= 256) { ZL(8, 1); }
       else { ZL(16, 1); }
@@ -1638,18 +1714,16 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
 #undef ZL
     GVX_CHECK(pba_launched("k_pba_z"));
   }
-  if (scan) {
+  if (chunks) {
     {
       ProfScope ps(timed ? "pba_y" : nullptr);
-      hipLaunchKernelGGL(k_pba_y_scan, dim3(nxr * dz), dim3(TB * YSC_WAVES), (size_t)(dy + 2) * TB * 4, s, zs, yb, dx,
-                         dy, udiv(dz), u);
-      GVX_CHECK(pba_launched("k_pba_y_scan"));
+      hipLaunchKernelGGL(k_pba_y_chunk, dim3(nxr * dz), dim3(TB * YC_WAVES), yc_lds(dy), s, zs, yb, dx, dy, udiv(dz), u);
+      GVX_CHECK(pba_launched("k_pba_y_chunk"));
     }
     ProfScope ps(timed ? "pba_x" : nullptr);
-    const uint32_t llog = dx <= 64 ? 3 : dx <= 128 ? 4 : dx <= 256 ? 5 : 6, rows = XSC_WAVES * (TB >> llog);
-    hipLaunchKernelGGL(k_pba_x_scan, dim3((unsigned)((lines + rows - 1) / rows)), dim3(TB * XSC_WAVES), 0, s, yb, map,
-                       dx, udiv(dy), dz, llog, u);
-    return pba_launched("k_pba_x_scan");
+    hipLaunchKernelGGL(k_pba_x_chunk, dim3((unsigned)((lines + XN_ROWS - 1) / XN_ROWS)), dim3(TB * XN_WAVES),
+                       xn_lds(dx), s, yb, map, dx, udiv(dy), dz, u);
+    return pba_launched("k_pba_x_chunk");
   }
   auto y_stack = [&](bool redo) {
     hipLaunchKernelGGL(k_pba_y, dim3((unsigned)ygroups), dim3(TB), 0, s, zs, yb, st, tflags, colm, xflags, yfs, dx, dy,
