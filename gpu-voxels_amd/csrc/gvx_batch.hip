@@ -32,8 +32,6 @@
 
 namespace gvx {
 
-int insert_points_async(MapS* m, const float* pts_dev, uint64_t n, const uint32_t* ends_dev, uint32_t ncl,
-                        const uint32_t* meanings_dev, uint32_t meaning, int* outside_dev);
 int map_clear_async(MapS* m);
 
 struct Schedule {

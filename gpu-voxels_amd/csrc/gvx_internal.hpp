@@ -41,6 +41,7 @@ struct Runtime {
   // small pinned host + device scratch for results
   void* host_small = nullptr;
   void* dev_small = nullptr;
+  uint32_t flag_seq = 0;  // see OutsideFlag
   bool profiling = false;
 };
 Runtime& rt();
@@ -70,6 +71,29 @@ int fill_bytes(void* dst, uint8_t value, uint64_t n_bytes);
 
 // exclusive scan of uint32 counts into uint32 offsets (n entries), total in *total_dev (may be null)
 int scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* total_dev);
+
+// Results that a call waits for.  Device counters (a 64-bit count, 8 mask words) are
+// zero between calls: results_fetch launches one wave that copies them to pinned host
+// memory and zeroes them again, then waits (a fill before the kernel and a copy after it
+// cost two more dependent launches: 19 us for a call on a tiny map, 16 us this way).
+struct ResultDev {
+  unsigned long long* count;
+  uint32_t* mask;
+};
+ResultDev results_dev();
+int results_fetch(uint64_t* count, uint8_t* mask);  // mask (32 bytes) may be null
+
+// "A point fell outside the map" (19 -> 14 us for an insert into a tiny map): the kernel itself raises the flag in pinned host
+// memory.  Each call has its own number, so nothing is cleared before and nothing copied
+// after; a device word with the same number keeps all but the first waves from writing
+// over the bus.
+struct OutsideFlag {
+  uint32_t* dev = nullptr;
+  uint32_t* host = nullptr;
+  uint32_t seq = 0;
+  bool raised() const { return *static_cast<volatile uint32_t*>(host) == seq; }  // after the call's wait
+};
+OutsideFlag outside_flag();  // a new number (under the runtime lock)
 
 inline unsigned grid_for(uint64_t n, unsigned block, unsigned cap = 1u << 20)
 {
@@ -234,6 +258,16 @@ __device__ __forceinline__ void left_shift_sv(uint32_t v[8], uint32_t shift)
 
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 
+// called by every active lane of a wave
+__device__ __forceinline__ void flag_outside(const OutsideFlag& f, bool outside)
+{
+  const uint64_t o = wave_ballot(outside);
+  if (o == 0ull || (threadIdx.x & 63) != (uint32_t)__builtin_ctzll(o)) return;
+  if (__hip_atomic_load(f.dev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == f.seq) return;
+  __hip_atomic_store(f.dev, f.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(f.host, f.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // n / d and n % d for a divisor d >= 1 with m = 0xFFFFFFFF / d from the host:
 // mulhi(n, m) is q or q - 1, one correction makes it exact (a handful of
 // instructions instead of a full division)
@@ -293,10 +327,34 @@ __device__ __forceinline__ uint32_t wave_run_head(bool in, uint64_t idx, uint32_
   const uint32_t end = above != 0ull ? (uint32_t)__builtin_ctzll(above) : 64u;
   return end - lane;
 }
+// OR over the 64 lanes (all active), the same in every lane: shifts inside the rows of
+// 16 lanes, then the four rows' last lanes (vector and scalar instructions only; a
+// butterfly of cross-lane reads waits for LDS at each of its 6 steps)
 __device__ __forceinline__ uint32_t wave_or(uint32_t v)
 {
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o);
-  return v;
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  return (uint32_t)(__builtin_amdgcn_readlane((int)v, 15) | __builtin_amdgcn_readlane((int)v, 31) |
+                    __builtin_amdgcn_readlane((int)v, 47) | __builtin_amdgcn_readlane((int)v, 63));
+}
+// the end of a collision kernel: each lane's count and the OR of its voxels' bits into
+// the call's counters; waves without a hit (most) leave at once
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v);
+__device__ __forceinline__ void add_hits(uint64_t c, const uint32_t (&acc)[8], unsigned long long* count, uint32_t* mask)
+{
+  if (wave_ballot(c != 0ull) == 0ull) return;
+  c = wave_sum_u64(c);
+  uint32_t m[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) m[k] = wave_or(acc[k]);
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(count, (unsigned long long)c);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (m[k]) atomicOr(mask + k, m[k]);
+  }
 }
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
 {

@@ -620,16 +620,9 @@ __global__ void __launch_bounds__(256) k_list_collide_map(const uint32_t* __rest
         }
       }
     }
-    c += __popcll(wave_ballot(hit));
+    c += hit ? 1u : 0u;
   }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = wave_or(acc[k]);
-  if ((threadIdx.x & 63) == 0) {
-    if (c) atomicAdd(count, (unsigned long long)c);
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (acc[k]) atomicOr(mask + k, acc[k]);
-  }
+  add_hits(c, acc, count, mask);
 }
 
 // binary search of A's ids in B (collideVoxellists / findMatchingVoxels)
@@ -655,16 +648,9 @@ __global__ void __launch_bounds__(256) k_list_collide_list(const uint32_t* __res
 #pragma unroll
       for (int k = 0; k < 8; ++k) acc[k] |= ba[8 * i + k] | bb[8 * lo + k];
     }
-    c += __popcll(wave_ballot(hit));
+    c += hit ? 1u : 0u;
   }
-#pragma unroll
-  for (int k = 0; k < 8; ++k) acc[k] = wave_or(acc[k]);
-  if ((threadIdx.x & 63) == 0) {
-    if (c) atomicAdd(count, (unsigned long long)c);
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (acc[k]) atomicOr(mask + k, acc[k]);
-  }
+  add_hits(c, acc, count, mask);
 }
 
 // collideWithBitcheck (BitVoxelList.hpp:260-292): ids of A also in B whose
@@ -1022,9 +1008,7 @@ int gvx_list_collide_map(gvx_list self, gvx_map map, float threshold, const int3
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
   uint32_t tm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (typemask) memcpy(tm, typemask, 32);
-  unsigned long long* dcount = (unsigned long long*)rt().dev_small;
-  uint32_t* dmask = (uint32_t*)rt().dev_small + 2;
-  GVX_CHECK(fill_u32(rt().dev_small, 0u, 12));
+  const ResultDev res = results_dev();
   if (self->n) {
     ProfScope ps("list_collide_map");
     unsigned g = grid_for(self->n, 256, 8192);
@@ -1033,20 +1017,16 @@ int gvx_list_collide_map(gvx_list self, gvx_map map, float threshold, const int3
     if (map->type == GVX_MT_BITVECTOR_VOXELMAP)
       hipLaunchKernelGGL(k_list_collide_map<GVX_MT_BITVECTOR_VOXELMAP>, dim3(g), dim3(256), 0, rt().stream, self->ids,
                          self->bits, self->n, (const uint8_t*)map->data, map->n, ao, ti, threshold, mode,
-                         make_uint4(tm[0], tm[1], tm[2], tm[3]), make_uint4(tm[4], tm[5], tm[6], tm[7]), dcount,
-                         dmask);
+                         make_uint4(tm[0], tm[1], tm[2], tm[3]), make_uint4(tm[4], tm[5], tm[6], tm[7]), res.count,
+                         res.mask);
     else
       hipLaunchKernelGGL(k_list_collide_map<GVX_MT_PROBAB_VOXELMAP>, dim3(g), dim3(256), 0, rt().stream, self->ids,
                          self->bits, self->n, (const uint8_t*)map->data, map->n, ao, ti, threshold, mode,
-                         make_uint4(tm[0], tm[1], tm[2], tm[3]), make_uint4(tm[4], tm[5], tm[6], tm[7]), dcount,
-                         dmask);
+                         make_uint4(tm[0], tm[1], tm[2], tm[3]), make_uint4(tm[4], tm[5], tm[6], tm[7]), res.count,
+                         res.mask);
     GVX_HIP(hipGetLastError());
   }
-  GVX_HIP(hipMemcpyAsync(rt().host_small, rt().dev_small, 40, hipMemcpyDeviceToHost, rt().stream));
-  GVX_CHECK(sync());
-  *count = *(unsigned long long*)rt().host_small;
-  if (mask_out) memcpy(mask_out, (uint8_t*)rt().host_small + 8, 32);
-  return GVX_OK;
+  return results_fetch(count, mask_out);
 }
 
 int gvx_list_collide_list(gvx_list self, gvx_list other, uint64_t* count, uint8_t mask_out[32])
@@ -1057,19 +1037,13 @@ int gvx_list_collide_list(gvx_list self, gvx_list other, uint64_t* count, uint8_
   std::unique_lock<std::recursive_mutex> g1(self->mu, std::defer_lock), g2(other->mu, std::defer_lock);
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
-  unsigned long long* dcount = (unsigned long long*)rt().dev_small;
-  uint32_t* dmask = (uint32_t*)rt().dev_small + 2;
-  GVX_CHECK(fill_u32(rt().dev_small, 0u, 12));
+  const ResultDev res = results_dev();
   if (self->n && other->n) {
     hipLaunchKernelGGL(k_list_collide_list, dim3(grid_for(self->n, 256, 8192)), dim3(256), 0, rt().stream, self->ids,
-                       self->bits, self->n, other->ids, other->bits, other->n, dcount, dmask);
+                       self->bits, self->n, other->ids, other->bits, other->n, res.count, res.mask);
     GVX_HIP(hipGetLastError());
   }
-  GVX_HIP(hipMemcpyAsync(rt().host_small, rt().dev_small, 40, hipMemcpyDeviceToHost, rt().stream));
-  GVX_CHECK(sync());
-  *count = *(unsigned long long*)rt().host_small;
-  if (mask_out) memcpy(mask_out, (uint8_t*)rt().host_small + 8, 32);
-  return GVX_OK;
+  return results_fetch(count, mask_out);
 }
 
 int gvx_list_shift_sv(gvx_list l, uint32_t shift)
@@ -1090,17 +1064,13 @@ int gvx_list_collide_bitcheck(gvx_list self, gvx_list other, uint32_t margin, ui
   std::unique_lock<std::recursive_mutex> g1(self->mu, std::defer_lock), g2(other->mu, std::defer_lock);
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
-  unsigned long long* dcount = (unsigned long long*)rt().dev_small;
-  GVX_CHECK(fill_u32(rt().dev_small, 0u, 2));
+  unsigned long long* dcount = results_dev().count;
   if (self->n && other->n) {
     hipLaunchKernelGGL(k_list_bitcheck, dim3(grid_for(self->n, 256, 8192)), dim3(256), 0, rt().stream, self->ids,
                        self->bits, self->n, other->ids, other->bits, other->n, margin, dcount);
     GVX_HIP(hipGetLastError());
   }
-  GVX_HIP(hipMemcpyAsync(rt().host_small, rt().dev_small, 8, hipMemcpyDeviceToHost, rt().stream));
-  GVX_CHECK(sync());
-  *count = *(unsigned long long*)rt().host_small;
-  return GVX_OK;
+  return results_fetch(count, nullptr);
 }
 
 int gvx_list_collide_per_meaning(gvx_list self, gvx_list other, uint64_t counts[256], uint64_t* total)

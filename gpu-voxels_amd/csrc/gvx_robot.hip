@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(256) k_robot_insert_bit(uint32_t* __restrict__
                                                           const uint32_t* __restrict__ meanings, uint32_t nl,
                                                           uint64_t n, const float* __restrict__ dh,
                                                           const float* __restrict__ base, const float* __restrict__ q,
-                                                          int* __restrict__ outside)
+                                                          OutsideFlag outside)
 {
   extern __shared__ float lds[];
   float* sA = lds;
@@ -99,12 +99,12 @@ __global__ void __launch_bounds__(256) k_robot_insert_bit(uint32_t* __restrict__
     const uint32_t m = sM[lo];
     const uint64_t idx = in ? ((uint64_t)z * dy + y) * dx + x : 0ull;
     if (wave_run_head(in, idx, m)) atomicOr(map + idx * 8 + (m >> 5), 1u << (m & 31));
-    if (wave_ballot(!in) && outside) *outside = 1;
+    flag_outside(outside, !in);
   }
 }
 
 int insert_points_async(MapS* m, const float* pts_dev, uint64_t n, const uint32_t* ends_dev, uint32_t ncl,
-                        const uint32_t* meanings_dev, uint32_t meaning, int* outside_dev);
+                        const uint32_t* meanings_dev, uint32_t meaning, const OutsideFlag& outside);
 int selfcoll_insert_async(MapS* m, const float* pts_dev, const uint32_t* sizes, uint32_t ncl,
                           const uint32_t* meanings, const uint8_t* masks, uint32_t* acc_dev);
 int selfcoll_finish(const uint32_t* acc_dev, uint8_t colliding[32], int* self_collision, int* points_outside);
@@ -209,24 +209,23 @@ int gvx_map_insert_robot(gvx_map map, const float* link_pts, const uint32_t* lin
   RobotStage S;
   uint64_t n = 0;
   GVX_CHECK(robot_stage(link_pts, link_sizes, n_links, dh, base, q, meanings, meaning, mem, &n, S));
-  GVX_CHECK(fill_u32(rt().dev_small, 0u, 4));
+  const OutsideFlag f = outside_flag();
   {
     ProfScope ps("insert_robot");
     if (map->type == GVX_MT_BITVECTOR_VOXELMAP && n_links <= 512) {  // 104 B of LDS per link
       if (n) {
         hipLaunchKernelGGL(k_robot_insert_bit, dim3(grid_for(n, 256, 4096)), dim3(256), n_links * 104, rt().stream,
                            (uint32_t*)map->data, map->dims[0], map->dims[1], map->dims[2], map->side, S.pin, S.ends,
-                           S.meanings, n_links, n, S.dh, S.base, S.q, (int*)rt().dev_small);
+                           S.meanings, n_links, n, S.dh, S.base, S.q, f);
         GVX_HIP(hipGetLastError());
       }
     } else {
       GVX_CHECK(robot_pose(S, n_links, n));
-      GVX_CHECK(insert_points_async(map, S.pout, n, S.ends, n_links, S.meanings, meaning, (int*)rt().dev_small));
+      GVX_CHECK(insert_points_async(map, S.pout, n, S.ends, n_links, S.meanings, meaning, f));
     }
   }
-  GVX_HIP(hipMemcpyAsync(rt().host_small, rt().dev_small, 4, hipMemcpyDeviceToHost, rt().stream));
   GVX_CHECK(sync());
-  if (points_outside) *points_outside = *(int*)rt().host_small;
+  if (points_outside) *points_outside = f.raised() ? 1 : 0;
   return GVX_OK;
 }
 

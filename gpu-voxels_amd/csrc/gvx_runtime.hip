@@ -186,6 +186,48 @@ int fill_bytes(void* dst, uint8_t value, uint64_t n_bytes)
   return GVX_OK;
 }
 
+// ---------------------------------------------------------------- results of a call
+// dev_small: [0, 1024) free scratch of the entry points, [1024, 1088) result counters
+// (zero between calls), [1088, 1092) the outside flag's device word.  host_small: [0,
+// 1024) free, [1024, 1088) results, [1088, 1092) the outside flag.
+constexpr size_t RES_AT = 1024, FLAG_AT = 1088;
+
+__global__ void k_results(uint32_t* __restrict__ dev, uint32_t* __restrict__ host)
+{
+  if (threadIdx.x >= 10) return;
+  __hip_atomic_store(host + threadIdx.x, dev[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  dev[threadIdx.x] = 0u;
+}
+
+ResultDev results_dev()
+{
+  char* d = (char*)rt().dev_small + RES_AT;
+  return ResultDev{(unsigned long long*)d, (uint32_t*)(d + 8)};
+}
+
+int results_fetch(uint64_t* count, uint8_t* mask)
+{
+  const char* h = (const char*)rt().host_small + RES_AT;
+  hipLaunchKernelGGL(k_results, dim3(1), dim3(64), 0, rt().stream, (uint32_t*)((char*)rt().dev_small + RES_AT),
+                     (uint32_t*)h);
+  GVX_HIP(hipGetLastError());
+  GVX_CHECK(sync());
+  memcpy(count, h, 8);
+  if (mask) memcpy(mask, h + 8, 32);
+  return GVX_OK;
+}
+
+OutsideFlag outside_flag()
+{
+  Runtime& r = rt();
+  if (++r.flag_seq == 0u) r.flag_seq = 1u;  // the words start at 0
+  OutsideFlag f;
+  f.dev = (uint32_t*)((char*)r.dev_small + FLAG_AT);
+  f.host = (uint32_t*)((char*)r.host_small + FLAG_AT);
+  f.seq = r.flag_seq;
+  return f;
+}
+
 // ---------------------------------------------------------------- exclusive scan (uint32)
 // Three-level scheme: each 256-thread block scans 2048 elements (8 per thread),
 // block totals are scanned recursively, then added back.
@@ -350,7 +392,10 @@ int gvx_init(int device)
   r.num_cus = prop.multiProcessorCount;
   GVX_HIP(hipStreamCreateWithFlags(&r.stream, hipStreamNonBlocking));
   GVX_CHECK(dalloc(&r.dev_small, 4096));
-  GVX_HIP(hipHostMalloc(&r.host_small, 4096, hipHostMallocDefault));
+  GVX_HIP(hipHostMalloc(&r.host_small, 4096, hipHostMallocCoherent));  // written by kernels, read after a wait
+  memset(r.host_small, 0, 4096);
+  GVX_CHECK(fill_u32(r.dev_small, 0u, 1024));
+  GVX_CHECK(sync());
   r.device = device;
   // device address of the EDT's fixed workspace; a failure is reported by the
   // one entry point that needs it, not here
