@@ -81,6 +81,7 @@ struct ResultDev {
   uint32_t* mask;
 };
 ResultDev results_dev();
+void result_word(uint32_t** dev, uint32_t** host);  // one more word, written by a kernel to both
 int results_fetch(uint64_t* count, uint8_t* mask);  // mask (32 bytes) may be null
 
 // "A point fell outside the map" (19 -> 14 us for an insert into a tiny map): the kernel itself raises the flag in pinned host
@@ -339,22 +340,41 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v)
   return (uint32_t)(__builtin_amdgcn_readlane((int)v, 15) | __builtin_amdgcn_readlane((int)v, 31) |
                     __builtin_amdgcn_readlane((int)v, 47) | __builtin_amdgcn_readlane((int)v, 63));
 }
-// the end of a collision kernel: each lane's count and the OR of its voxels' bits into
-// the call's counters; waves without a hit (most) leave at once
+// the end of a collision kernel of 256 threads: each lane's count and the OR of its
+// voxels' bits into the call's counters, one atomic per block and word (atomics on one
+// address take their turn, about 11 ns each); blocks without a hit (most) leave at once
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v);
 __device__ __forceinline__ void add_hits(uint64_t c, const uint32_t (&acc)[8], unsigned long long* count, uint32_t* mask)
 {
-  if (wave_ballot(c != 0ull) == 0ull) return;
+  __shared__ unsigned long long sc[4];
+  __shared__ uint32_t sm[4][8];
+  if (!__syncthreads_or(c != 0ull)) return;
   c = wave_sum_u64(c);
   uint32_t m[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) m[k] = wave_or(acc[k]);
+  const uint32_t w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    atomicAdd(count, (unsigned long long)c);
+    sc[w] = c;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (m[k]) atomicOr(mask + k, m[k]);
+    for (int k = 0; k < 8; ++k) sm[w][k] = m[k];
   }
+  __syncthreads();
+  if (threadIdx.x < 8) {
+    const uint32_t v = sm[0][threadIdx.x] | sm[1][threadIdx.x] | sm[2][threadIdx.x] | sm[3][threadIdx.x];
+    if (v) atomicOr(mask + threadIdx.x, v);
+  } else if (threadIdx.x == 8) {
+    atomicAdd(count, sc[0] + sc[1] + sc[2] + sc[3]);
+  }
+}
+__device__ __forceinline__ void add_count(uint64_t c, unsigned long long* count)
+{
+  __shared__ unsigned long long sc[4];
+  if (!__syncthreads_or(c != 0ull)) return;
+  c = wave_sum_u64(c);
+  if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(count, sc[0] + sc[1] + sc[2] + sc[3]);
 }
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
 {

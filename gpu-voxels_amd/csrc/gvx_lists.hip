@@ -165,6 +165,26 @@ __global__ void __launch_bounds__(256) k_copy_entries(const uint32_t* __restrict
   }
 }
 
+// the entries into other device buffers (any may be null): one launch for the three arrays
+// (a copy call each took three launches), 4-byte words since the caller's buffers need no
+// wider alignment
+__global__ void __launch_bounds__(256) k_read_entries(uint64_t n, const uint32_t* __restrict__ ids,
+                                                      const uint32_t* __restrict__ coords,
+                                                      const uint32_t* __restrict__ bits, uint32_t* __restrict__ oids,
+                                                      uint32_t* __restrict__ ocoords, uint32_t* __restrict__ obits)
+{
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 12 * n; i += stride) {
+    if (i < 8 * n) {
+      if (obits) obits[i] = bits[i];
+    } else if (i < 11 * n) {
+      if (ocoords) ocoords[i - 8 * n] = coords[i - 8 * n];
+    } else if (oids) {
+      oids[i - 11 * n] = ids[i - 11 * n];
+    }
+  }
+}
+
 // ---------------------------------------------------------------- LSD radix sort (8-bit digits)
 constexpr int RS_BLOCK = 256, RS_ROUNDS = 16, RS_TILE = RS_BLOCK * RS_ROUNDS;
 
@@ -350,118 +370,317 @@ static int radix_sort(ListS* L, uint32_t* keys, uint32_t* vals, uint64_t n)
 // For lists whose ids lie in [0, dx*dy*dz): mark every id in a bitmap of the map
 // (one bit per voxel, zero at rest), rank = occupied voxels before the id (prefix of
 // the words' popcounts + popcount inside the word), so entries land sorted by id
-// with duplicates on one slot, where their payloads are ORed and their (identical)
-// id and coordinates written.  Same output as sort + run-length OR.
-__global__ void __launch_bounds__(256) k_lu_mark(const uint32_t* __restrict__ ids, const uint32_t* __restrict__ keep,
-                                                 uint64_t keep_from, uint64_t n, unsigned long long* __restrict__ bm)
+// with duplicates on one slot, where their payloads are ORed.  Same output as sort +
+// run-length OR.  Four kernels, each bound by launch latency at the usual sizes (50 k
+// points into a 128^3 list: 7.5 + 2.6 + 7.6 + 4.3 us; twelve launches that wrote every
+// point as an entry, scanned per word and copied the result back took 37 us):
+//   mark     ids of the new points (kept for the last kernel) and of the list's entries
+//   tiles    occupied voxels per tile of LU_TILE words
+//   emit     a block per tile: the sum of the tiles before it, the prefix of its words,
+//            then one thread per entry writes id, coordinates and an empty payload;
+//            occupied words are saved with their prefix for the last kernel and cleared
+//   payload  every point and old entry ORs its bits into its voxel's entry
+// words per block: 4 per thread, or 1 for maps of few words, whose 1024-word tiles would
+// be few blocks with many entries each (128^3, 32 tiles: emit 11.9 us; 128 tiles: 7.6 us)
+constexpr int LU_TILE = 1024, LU_TILE_SMALL = 256;
+constexpr uint64_t LU_SMALL_WORDS = 1ull << 18;
+constexpr uint64_t LU_DIRECT = 4096;   // tiles up to which every emit block sums the ones before it itself
+constexpr uint32_t LU_OUT = 0xFFFFFFFFu;  // a point outside the map (the map has at most 2^32 - 1 voxels here)
+
+// what goes into the list: its entries [0, n_old) and n new points or coordinates, whose
+// meanings come from a table of clouds (small: by value, else in memory) or are all one
+constexpr uint32_t LU_CLOUDS = 16;
+struct LuSource {
+  const uint32_t* old_ids = nullptr;
+  const uint32_t* old_bits = nullptr;
+  uint64_t n_old = 0;
+  const float* pts = nullptr;
+  const uint32_t* crd = nullptr;
+  uint64_t n = 0;
+  const uint32_t* ends = nullptr;
+  const uint32_t* meanings = nullptr;
+  uint32_t ncl = 0, meaning = 0;
+  bool small = false;
+  uint32_t s_ends[LU_CLOUDS], s_meanings[LU_CLOUDS];
+};
+
+__global__ void __launch_bounds__(256) k_lu_mark(const LuSource src, uint32_t dx, uint32_t dy, uint32_t dz, float side,
+                                                 uint32_t* __restrict__ pid, unsigned long long* __restrict__ bm)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const bool in = i < keep_from || keep[i - keep_from] != 0u;
-    const uint32_t id = in ? ids[i] : 0u;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < src.n_old + src.n; i += stride) {
+    uint32_t id;
+    bool in = true;
+    if (i < src.n_old) {
+      id = src.old_ids[i];
+    } else {
+      const uint64_t k = i - src.n_old;
+      uint32_t x, y, z;
+      if (src.pts) {
+        x = quantize(src.pts[3 * k], side);
+        y = quantize(src.pts[3 * k + 1], side);
+        z = quantize(src.pts[3 * k + 2], side);
+      } else {
+        x = src.crd[3 * k];
+        y = src.crd[3 * k + 1];
+        z = src.crd[3 * k + 2];
+      }
+      in = x < dx && y < dy && z < dz;
+      id = (z * dy + y) * dx + x;
+      pid[k] = in ? id : LU_OUT;
+    }
     // neighbouring points of an image often share a voxel: one atomic per run of lanes
     if (wave_run_head(in, id, 0u)) atomicOr(bm + (id >> 6), 1ull << (id & 63));
   }
 }
 
-__global__ void __launch_bounds__(256) k_lu_popc(const unsigned long long* __restrict__ bm, uint64_t words,
-                                                 uint32_t* __restrict__ pc)
+// a thread's WPT consecutive words of its block's tile
+template <int WPT>
+__device__ __forceinline__ void lu_words(const unsigned long long* __restrict__ bm, unsigned long long (&w)[WPT])
 {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < words; w += stride)
-    pc[w] = (uint32_t)__popcll(bm[w]);
-}
-
-__global__ void __launch_bounds__(256) k_lu_scatter(const uint32_t* __restrict__ ids, const uint32_t* __restrict__ coords,
-                                                    const uint32_t* __restrict__ bits, const uint32_t* __restrict__ keep,
-                                                    uint64_t keep_from, uint64_t n,
-                                                    const unsigned long long* __restrict__ bm,
-                                                    const uint32_t* __restrict__ wpre, uint32_t* __restrict__ oids,
-                                                    uint32_t* __restrict__ ocoords, uint32_t* __restrict__ obits)
-{
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    if (i >= keep_from && !keep[i - keep_from]) continue;
-    const uint32_t id = ids[i];
-    const uint64_t o = wpre[id >> 6] + (uint32_t)__popcll(bm[id >> 6] & ((1ull << (id & 63)) - 1ull));
-    oids[o] = id;
-    ocoords[3 * o] = coords[3 * i];
-    ocoords[3 * o + 1] = coords[3 * i + 1];
-    ocoords[3 * o + 2] = coords[3 * i + 2];
-    const uint4* b = reinterpret_cast<const uint4*>(bits + 8 * i);
-    const uint4 a0 = b[0], a1 = b[1];
-    const uint32_t v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+  const uint64_t at = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * WPT;
+  if constexpr (WPT == 4) {
+    const ulonglong2 a = reinterpret_cast<const ulonglong2*>(bm + at)[0], b = reinterpret_cast<const ulonglong2*>(bm + at)[1];
+    w[0] = a.x; w[1] = a.y; w[2] = b.x; w[3] = b.y;
+  } else {
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (v[k]) atomicOr(obits + 8 * o + k, v[k]);
+    for (int k = 0; k < WPT; ++k) w[k] = bm[at + k];
   }
 }
 
-__global__ void __launch_bounds__(256) k_lu_clear(const uint32_t* __restrict__ ids, const uint32_t* __restrict__ keep,
-                                                  uint64_t keep_from, uint64_t n, unsigned long long* __restrict__ bm)
+// sum of v over the block's 256 threads, in every thread
+__device__ __forceinline__ uint32_t lu_block_sum(uint32_t v, uint32_t* lds)
 {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-    if (i < keep_from || keep[i - keep_from]) bm[ids[i] >> 6] = 0ull;  // dropped entries may hold any id
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = lds[0] + lds[1] + lds[2] + lds[3];
+  __syncthreads();
+  return v;
 }
 
-// the bitmap (zero at rest) and the per-word counts and prefix, shared by all lists
-// (list calls hold the runtime lock)
-static int lu_buffers(uint64_t words, unsigned long long** bm, uint32_t** pc, uint32_t** wpre)
+template <int WPT>
+__global__ void __launch_bounds__(256) k_lu_tiles(const unsigned long long* __restrict__ bm, uint32_t* __restrict__ sums)
 {
-  static unsigned long long* b = nullptr;
-  static uint32_t *c = nullptr, *p = nullptr;
+  __shared__ uint32_t lds[4];
+  unsigned long long w[WPT];
+  lu_words<WPT>(bm, w);
+  uint32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < WPT; ++k) c += (uint32_t)__popcll(w[k]);
+  const uint32_t t = lu_block_sum(c, lds);
+  if (threadIdx.x == 0) sums[blockIdx.x] = t;
+}
+
+// position of the k-th (from 0) set bit of w
+__device__ __forceinline__ uint32_t lu_select(unsigned long long w, uint32_t k)
+{
+  uint32_t v = (uint32_t)w, pos = 0, c = (uint32_t)__popc(v);
+  if (k >= c) { k -= c; v = (uint32_t)(w >> 32); pos = 32; }
+#pragma unroll
+  for (uint32_t half = 16; half >= 1; half >>= 1) {
+    c = (uint32_t)__popc(v & ((1u << half) - 1u));
+    if (k >= c) { k -= c; v >>= half; pos += half; }
+  }
+  return pos;
+}
+
+// sums: per tile, or (scanned) their exclusive prefix.  count: total to the device and to
+// pinned host memory.
+template <int WPT>
+__global__ void __launch_bounds__(256) k_lu_emit(unsigned long long* __restrict__ bm, const uint32_t* __restrict__ sums,
+                                                 bool scanned, UDiv dxd, UDiv dyd, uint32_t* __restrict__ wpre,
+                                                 unsigned long long* __restrict__ wcopy, uint32_t* __restrict__ oids,
+                                                 uint32_t* __restrict__ ocoords, uint32_t* __restrict__ obits,
+                                                 uint32_t* __restrict__ count_dev, uint32_t* __restrict__ count_host)
+{
+  __shared__ uint32_t lds[4];
+  constexpr int TILE = 256 * WPT;
+  __shared__ uint32_t sp[TILE];            // prefix of each word inside the tile
+  __shared__ unsigned long long sw[TILE];  // the words
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint64_t at = ((uint64_t)blockIdx.x * 256 + tid) * WPT;
+  unsigned long long wd[WPT];
+  lu_words<WPT>(bm, wd);
+  uint32_t before = 0;
+  if (scanned) {
+    before = sums[blockIdx.x];
+  } else {
+    for (uint32_t t = tid; t < blockIdx.x; t += 256) before += sums[t];
+    before = lu_block_sum(before, lds);
+  }
+  // exclusive prefix of the threads' words
+  uint32_t mine = 0;
+#pragma unroll
+  for (int k = 0; k < WPT; ++k) mine += (uint32_t)__popcll(wd[k]);
+  uint32_t incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o);
+    if (lane >= (uint32_t)o) incl += y;
+  }
+  if (lane == 63) lds[tid >> 6] = incl;
+  __syncthreads();
+  uint32_t pre = incl - mine, total = 0;
+  for (uint32_t w = 0; w < 4; ++w) {
+    if (w < tid >> 6) pre += lds[w];
+    total += lds[w];
+  }
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) {
+    *count_dev = before + total;
+    __hip_atomic_store(count_host, before + total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (total == 0u) return;  // uniform over the block
+#pragma unroll
+  for (int k = 0; k < WPT; ++k) {
+    sp[WPT * tid + k] = pre;
+    sw[WPT * tid + k] = wd[k];
+    if (wd[k]) {
+      wpre[at + k] = before + pre;
+      wcopy[at + k] = wd[k];
+      bm[at + k] = 0ull;
+    }
+    pre += (uint32_t)__popcll(wd[k]);
+  }
+  __syncthreads();
+  for (uint32_t e = tid; e < total; e += 256) {
+    uint32_t lo = 0, hi = TILE;  // the last word whose prefix is at most e holds entry e
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (sp[mid] <= e) lo = mid; else hi = mid;
+    }
+    const uint32_t id = (blockIdx.x * (uint32_t)TILE + lo) * 64u + lu_select(sw[lo], e - sp[lo]);
+    const uint64_t o = (uint64_t)before + e;
+    uint32_t x, y;
+    const uint32_t z = dyd.div(dxd.div(id, x), y);
+    oids[o] = id;
+    ocoords[3 * o] = x;
+    ocoords[3 * o + 1] = y;
+    ocoords[3 * o + 2] = z;
+    uint4* ob = reinterpret_cast<uint4*>(obits + 8 * o);
+    ob[0] = make_uint4(0u, 0u, 0u, 0u);
+    ob[1] = make_uint4(0u, 0u, 0u, 0u);
+  }
+}
+
+__global__ void __launch_bounds__(256) k_lu_payload(const LuSource src, const uint32_t* __restrict__ pid,
+                                                    const uint32_t* __restrict__ wpre,
+                                                    const unsigned long long* __restrict__ wcopy,
+                                                    uint32_t* __restrict__ obits)
+{
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  auto slot = [&](uint32_t id) {
+    return (uint64_t)(wpre[id >> 6] + (uint32_t)__popcll(wcopy[id >> 6] & ((1ull << (id & 63)) - 1ull)));
+  };
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < src.n_old + src.n; i += stride) {
+    if (i < src.n_old) {
+      const uint64_t o = slot(src.old_ids[i]);
+      const uint4* b = reinterpret_cast<const uint4*>(src.old_bits + 8 * i);
+      const uint4 a0 = b[0], a1 = b[1];
+      const uint32_t v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (v[k]) atomicOr(obits + 8 * o + k, v[k]);
+      continue;
+    }
+    const uint64_t k = i - src.n_old;
+    const uint32_t id = pid[k];
+    uint32_t m = src.meaning;
+    if (src.small) {
+      m = src.s_meanings[0];
+#pragma unroll
+      for (uint32_t c = 1; c < LU_CLOUDS; ++c)
+        if (c < src.ncl && k >= src.s_ends[c - 1]) m = src.s_meanings[c];
+    } else if (src.ends) {
+      uint32_t lo = 0, hi = src.ncl - 1;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if ((uint64_t)src.ends[mid] > k) hi = mid; else lo = mid + 1;
+      }
+      m = src.meanings[lo];
+    }
+    if (wave_run_head(id != LU_OUT, id, m)) atomicOr(obits + 8 * slot(id) + (m >> 5), 1u << (m & 31));
+  }
+}
+
+// the bitmap (zero at rest), the saved words with their prefixes and the tiles' counts,
+// shared by all lists (list calls hold the runtime lock); whole tiles
+struct LuBuffers {
+  unsigned long long *bm = nullptr, *wcopy = nullptr;
+  uint32_t *wpre = nullptr, *sums = nullptr, *offs = nullptr;
+};
+static int lu_buffers(uint64_t map_words, LuBuffers* out)
+{
+  static LuBuffers b;
   static uint64_t cap = 0;
-  if (cap < words) {
+  if (cap < map_words) {
     GVX_CHECK(sync());
-    dfree(b); dfree(c); dfree(p);
-    b = nullptr; c = nullptr; p = nullptr;
+    dfree(b.bm); dfree(b.wcopy); dfree(b.wpre); dfree(b.sums); dfree(b.offs);
+    b = LuBuffers();
     cap = 0;
-    GVX_CHECK(dalloc((void**)&b, words * 8));
-    GVX_CHECK(dalloc((void**)&c, words * 4));
-    GVX_CHECK(dalloc((void**)&p, (words + 1) * 4));
-    GVX_CHECK(fill_u32(b, 0u, words * 2));
+    const uint64_t words = (map_words + LU_TILE - 1) / LU_TILE * LU_TILE, tiles = words / LU_TILE_SMALL;
+    GVX_CHECK(dalloc((void**)&b.bm, words * 8));
+    GVX_CHECK(dalloc((void**)&b.wcopy, words * 8));
+    GVX_CHECK(dalloc((void**)&b.wpre, words * 4));
+    GVX_CHECK(dalloc((void**)&b.sums, tiles * 4));
+    GVX_CHECK(dalloc((void**)&b.offs, tiles * 4));
+    GVX_CHECK(fill_u32(b.bm, 0u, words * 2));
     cap = words;
   }
-  *bm = b; *pc = c; *wpre = p;
+  *out = b;
   return GVX_OK;
 }
 
 static bool lu_suits(const ListS* L, uint64_t entries)
 {
   const uint64_t nv = nvox3(L->dims);
-  if (!L->ids_in_range || nv > (1ull << 32) || entries == 0) return false;
+  if (!L->ids_in_range || nv >= (1ull << 32) || entries == 0) return false;
   const uint64_t words = (nv + 63) / 64;
   return words <= (1ull << 16) || words <= 64 * entries;
 }
 
-// entries [0, n) of L (entries from keep_from on only where keep[i - keep_from]) ->
-// the sorted, duplicate-free list
-static int lu_unique(ListS* L, uint64_t n, const uint32_t* keep, uint64_t keep_from)
+// the sorted, duplicate-free list of src (buffers reserved for n_old + n entries)
+static int lu_unique(ListS* L, LuSource& src)
 {
   hipStream_t s = rt().stream;
   ProfScope ps("list_make_unique");
-  const uint64_t words = (nvox3(L->dims) + 63) / 64;
-  unsigned long long* bm = nullptr;
-  uint32_t *pc = nullptr, *wpre = nullptr;
-  GVX_CHECK(lu_buffers(words, &bm, &pc, &wpre));
-  const unsigned gn = grid_for(n, 256, 4096), gw = grid_for(words, 256, 8192);
-  hipLaunchKernelGGL(k_lu_mark, dim3(gn), dim3(256), 0, s, L->ids, keep, keep_from, n, bm);
-  hipLaunchKernelGGL(k_lu_popc, dim3(gw), dim3(256), 0, s, bm, words, pc);
+  const uint64_t words = (nvox3(L->dims) + 63) / 64, n = src.n_old + src.n;
+  const bool few = words <= LU_SMALL_WORDS;
+  const uint64_t per = few ? LU_TILE_SMALL : LU_TILE, tiles = (words + per - 1) / per;
+  LuBuffers B;
+  GVX_CHECK(lu_buffers(words, &B));
+  src.old_ids = L->ids;
+  src.old_bits = L->bits;
+  uint32_t* pid = L->flags;
+  const unsigned gn = grid_for(n, 256, 4096);
+  hipLaunchKernelGGL(k_lu_mark, dim3(gn), dim3(256), 0, s, src, L->dims[0], L->dims[1], L->dims[2], L->side, pid,
+                     B.bm);
+  if (few) hipLaunchKernelGGL(k_lu_tiles<1>, dim3((unsigned)tiles), dim3(256), 0, s, B.bm, B.sums);
+  else hipLaunchKernelGGL(k_lu_tiles<4>, dim3((unsigned)tiles), dim3(256), 0, s, B.bm, B.sums);
   GVX_HIP(hipGetLastError());
-  GVX_CHECK(scan_u32(pc, wpre, words, wpre + words));
-  GVX_CHECK(fill_u32(L->bits_t, 0u, n * 8));
-  hipLaunchKernelGGL(k_lu_scatter, dim3(gn), dim3(256), 0, s, L->ids, L->coords, L->bits, keep, keep_from, n, bm, wpre,
-                     L->ids_t, L->coords_t, L->bits_t);
-  hipLaunchKernelGGL(k_lu_clear, dim3(gn), dim3(256), 0, s, L->ids, keep, keep_from, n, bm);
+  const bool scanned = tiles > LU_DIRECT;
+  if (scanned) GVX_CHECK(scan_u32(B.sums, B.offs, tiles, nullptr));
+  // an empty list's entries are written in place; otherwise they are merged beside the old
+  // ones, which the payload kernel still reads, and copied back
+  const bool beside = src.n_old != 0;
+  uint32_t *oi = beside ? L->ids_t : L->ids, *oc = beside ? L->coords_t : L->coords, *ob = beside ? L->bits_t : L->bits;
+  uint32_t *count_dev = nullptr, *count_host = nullptr;
+  result_word(&count_dev, &count_host);
+#define LU_EMIT(WPT)                                                                                               \
+  hipLaunchKernelGGL(k_lu_emit<WPT>, dim3((unsigned)tiles), dim3(256), 0, s, B.bm, scanned ? B.offs : B.sums, scanned, \
+                     udiv(L->dims[0]), udiv(L->dims[1]), B.wpre, B.wcopy, oi, oc, ob, count_dev, count_host)
+  if (few) LU_EMIT(1);
+  else LU_EMIT(4);
+#undef LU_EMIT
+  hipLaunchKernelGGL(k_lu_payload, dim3(gn), dim3(256), 0, s, src, pid, B.wpre, B.wcopy, ob);
   // the unique count stays on the device for the copy back; the host reads it after
   // the call's one synchronisation (no wait in the middle of the call)
-  hipLaunchKernelGGL(k_copy_entries, dim3(gn), dim3(256), 0, s, wpre + words, n, L->ids_t, L->coords_t, L->bits_t,
-                     L->ids, L->coords, L->bits);
+  if (beside)
+    hipLaunchKernelGGL(k_copy_entries, dim3(gn), dim3(256), 0, s, count_dev, n, L->ids_t, L->coords_t, L->bits_t,
+                       L->ids, L->coords, L->bits);
   GVX_HIP(hipGetLastError());
-  GVX_HIP(hipMemcpyAsync(rt().host_small, wpre + words, 4, hipMemcpyDeviceToHost, s));
   GVX_CHECK(sync());
-  L->n = *(const uint32_t*)rt().host_small;
+  L->n = *static_cast<volatile uint32_t*>(count_host);
   return GVX_OK;
 }
 
@@ -472,7 +691,9 @@ static int make_unique(ListS* L)
   if (n == 0) return GVX_OK;
   if (lu_suits(L, n)) {
     GVX_CHECK(tmp_reserve(L, n));
-    return lu_unique(L, n, nullptr, n);
+    LuSource src;
+    src.n_old = n;
+    return lu_unique(L, src);
   }
   GVX_CHECK(tmp_reserve(L, n));
   hipStream_t s = rt().stream;
@@ -736,18 +957,40 @@ static int64_t signed_index(const uint32_t d[3], const int32_t* o)
   return (int64_t)o[2] * (int64_t)d[0] * (int64_t)d[1] + (int64_t)o[1] * (int64_t)d[0] + (int64_t)o[0];
 }
 
-// append points already on the device (cloud table on the device too), then
-// remove_out_of_bounds and make_unique; does not touch the staging buffer
-int list_insert_device(void* lv, const float* dp, uint64_t n, const uint32_t* ends, uint32_t ncl,
-                       const uint32_t* meanings, uint32_t meaning)
+// append points already on the device, with one meaning, a cloud table on the device
+// (ends, meanings) or a small one on the host (tab: ncl ends, then ncl meanings), then
+// remove_out_of_bounds and make_unique; does not touch the staging buffer.  A host table
+// is used only where list_takes_table(l, n, ncl).
+static bool list_takes_table(const ListS* l, uint64_t n, uint32_t ncl)
 {
-  ListS* l = static_cast<ListS*>(static_cast<gvx_list_s*>(lv));
+  return ncl <= LU_CLOUDS && lu_suits(l, l->n + n);
+}
+
+static int list_insert(ListS* l, const float* dp, uint64_t n, const uint32_t* ends, uint32_t ncl,
+                       const uint32_t* meanings, uint32_t meaning, const uint32_t* tab)
+{
   if (n == 0) return GVX_OK;
   std::lock_guard<std::recursive_mutex> g(l->mu);
   std::lock_guard<std::recursive_mutex> g2(rt().mu);
   const uint64_t base = l->n;
   GVX_CHECK(list_reserve(l, base + n));
   GVX_CHECK(tmp_reserve(l, base + n));
+  if (lu_suits(l, base + n)) {  // out-of-map points are not marked
+    LuSource src;
+    src.n_old = base;
+    src.pts = dp;
+    src.n = n;
+    src.ends = ends;
+    src.meanings = meanings;
+    src.ncl = ncl;
+    src.meaning = meaning;
+    if (tab) {
+      src.small = true;
+      memcpy(src.s_ends, tab, ncl * 4);
+      memcpy(src.s_meanings, tab + ncl, ncl * 4);
+    }
+    return lu_unique(l, src);
+  }
   {
     ProfScope ps("list_insert_points");
     hipLaunchKernelGGL(k_list_points, dim3(grid_for(n, 256, 1u << 16)), dim3(256), 0, rt().stream, dp, n, l->dims[0],
@@ -755,9 +998,14 @@ int list_insert_device(void* lv, const float* dp, uint64_t n, const uint32_t* en
                        l->coords + 3 * base, l->bits + 8 * base, l->flags);
     GVX_HIP(hipGetLastError());
   }
-  if (lu_suits(l, base + n)) return lu_unique(l, base + n, l->flags, base);  // out-of-map points: keep flag 0
   GVX_CHECK(compact_tail(l, base, n));
   return make_unique(l);
+}
+
+int list_insert_device(void* lv, const float* dp, uint64_t n, const uint32_t* ends, uint32_t ncl,
+                       const uint32_t* meanings, uint32_t meaning)
+{
+  return list_insert(static_cast<ListS*>(static_cast<gvx_list_s*>(lv)), dp, n, ends, ncl, meanings, meaning, nullptr);
 }
 
 }  // namespace gvx
@@ -847,6 +1095,12 @@ int gvx_list_read(gvx_list l, uint32_t* ids, uint32_t* coords, uint8_t* bits, in
 {
   GVX_CHECK(check_list(l));
   std::lock_guard<std::recursive_mutex> g(l->mu);
+  if (mem == GVX_MEM_DEVICE && l->n && (((uintptr_t)ids | (uintptr_t)coords | (uintptr_t)bits) & 3) == 0) {
+    hipLaunchKernelGGL(k_read_entries, dim3(grid_for(12 * l->n, 256, 8192)), dim3(256), 0, rt().stream, l->n, l->ids,
+                       l->coords, l->bits, ids, coords, (uint32_t*)bits);
+    GVX_HIP(hipGetLastError());
+    return sync();
+  }
   if (ids) GVX_CHECK(copy_out(ids, l->ids, l->n * 4, mem));
   if (coords) GVX_CHECK(copy_out(coords, l->coords, l->n * 12, mem));
   if (bits) GVX_CHECK(copy_out(bits, l->bits, l->n * 32, mem));
@@ -885,6 +1139,8 @@ int gvx_list_insert_points(gvx_list l, const float* xyz, uint64_t n, const uint3
     return fail(GVX_ERR_BAD_ARG, "meaning > 255");
   }
   if (n == 0) return GVX_OK;
+  // the list's lock first: its size decides the path
+  std::lock_guard<std::recursive_mutex> g(l->mu);
   std::lock_guard<std::recursive_mutex> g2(rt().mu);
   size_t pb = (n * 12 + 255) & ~(size_t)255;
   void* st = nullptr;
@@ -894,6 +1150,8 @@ int gvx_list_insert_points(gvx_list l, const float* xyz, uint64_t n, const uint3
     GVX_HIP(hipMemcpyAsync(st, xyz, n * 12, hipMemcpyHostToDevice, rt().stream));
     dp = (const float*)st;
   }
+  if (!tab.empty() && list_takes_table(l, n, ncl))  // a few clouds go along with the launch
+    return list_insert(l, dp, n, nullptr, ncl, nullptr, meaning, tab.data());
   uint32_t* dtab = nullptr;
   if (!tab.empty()) {
     dtab = (uint32_t*)((char*)st + pb);
@@ -915,11 +1173,18 @@ int gvx_list_insert_coords(gvx_list l, const uint32_t* xyz, uint64_t n, uint32_t
   GVX_CHECK(tmp_reserve(l, base + n));
   const void* d = nullptr;
   GVX_CHECK(stage_input(xyz, n * 12, mem, &d));
+  if (lu_suits(l, base + n)) {
+    LuSource src;
+    src.n_old = base;
+    src.crd = (const uint32_t*)d;
+    src.n = n;
+    src.meaning = meaning;
+    return lu_unique(l, src);
+  }
   hipLaunchKernelGGL(k_list_coords, dim3(grid_for(n, 256, 1u << 16)), dim3(256), 0, rt().stream, (const uint32_t*)d,
                      n, l->dims[0], l->dims[1], l->dims[2], meaning, l->ids + base, l->coords + 3 * base,
                      l->bits + 8 * base, l->flags);
   GVX_HIP(hipGetLastError());
-  if (lu_suits(l, base + n)) return lu_unique(l, base + n, l->flags, base);
   GVX_CHECK(compact_tail(l, base, n));
   return make_unique(l);
 }

@@ -179,9 +179,7 @@ __global__ void __launch_bounds__(256) k_collide_bits(uint8_t* __restrict__ a, c
       ++c;
     }
   });
-  if (wave_ballot(c != 0ull) == 0ull) return;
-  c = wave_sum_u64(c);
-  if ((threadIdx.x & 63) == 0) atomicAdd(count, (unsigned long long)c);
+  add_count(c, count);
 }
 
 constexpr int kLoadsInFlight = 4;  // per lane, in the kernels that stream a ProbVoxelMap
@@ -263,9 +261,7 @@ __global__ void __launch_bounds__(256) k_collide_prob(uint8_t* __restrict__ a, c
       });
     }
   }
-  if (wave_ballot(c != 0ull) == 0ull) return;
-  c = wave_sum_u64(c);
-  if ((threadIdx.x & 63) == 0) atomicAdd(count, (unsigned long long)c);
+  add_count(c, count);
 }
 
 // kernelCollideVoxelMapsBitvector (VoxelMapOperations.hpp:187-239) with SVCollider,

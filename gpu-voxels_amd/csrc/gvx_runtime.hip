@@ -188,9 +188,9 @@ int fill_bytes(void* dst, uint8_t value, uint64_t n_bytes)
 
 // ---------------------------------------------------------------- results of a call
 // dev_small: [0, 1024) free scratch of the entry points, [1024, 1088) result counters
-// (zero between calls), [1088, 1092) the outside flag's device word.  host_small: [0,
-// 1024) free, [1024, 1088) results, [1088, 1092) the outside flag.
-constexpr size_t RES_AT = 1024, FLAG_AT = 1088;
+// (zero between calls), [1088, 1092) the outside flag's device word, [1092, 1096)
+// result_word.  host_small: the same on the host.
+constexpr size_t RES_AT = 1024, FLAG_AT = 1088, WORD_AT = 1092;
 
 __global__ void k_results(uint32_t* __restrict__ dev, uint32_t* __restrict__ host)
 {
@@ -215,6 +215,12 @@ int results_fetch(uint64_t* count, uint8_t* mask)
   memcpy(count, h, 8);
   if (mask) memcpy(mask, h + 8, 32);
   return GVX_OK;
+}
+
+void result_word(uint32_t** dev, uint32_t** host)
+{
+  *dev = (uint32_t*)((char*)rt().dev_small + WORD_AT);
+  *host = (uint32_t*)((char*)rt().host_small + WORD_AT);
 }
 
 OutsideFlag outside_flag()

@@ -228,3 +228,34 @@ def test_unique_fallback_paths(gvx_lib):
     a.clear(); oa = O.List(dims, side)
     a.insert_points(pc, meaning=4); oa.insert_points(pc, meaning=4)     # cleared: bitmap path again
     _same(a, oa)
+
+
+@pytest.mark.parametrize("d", [(1, 1, 1), (63, 1, 1), (64, 32, 32), (65, 33, 31), (300, 200, 150),
+                               (1024, 1024, 300)])
+@pytest.mark.parametrize("clouds", [1, 2, 16, 17])
+def test_bitmap_unique_edges(gvx_lib, d, clouds):
+    """Tiles, words and tables of the dense-bitmap unique: empty and filled lists, points outside,
+    empty clouds, more clouds than go along with the launch."""
+    gvx = gvx_lib
+    rng = np.random.default_rng(sum(d) + clouds)
+    side = 0.01
+    n = max(40, int(np.prod(d)) // 4000)
+    lst = gvx.VoxelList(d, side)
+    want = {}
+    for _ in range(3):
+        pts = rng.uniform(-0.02, np.array(d) * side + 0.02, (n, 3)).astype(np.float32)
+        cuts = np.sort(rng.integers(0, n + 1, clouds - 1))
+        sizes = np.diff(np.concatenate([[0], cuts, [n]])).astype(np.uint32)
+        meanings = rng.integers(0, 256, clouds).astype(np.uint32)
+        lst.insert_points(pts, sizes=sizes, meanings=meanings)
+        m = np.repeat(meanings, sizes)
+        v = np.floor(pts / np.float32(side))
+        v = np.maximum(v, 0)  # negative coordinates saturate to 0 as the GPU cast does
+        ok = (v < np.array(d)).all(axis=1)
+        ids = (v[ok] @ np.array([1, d[0], d[0] * d[1]])).astype(np.int64)
+        for i, b in zip(ids, m[ok]):
+            want[int(i)] = want.get(int(i), 0) | 1 << int(b)
+        got_ids, got_coords, got_bits = lst.read()
+        assert np.array_equal(got_ids, np.array(sorted(want), np.uint32))
+        assert np.array_equal(got_coords @ np.array([1, d[0], d[0] * d[1]]), got_ids)
+        assert [int.from_bytes(b.tobytes(), "little") for b in got_bits] == [want[k] for k in sorted(want)]
