@@ -1,4 +1,6 @@
 // gvx_maps.hip -- dense voxel maps: create/clear, voxelization, map x map collision.
+#include <algorithm>
+
 #include "gvx_internal.hpp"
 
 namespace gvx {
@@ -545,11 +547,19 @@ __device__ __forceinline__ void prob_add_n(uint8_t* map, uint64_t idx, int delta
 // rule).  The representative of a voxel is its lowest-indexed point, so the
 // representatives keep the image order (neighbouring lanes walk neighbouring rays).
 //
+// counters of one scan: distinct targets, (ray, brick) pairs, chunks of pairs, bricks with
+// several chunks; cleared by the tag kernel
+struct SensorState {
+  uint32_t targets, pairs, chunks, split;
+};
+
 // tag: hits[voxel] = max over its points of ~i (hits is zero at rest)
 __global__ void __launch_bounds__(256) k_sensor_tag(uint32_t* __restrict__ hits, uint32_t dx, uint32_t dy, uint32_t dz,
                                                     float side, bool sensor_in, const float* __restrict__ pts,
-                                                    uint64_t n, const uint8_t* __restrict__ robot, uint32_t robot_bit)
+                                                    uint64_t n, const uint8_t* __restrict__ robot, uint32_t robot_bit,
+                                                    SensorState* __restrict__ st)
 {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *st = SensorState{0u, 0u, 0u, 0u};
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     uint32_t x = 0, y = 0, z = 0;
@@ -560,30 +570,58 @@ __global__ void __launch_bounds__(256) k_sensor_tag(uint32_t* __restrict__ hits,
   }
 }
 
-// rep[i] = 1 when point i is its voxel's representative
-__global__ void __launch_bounds__(256) k_sensor_rep(const uint32_t* __restrict__ hits, uint32_t dx, uint32_t dy,
-                                                    uint32_t dz, float side, bool sensor_in,
-                                                    const float* __restrict__ pts, uint64_t n,
-                                                    const uint8_t* __restrict__ robot, uint32_t robot_bit,
-                                                    uint32_t* __restrict__ rep)
+// the representatives, compacted: slot k holds a voxel (list), a weight to be counted and
+// pos[representative] = k.  A block's slots are consecutive and in image order
+// (neighbouring lanes walk neighbouring rays); blocks take theirs as they come (one
+// atomic each), which changes no result.  A scan of flags took five launches.
+constexpr int REP_BLOCK = 1024;
+__global__ void __launch_bounds__(REP_BLOCK) k_sensor_rep(const uint32_t* __restrict__ hits, uint32_t dx, uint32_t dy,
+                                                          uint32_t dz, float side, bool sensor_in,
+                                                          const float* __restrict__ pts, uint64_t n,
+                                                          const uint8_t* __restrict__ robot, uint32_t robot_bit,
+                                                          SensorState* __restrict__ st, uint32_t* __restrict__ pos,
+                                                          uint64_t* __restrict__ list, uint32_t* __restrict__ weight)
 {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    uint32_t x, y, z;
+  __shared__ uint32_t wsum[REP_BLOCK / 64], wbase;
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (uint64_t i0 = (uint64_t)blockIdx.x * REP_BLOCK; i0 < n; i0 += (uint64_t)gridDim.x * REP_BLOCK) {  // uniform
+    const uint64_t i = i0 + threadIdx.x;
+    uint32_t x = 0, y = 0, z = 0;
+    uint64_t v = 0;
     bool r = false;
-    if (sensor_point(pts + 3 * i, side, dx, dy, dz, sensor_in, robot, robot_bit, x, y, z))
-      r = hits[((uint64_t)z * dy + y) * dx + x] == ~(uint32_t)i;
-    rep[i] = r ? 1u : 0u;
+    if (i < n && sensor_point(pts + 3 * i, side, dx, dy, dz, sensor_in, robot, robot_bit, x, y, z)) {
+      v = ((uint64_t)z * dy + y) * dx + x;
+      r = hits[v] == ~(uint32_t)i;
+    }
+    const uint64_t bal = wave_ballot(r);
+    if (lane == 0) wsum[w] = (uint32_t)__popcll(bal);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t t = 0;
+      for (int k = 0; k < REP_BLOCK / 64; ++k) {
+        const uint32_t c = wsum[k];
+        wsum[k] = t;
+        t += c;
+      }
+      wbase = t ? atomicAdd(&st->targets, t) : 0u;
+    }
+    __syncthreads();
+    if (r) {
+      const uint32_t k = wbase + wsum[w] + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
+      pos[i] = k;
+      list[k] = v;
+      weight[k] = 0u;
+    }
+    __syncthreads();  // wsum and wbase are free again
   }
 }
 
-// weight[pos[r]] += 1 for every point of representative r; list[pos[r]] = voxel of r
+// weight[pos[r]] += 1 for every point of representative r
 __global__ void __launch_bounds__(256) k_sensor_weigh(const uint32_t* __restrict__ hits, uint32_t dx, uint32_t dy,
                                                       uint32_t dz, float side, bool sensor_in,
                                                       const float* __restrict__ pts, uint64_t n,
                                                       const uint8_t* __restrict__ robot, uint32_t robot_bit,
-                                                      const uint32_t* __restrict__ pos, uint64_t* __restrict__ list,
-                                                      uint32_t* __restrict__ weight)
+                                                      const uint32_t* __restrict__ pos, uint32_t* __restrict__ weight)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
@@ -591,24 +629,316 @@ __global__ void __launch_bounds__(256) k_sensor_weigh(const uint32_t* __restrict
     const bool in = sensor_point(pts + 3 * i, side, dx, dy, dz, sensor_in, robot, robot_bit, x, y, z);
     const uint64_t v = in ? ((uint64_t)z * dy + y) * dx + x : 0ull;
     const uint32_t run = wave_run_head(in, v, 0u);  // consecutive points in one voxel add their count once
-    if (!in) continue;
-    const uint32_t r = ~hits[v];
-    if (run) atomicAdd(weight + pos[r], run);
-    if (r == (uint32_t)i) list[pos[r]] = v;
+    if (run) atomicAdd(weight + pos[~hits[v]], run);
   }
 }
 
 // hits back to zero under the representatives' voxels
 __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hits, const uint64_t* __restrict__ list,
-                                                      const uint32_t* __restrict__ count)
+                                                      const SensorState* __restrict__ st)
 {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x, m = *count;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x, m = st->targets;
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < m; k += stride) hits[list[k]] = 0u;
 }
 
-// pass 1: one lane per distinct target voxel walks RayCaster::rayCast's 3-D
-// integer line (VoxelMapOperations.h:218-340) from the sensor voxel to the target
-// and adds the target's weight to the 32-bit counter of every cell it visits
+// ---- pass 1, by bricks.  Every cell of every distinct target's ray (RayCaster::rayCast's
+// 3-D integer line, VoxelMapOperations.h:218-340) adds the target's weight to a counter.
+// Added to counters in memory, even merged over runs of neighbouring lanes, these are 21 M
+// device-scope atomics for a 640 x 480 depth image in a 512^3 map (0.6-1.1 ms), which bound
+// the scan.  So the cells are counted where they lie: the map is cut into bricks of 16^3
+// voxels; each ray is cut into its stretches inside bricks ((ray, entry cell) pairs, about
+// one per 16 cells, found without walking: SENSORTIMES), the pairs are sorted by brick, and
+// a block walks a brick's pairs with the 4096 counters in LDS and updates the brick's
+// voxels itself.  Bricks near the sensor hold most rays: their pairs are cut into chunks of
+// SB_CHUNK, whose counters meet in memory (hits, zero at rest) before the voxels are
+// updated.
+//
+// The line steps along x when tx < ty and tx < tz, else along y when ty < tz, else along z,
+// where the i-th step of an axis of length d has the time t = (2i + 1) / (2d): the errors of
+// the integer walk are these comparisons multiplied out.  So the steps of all axes are one
+// sequence ordered by time (ties: z, then y, then x), and both the next brick boundary (the
+// earliest of three steps) and the position on the other axes at that moment (steps earlier
+// than it) have closed forms.
+constexpr uint32_t SB = 16, SB_CELLS = SB * SB * SB;
+constexpr uint32_t SB_CHUNK = 2048;      // pairs per block at a time
+constexpr uint32_t SB_EDGE = 32767;      // longest map edge: products of two step numbers fit 32 bits
+constexpr uint32_t SH_SLOTS = 2048;      // bricks a block of 256 rays counts in LDS
+constexpr uint32_t SH_NONE = 0xFFFFFFFFu;
+
+struct SensorGeom {
+  uint32_t s[3];       // sensor voxel
+  UDiv dxd, dyd;       // map dimensions
+  uint32_t bx, by;     // bricks along x and y
+};
+
+__device__ __forceinline__ void sensor_target(const SensorGeom& g, uint64_t v, uint32_t (&t)[3])
+{
+  t[2] = g.dyd.div(g.dxd.div((uint32_t)v, t[0]), t[1]);  // a map has at most 2^32 voxels
+}
+
+// emit(brick, cell inside it) for every brick that the ray from the sensor to t enters
+template <typename Emit>
+__device__ __forceinline__ void sensor_bricks(const SensorGeom& g, const uint32_t (&t)[3], Emit&& emit)
+{
+  uint32_t d[3], e[3], c[3];  // steps per axis, index of the step into the next brick, current cell
+  bool up[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    up[a] = t[a] > g.s[a];
+    d[a] = up[a] ? t[a] - g.s[a] : g.s[a] - t[a];
+    e[a] = up[a] ? SB - 1 - g.s[a] % SB : g.s[a] % SB;
+    c[a] = g.s[a];
+  }
+  for (;;) {
+    emit(((c[2] / SB) * g.by + c[1] / SB) * g.bx + c[0] / SB, ((c[2] % SB) * SB + c[1] % SB) * SB + c[0] % SB);
+    const bool h0 = e[0] < d[0], h1 = e[1] < d[1], h2 = e[2] < d[2];
+    if (!(h0 || h1 || h2)) return;
+    const uint32_t u0 = 2 * e[0] + 1, u1 = 2 * e[1] + 1, u2 = 2 * e[2] + 1;
+    const bool xy = h0 && (!h1 || u0 * d[1] < u1 * d[0]), xz = h0 && (!h2 || u0 * d[2] < u2 * d[0]);
+    const bool yz = h1 && (!h2 || u1 * d[2] < u2 * d[1]);
+    const int ax = xy && xz ? 0 : yz ? 1 : 2;
+    const uint32_t ua = ax == 0 ? u0 : ax == 1 ? u1 : u2, da = ax == 0 ? d[0] : ax == 1 ? d[1] : d[2];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      uint32_t k;  // steps of axis a up to and with this one
+      if (a == ax) {
+        k = e[a] + 1;
+        e[a] += SB;
+      } else {  // (2j + 1) / d[a] before ua / da, or with it when a comes first (a > ax)
+        k = d[a] == 0u ? 0u : ((ua * d[a] - (a > ax ? 0u : 1u)) / da + 1) / 2;
+      }
+      c[a] = up[a] ? g.s[a] + k : g.s[a] - k;
+    }
+  }
+}
+
+// a block's bricks with their pairs: slot of brick b, or SH_NONE when the table is full
+__device__ __forceinline__ uint32_t sensor_slot(uint32_t* keys, uint32_t b)
+{
+  uint32_t h = (b * 2654435761u) >> 21;  // SH_SLOTS = 2^11
+  for (int probe = 0; probe < 16; ++probe) {
+    const uint32_t k = keys[h];
+    if (k == b) return h;
+    if (k == SH_NONE) {
+      const uint32_t old = atomicCAS(&keys[h], SH_NONE, b);
+      if (old == SH_NONE || old == b) return h;
+    }
+    h = (h + 1) % SH_SLOTS;
+  }
+  return SH_NONE;
+}
+
+// pairs per brick: counted per block of 256 rays first (neighbouring rays share bricks).
+// Also clears the targets' tags.
+__global__ void __launch_bounds__(256) k_sensor_count(const SensorGeom g, const SensorState* __restrict__ st,
+                                                      const uint64_t* __restrict__ list, uint32_t* __restrict__ hits,
+                                                      uint32_t* __restrict__ cnt)
+{
+  __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
+  const uint32_t m = st->targets, k = blockIdx.x * 256 + threadIdx.x;
+  if (blockIdx.x * 256 >= m) return;  // uniform
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256) {
+    keys[i] = SH_NONE;
+    num[i] = 0u;
+  }
+  __syncthreads();
+  if (k < m) {
+    const uint64_t v = list[k];
+    hits[v] = 0u;
+    uint32_t t[3];
+    sensor_target(g, v, t);
+    sensor_bricks(g, t, [&](uint32_t b, uint32_t) {
+      const uint32_t h = sensor_slot(keys, b);
+      if (h != SH_NONE) atomicAdd(&num[h], 1u);
+      else atomicAdd(cnt + b, 1u);
+    });
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256)
+    if (num[i]) atomicAdd(cnt + keys[i], num[i]);
+}
+
+// places of the bricks' pairs (any order of bricks serves) and their chunks; counts back to zero
+__global__ void __launch_bounds__(256) k_sensor_place(uint32_t nb, SensorState* __restrict__ st, uint32_t* __restrict__ cnt,
+                                                      uint32_t* __restrict__ cursor, uint4* __restrict__ chunks,
+                                                      uint32_t* __restrict__ split)
+{
+  const uint32_t b = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+  const uint32_t c = b < nb ? cnt[b] : 0u, cc = (c + SB_CHUNK - 1) / SB_CHUNK;
+  uint32_t pc = c, pk = cc;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y0 = __shfl_up(pc, o), y1 = __shfl_up(pk, o);
+    if (lane >= (uint32_t)o) {
+      pc += y0;
+      pk += y1;
+    }
+  }
+  uint32_t base = 0, kbase = 0;
+  if (lane == 63 && pc) {
+    base = atomicAdd(&st->pairs, pc);
+    kbase = atomicAdd(&st->chunks, pk);
+  }
+  base = __shfl(base, 63) + pc - c;
+  kbase = __shfl(kbase, 63) + pk - cc;
+  if (c == 0u) return;
+  cnt[b] = 0u;
+  cursor[b] = base;
+  for (uint32_t k = 0; k < cc; ++k)
+    chunks[kbase + k] = make_uint4(b, base + k * SB_CHUNK, min(SB_CHUNK, c - k * SB_CHUNK), cc > 1 ? 1u : 0u);
+  if (cc > 1) split[atomicAdd(&st->split, 1u)] = b;
+}
+
+// the pairs, sorted by brick: a block takes a stretch per brick, its rays fill it
+__global__ void __launch_bounds__(256) k_sensor_pairs(const SensorGeom g, const SensorState* __restrict__ st,
+                                                      const uint64_t* __restrict__ list, uint32_t* __restrict__ cursor,
+                                                      uint2* __restrict__ pairs)
+{
+  __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
+  const uint32_t m = st->targets, k = blockIdx.x * 256 + threadIdx.x;
+  if (blockIdx.x * 256 >= m) return;  // uniform
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256) {
+    keys[i] = SH_NONE;
+    num[i] = 0u;
+  }
+  __syncthreads();
+  uint32_t t[3];
+  if (k < m) {
+    sensor_target(g, list[k], t);
+    sensor_bricks(g, t, [&](uint32_t b, uint32_t) {
+      const uint32_t h = sensor_slot(keys, b);
+      if (h != SH_NONE) atomicAdd(&num[h], 1u);
+    });
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256)
+    if (num[i]) num[i] = atomicAdd(cursor + keys[i], num[i]);
+  __syncthreads();
+  if (k < m)
+    sensor_bricks(g, t, [&](uint32_t b, uint32_t cell) {
+      // the keys are complete: the same slot as before, or none where there was none
+      uint32_t h = (b * 2654435761u) >> 21, at = SH_NONE;
+      for (int probe = 0; probe < 16 && at == SH_NONE; ++probe) {
+        if (keys[h] == b) at = h;
+        h = (h + 1) % SH_SLOTS;
+      }
+      const uint32_t i = at != SH_NONE ? atomicAdd(&num[at], 1u) : atomicAdd(cursor + b, 1u);
+      pairs[i] = make_uint2(k, cell);
+    });
+}
+
+// F free updates in a row on one voxel = max((unknown ? 0 : v) - 10 F, -127)
+// (updateOccupancy saturates at MIN_PROBABILITY)
+__device__ __forceinline__ uint8_t sensor_free(uint8_t old, uint32_t f)
+{
+  int v = (int)(int8_t)old;
+  if (v == PROB_UNKNOWN) v = 0;
+  return (uint8_t)(int8_t)max(v - 10 * (int)min(f, 64u), PROB_MIN);
+}
+
+__device__ __forceinline__ uint64_t sensor_voxel(const SensorGeom& g, uint32_t brick, uint32_t cell)
+{
+  const uint32_t x = brick % g.bx * SB + cell % SB, y = brick / g.bx % g.by * SB + cell / SB % SB,
+                 z = brick / (g.bx * g.by) * SB + cell / (SB * SB);
+  return ((uint64_t)z * g.dyd.d + y) * g.dxd.d + x;
+}
+
+__global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const SensorState* __restrict__ st,
+                                                      const uint4* __restrict__ chunks, const uint2* __restrict__ pairs,
+                                                      const uint64_t* __restrict__ list,
+                                                      const uint32_t* __restrict__ weight, uint8_t* __restrict__ map,
+                                                      uint32_t* __restrict__ hits)
+{
+  __shared__ uint4 num4[SB_CELLS / 4];
+  uint32_t* num = reinterpret_cast<uint32_t*>(num4);
+  const uint32_t nc = st->chunks;
+  for (uint32_t c = blockIdx.x; c < nc; c += gridDim.x) {  // uniform over the block
+    const uint4 ch = chunks[c];
+    for (uint32_t i = threadIdx.x; i < SB_CELLS / 4; i += 256) num4[i] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    const uint32_t o[3] = {ch.x % g.bx * SB, ch.x / g.bx % g.by * SB, ch.x / (g.bx * g.by) * SB};
+    for (uint32_t i = threadIdx.x; i < ch.z; i += 256) {
+      const uint2 pr = pairs[ch.y + i];
+      const uint32_t wgt = weight[pr.x];
+      uint32_t t[3];
+      sensor_target(g, list[pr.x], t);
+      uint32_t cell = pr.y;
+      const uint32_t l[3] = {cell % SB, cell / SB % SB, cell / (SB * SB)};
+      uint32_t d[3], k[3], room[3];  // steps per axis, taken so far, left before the brick's face
+      bool up[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        up[a] = t[a] > g.s[a];
+        d[a] = up[a] ? t[a] - g.s[a] : g.s[a] - t[a];
+        const uint32_t at = o[a] + l[a];
+        k[a] = up[a] ? at - g.s[a] : g.s[a] - at;
+        room[a] = up[a] ? SB - 1 - l[a] : l[a];
+      }
+      // the walk's errors at this cell (exact modulo 2^32, and small)
+      int32_t exy = (int32_t)(d[0] - d[1] - 2 * k[0] * d[1] + 2 * k[1] * d[0]);
+      int32_t exz = (int32_t)(d[0] - d[2] - 2 * k[0] * d[2] + 2 * k[2] * d[0]);
+      int32_t eyz = (int32_t)(d[1] - d[2] - 2 * k[1] * d[2] + 2 * k[2] * d[1]);
+      const int32_t d0 = (int32_t)(2 * d[0]), d1 = (int32_t)(2 * d[1]), d2 = (int32_t)(2 * d[2]);
+      uint32_t left = d[0] - k[0] + d[1] - k[1] + d[2] - k[2];
+      const uint32_t sx = up[0] ? 1u : 0u - 1u, sy = up[1] ? SB : 0u - SB, sz = up[2] ? SB * SB : 0u - SB * SB;
+      for (;;) {
+        atomicAdd(&num[cell], wgt);
+        if (left-- == 0u) break;
+        if (exy > 0 && exz > 0) {
+          if (room[0]-- == 0u) break;
+          cell += sx;
+          exy -= d1;
+          exz -= d2;
+        } else if (eyz > 0) {
+          if (room[1]-- == 0u) break;
+          cell += sy;
+          exy += d0;
+          eyz -= d2;
+        } else {
+          if (room[2]-- == 0u) break;
+          cell += sz;
+          exz += d0;
+          eyz += d1;
+        }
+      }
+    }
+    __syncthreads();
+    // 16 neighbouring lanes are 16 neighbouring voxels; bytes, since a word may belong to
+    // two bricks
+    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += 256) {
+      const uint32_t f = num[i];
+      if (!f) continue;
+      const uint64_t v = sensor_voxel(g, ch.x, i);
+      if (ch.w) atomicAdd(hits + v, f);
+      else map[v] = sensor_free(map[v], f);
+    }
+    __syncthreads();
+  }
+}
+
+// bricks whose pairs were cut into several chunks
+__global__ void __launch_bounds__(256) k_sensor_split(const SensorGeom g, const SensorState* __restrict__ st,
+                                                      const uint32_t* __restrict__ split, uint32_t dz,
+                                                      uint8_t* __restrict__ map, uint32_t* __restrict__ hits)
+{
+  const uint32_t n = st->split;
+  for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
+    const uint32_t brick = split[b];
+    const uint32_t x0 = brick % g.bx * SB, y0 = brick / g.bx % g.by * SB, z0 = brick / (g.bx * g.by) * SB;
+    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += 256) {
+      if (x0 + i % SB >= g.dxd.d || y0 + i / SB % SB >= g.dyd.d || z0 + i / (SB * SB) >= dz) continue;
+      const uint64_t v = sensor_voxel(g, brick, i);
+      const uint32_t f = hits[v];
+      if (!f) continue;
+      hits[v] = 0u;
+      map[v] = sensor_free(map[v], f);
+    }
+  }
+}
+
+// pass 1 without bricks, for maps with an edge above SB_EDGE and for scans whose pairs
+// would pass SB_PAIR_BYTES: one lane per distinct target voxel walks the line from the
+// sensor voxel to the target and adds the target's weight to the 32-bit counter of every cell it visits
 // (atomics without a return value: the walk never waits).  Rays of neighbouring
 // targets (consecutive lanes) share many cells, so at every step each run of
 // consecutive lanes on one cell adds its summed weight once (a 640 x 480 depth
@@ -617,11 +947,11 @@ __global__ void __launch_bounds__(256) k_sensor_rays(uint32_t* __restrict__ hits
                                                      uint32_t sx, uint32_t sy, uint32_t sz,
                                                      const uint64_t* __restrict__ list,
                                                      const uint32_t* __restrict__ weight,
-                                                     const uint32_t* __restrict__ count)
+                                                     const SensorState* __restrict__ st)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t m = *count;
+  const uint64_t m = st->targets;
   const uint64_t rounds = (m + stride - 1) / stride;  // uniform trip count: every lane reaches the ballots
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t plane = (uint64_t)dx * dy;
@@ -676,9 +1006,8 @@ __global__ void __launch_bounds__(256) k_sensor_rays(uint32_t* __restrict__ hits
   }
 }
 
-// pass 1b: F free updates in a row on one voxel = max((unknown ? 0 : v) - 10 F,
-// -127) (updateOccupancy saturates at MIN_PROBABILITY); the counters go back to
-// zero for the next scan.  Four voxels per thread.
+// pass 1b of that: the counters applied to the voxels and back to zero for the next scan.
+// Four voxels per thread.
 __global__ void __launch_bounds__(256) k_sensor_apply(uint8_t* __restrict__ map, uint32_t* __restrict__ hits, uint64_t n)
 {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -692,10 +1021,7 @@ __global__ void __launch_bounds__(256) k_sensor_apply(uint8_t* __restrict__ map,
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         if (!hc[k]) continue;
-        int v = (int)(int8_t)((w >> (8 * k)) & 0xFFu);
-        if (v == PROB_UNKNOWN) v = 0;
-        v = max(v - 10 * (int)min(hc[k], 64u), PROB_MIN);
-        w = (w & ~(0xFFu << (8 * k))) | ((uint32_t)(uint8_t)(int8_t)v << (8 * k));
+        w = (w & ~(0xFFu << (8 * k))) | ((uint32_t)sensor_free((uint8_t)(w >> (8 * k)), hc[k]) << (8 * k));
       }
       reinterpret_cast<uint32_t*>(map)[q] = w;
       reinterpret_cast<uint4*>(hits)[q] = make_uint4(0u, 0u, 0u, 0u);
@@ -703,9 +1029,7 @@ __global__ void __launch_bounds__(256) k_sensor_apply(uint8_t* __restrict__ map,
       for (uint64_t i = i0; i < n; ++i) {
         const uint32_t c = hits[i];
         if (!c) continue;
-        int v = (int)(int8_t)map[i];
-        if (v == PROB_UNKNOWN) v = 0;
-        map[i] = (uint8_t)(int8_t)max(v - 10 * (int)min(c, 64u), PROB_MIN);
+        map[i] = sensor_free(map[i], c);
         hits[i] = 0u;
       }
     }
@@ -715,9 +1039,9 @@ __global__ void __launch_bounds__(256) k_sensor_apply(uint8_t* __restrict__ map,
 // pass 2: the measured voxels, each with its point count
 __global__ void __launch_bounds__(256) k_sensor_hits(uint8_t* __restrict__ map, const uint64_t* __restrict__ list,
                                                      const uint32_t* __restrict__ weight,
-                                                     const uint32_t* __restrict__ count)
+                                                     const SensorState* __restrict__ st)
 {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x, m = *count;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x, m = st->targets;
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < m; k += stride)
     prob_add_n(map, list[k], SENSOR_OCC, weight[k]);
 }
@@ -772,8 +1096,8 @@ __global__ void __launch_bounds__(256) k_shift_sv(uint8_t* __restrict__ v, uint6
   }
 }
 
-// per-voxel ray counters of insertSensorData: allocated zeroed once per size and
-// left zeroed by every scan (k_sensor_apply clears what it consumed)
+// per-voxel words of insertSensorData (tags, then ray counters): allocated zeroed once
+// per size and left zeroed by every scan
 static int sensor_hits_buffer(uint64_t n, uint32_t** out)
 {
   static uint32_t* buf = nullptr;
@@ -791,9 +1115,14 @@ static int sensor_hits_buffer(uint64_t n, uint32_t** out)
   return GVX_OK;
 }
 
-// per-point arrays of insertSensorData (grown on demand, kept): representative flags
-// and their scan (n + 1 words), weights (n words), target voxels (n u64)
-static int sensor_scratch(uint64_t n, uint32_t** rep, uint32_t** pos, uint32_t** weight, uint64_t** list)
+// arrays of one scan (grown on demand, kept): representative slots and weights (n words
+// each), target voxels (n u64)
+struct SensorPoints {
+  SensorState* st = nullptr;
+  uint32_t *pos = nullptr, *weight = nullptr;
+  uint64_t* list = nullptr;
+};
+static int sensor_points(uint64_t n, SensorPoints* out)
 {
   static uint8_t* buf = nullptr;
   static uint64_t cap = 0;
@@ -803,13 +1132,45 @@ static int sensor_scratch(uint64_t n, uint32_t** rep, uint32_t** pos, uint32_t**
     dfree(buf);
     buf = nullptr;
     cap = 0;
-    GVX_CHECK(dalloc((void**)&buf, al(4 * n) + al(4 * (n + 1)) + al(4 * n) + al(8 * n)));
+    GVX_CHECK(dalloc((void**)&buf, 256 + al(4 * n) + al(4 * n) + al(8 * n)));
     cap = n;
   }
-  *rep = (uint32_t*)buf;
-  *pos = (uint32_t*)(buf + al(4 * cap));
-  *weight = (uint32_t*)(buf + al(4 * cap) + al(4 * (cap + 1)));
-  *list = (uint64_t*)(buf + al(4 * cap) + al(4 * (cap + 1)) + al(4 * cap));
+  out->st = (SensorState*)buf;
+  out->pos = (uint32_t*)(buf + 256);
+  out->weight = (uint32_t*)(buf + 256 + al(4 * cap));
+  out->list = (uint64_t*)(buf + 256 + 2 * al(4 * cap));
+  return GVX_OK;
+}
+
+// bricks and pairs of one scan: n rays enter at most nb_edges bricks each (the sum of the
+// brick counts along the axes); counts are zero between scans
+constexpr uint64_t SB_PAIR_BYTES = 2ull << 30;
+struct SensorBricks {
+  uint32_t *cnt = nullptr, *cursor = nullptr, *split = nullptr;
+  uint4* chunks = nullptr;
+  uint2* pairs = nullptr;
+};
+static int sensor_bricks_buffers(uint64_t nb, uint64_t pairs, SensorBricks* out)
+{
+  static SensorBricks b;
+  static uint64_t cap_b = 0, cap_p = 0;
+  if (cap_b < nb || cap_p < pairs) {
+    GVX_CHECK(sync());
+    dfree(b.cnt); dfree(b.cursor); dfree(b.split); dfree(b.chunks); dfree(b.pairs);
+    b = SensorBricks();
+    nb = std::max(nb, cap_b);
+    pairs = std::max(pairs, cap_p);
+    cap_b = cap_p = 0;
+    GVX_CHECK(dalloc((void**)&b.cnt, nb * 4));
+    GVX_CHECK(dalloc((void**)&b.cursor, nb * 4));
+    GVX_CHECK(dalloc((void**)&b.split, nb * 4));
+    GVX_CHECK(dalloc((void**)&b.chunks, (nb + pairs / SB_CHUNK + 1) * 16));
+    GVX_CHECK(dalloc((void**)&b.pairs, pairs * 8));
+    GVX_CHECK(fill_u32(b.cnt, 0u, nb));
+    cap_b = nb;
+    cap_p = pairs;
+  }
+  *out = b;
   return GVX_OK;
 }
 
@@ -1053,32 +1414,45 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
   if (n >= 0xFFFFFFFFull) return fail(GVX_ERR_UNSUPPORTED, "insertSensorData: more than 2^32 - 2 points");
   uint32_t* hits = nullptr;
   GVX_CHECK(sensor_hits_buffer(m->n, &hits));
-  uint32_t *rep = nullptr, *pos = nullptr, *weight = nullptr;
-  uint64_t* list = nullptr;
-  GVX_CHECK(sensor_scratch(n, &rep, &pos, &weight, &list));
-  const uint32_t* count = pos + n;
+  SensorPoints P;
+  GVX_CHECK(sensor_points(n, &P));
+  const uint32_t dx = m->dims[0], dy = m->dims[1], dz = m->dims[2];
+  const uint32_t bx = (dx + SB - 1) / SB, by = (dy + SB - 1) / SB, bz = (dz + SB - 1) / SB;
+  const uint64_t nb = (uint64_t)bx * by * bz, pairs = n * (uint64_t)(bx + by + bz);
+  const bool bricks = std::max(dx, std::max(dy, dz)) <= SB_EDGE && pairs * 8 <= SB_PAIR_BYTES;
+  SensorBricks B;
+  if (enable_raycasting && bricks) GVX_CHECK(sensor_bricks_buffers(nb, pairs, &B));
+  const SensorGeom geom = {{sx, sy, sz}, udiv(dx), udiv(dy), bx, by};
   const unsigned gp = grid_for(n, 256, 1u << 14);
   {
     // distinct target voxels (in image order) and their point counts
     ProfScope ps("sensor_targets");
     const float* pts = (const float*)d;
-    hipLaunchKernelGGL(k_sensor_tag, dim3(gp), dim3(256), 0, s, hits, m->dims[0], m->dims[1], m->dims[2], side, sin,
-                       pts, n, robot, robot_meaning);
-    hipLaunchKernelGGL(k_sensor_rep, dim3(gp), dim3(256), 0, s, hits, m->dims[0], m->dims[1], m->dims[2], side, sin,
-                       pts, n, robot, robot_meaning, rep);
-    GVX_HIP(hipGetLastError());
-    GVX_CHECK(scan_u32(rep, pos, n, pos + n));
-    GVX_CHECK(fill_u32(weight, 0u, n));
-    hipLaunchKernelGGL(k_sensor_weigh, dim3(gp), dim3(256), 0, s, hits, m->dims[0], m->dims[1], m->dims[2], side,
-                       sin, pts, n, robot, robot_meaning, pos, list, weight);
-    hipLaunchKernelGGL(k_sensor_untag, dim3(gp), dim3(256), 0, s, hits, list, count);
+    hipLaunchKernelGGL(k_sensor_tag, dim3(gp), dim3(256), 0, s, hits, dx, dy, dz, side, sin, pts, n, robot, robot_meaning,
+                       P.st);
+    hipLaunchKernelGGL(k_sensor_rep, dim3(grid_for(n, REP_BLOCK, 1u << 14)), dim3(REP_BLOCK), 0, s, hits, dx, dy, dz,
+                       side, sin, pts, n, robot, robot_meaning, P.st, P.pos, P.list, P.weight);
+    hipLaunchKernelGGL(k_sensor_weigh, dim3(gp), dim3(256), 0, s, hits, dx, dy, dz, side, sin, pts, n, robot,
+                       robot_meaning, P.pos, P.weight);
+    if (!(enable_raycasting && bricks)) hipLaunchKernelGGL(k_sensor_untag, dim3(gp), dim3(256), 0, s, hits, P.list, P.st);
     GVX_HIP(hipGetLastError());
   }
-  if (enable_raycasting) {
+  if (enable_raycasting && bricks) {
+    ProfScope ps("sensor_rays");
+    const unsigned gr = (unsigned)((n + 255) / 256);
+    hipLaunchKernelGGL(k_sensor_count, dim3(gr), dim3(256), 0, s, geom, P.st, P.list, hits, B.cnt);
+    hipLaunchKernelGGL(k_sensor_place, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, (uint32_t)nb, P.st, B.cnt,
+                       B.cursor, B.chunks, B.split);
+    hipLaunchKernelGGL(k_sensor_pairs, dim3(gr), dim3(256), 0, s, geom, P.st, P.list, B.cursor, B.pairs);
+    const unsigned gc = (unsigned)(rt().num_cus > 0 ? rt().num_cus : 256) * 8;
+    hipLaunchKernelGGL(k_sensor_cells, dim3(gc), dim3(256), 0, s, geom, P.st, B.chunks, B.pairs, P.list, P.weight,
+                       (uint8_t*)m->data, hits);
+    hipLaunchKernelGGL(k_sensor_split, dim3(256), dim3(256), 0, s, geom, P.st, B.split, dz, (uint8_t*)m->data, hits);
+    GVX_HIP(hipGetLastError());
+  } else if (enable_raycasting) {
     {
       ProfScope ps("sensor_rays");
-      hipLaunchKernelGGL(k_sensor_rays, dim3(gp), dim3(256), 0, s, hits, m->dims[0], m->dims[1], m->dims[2], sx, sy,
-                         sz, list, weight, count);
+      hipLaunchKernelGGL(k_sensor_rays, dim3(gp), dim3(256), 0, s, hits, dx, dy, dz, sx, sy, sz, P.list, P.weight, P.st);
       GVX_HIP(hipGetLastError());
     }
     {
@@ -1090,8 +1464,8 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
   }
   {
     ProfScope ps("sensor_hits");
-    hipLaunchKernelGGL(k_sensor_hits, dim3(grid_for(n, 256, 1u << 16)), dim3(256), 0, s, (uint8_t*)m->data, list,
-                       weight, count);
+    hipLaunchKernelGGL(k_sensor_hits, dim3(grid_for(n, 256, 1u << 16)), dim3(256), 0, s, (uint8_t*)m->data, P.list,
+                       P.weight, P.st);
     GVX_HIP(hipGetLastError());
   }
   return sync();

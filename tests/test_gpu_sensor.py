@@ -94,3 +94,22 @@ def test_sensor_depth_image_512(gvx_lib):
     got = g.read()
     assert np.array_equal(got, o), f"{int((got != o).sum())} voxels differ"
     assert int((o == 127).sum()) > 1000 and int((o == -127).sum()) > 100000
+
+
+@pytest.mark.parametrize("dims", [(16, 16, 16), (17, 15, 33), (200, 180, 160), (1, 1, 300), (40000, 6, 5)])
+@pytest.mark.parametrize("n", [1, 300, 30000])
+def test_sensor_bricks(gvx_lib, dims, n):
+    """Whole and partial bricks, one to many rays per brick (several chunks near the sensor), a sensor
+    at the map's corner and inside, and an edge too long for bricks."""
+    gvx = gvx_lib
+    side = 0.05
+    rng = np.random.default_rng(sum(dims) + n)
+    for at in (0.0, 0.37, 0.999):
+        sensor = (np.array(dims) * side * at).astype(np.float32)
+        g = gvx.Map(gvx.PROBAB_VOXELMAP, dims, side)
+        o = O.new_map(O.PROB_MAP, dims)
+        for _ in range(2):
+            pts = _scan(rng, max(n, 64), dims, side, sensor)[-n:]
+            g.insert_sensor_data(pts, sensor)
+            O.prob_insert_sensor(o, dims, side, sensor, pts)
+            assert np.array_equal(g.read(), o)
