@@ -647,11 +647,12 @@ __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hit
 // device-scope atomics for a 640 x 480 depth image in a 512^3 map (0.6-1.1 ms), which bound
 // the scan.  So the cells are counted where they lie: the map is cut into bricks of 16^3
 // voxels; each ray is cut into its stretches inside bricks ((ray, entry cell) pairs, about
-// one per 16 cells, found without walking: SENSORTIMES), the pairs are sorted by brick, and
+// one per 16 cells, found without walking), the pairs are sorted by brick, and
 // a block walks a brick's pairs with the 4096 counters in LDS and updates the brick's
 // voxels itself.  Bricks near the sensor hold most rays: their pairs are cut into chunks of
 // SB_CHUNK, whose counters meet in memory (hits, zero at rest) before the voxels are
-// updated.
+// updated.  That frame: count 27, place 7, pairs 60, cells 72, split 6 us; all of them
+// half bound by instruction issue, half by latency.
 //
 // The line steps along x when tx < ty and tx < tz, else along y when ty < tz, else along z,
 // where the i-th step of an axis of length d has the time t = (2i + 1) / (2d): the errors of
@@ -661,8 +662,9 @@ __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hit
 // than it) have closed forms.
 constexpr uint32_t SB = 16, SB_CELLS = SB * SB * SB;
 constexpr uint32_t SB_CHUNK = 2048;      // pairs per block at a time
-constexpr uint32_t SB_EDGE = 32767;      // longest map edge: products of two step numbers fit 32 bits
-constexpr uint32_t SH_SLOTS = 2048;      // bricks a block of 256 rays counts in LDS
+constexpr uint32_t SB_EDGE = 4095;       // longest map edge: keeps products of step numbers and times in 32 bits
+constexpr uint32_t SR_RAYS = 128, SR_THREADS = 512;  // rays and threads of a block that cuts rays
+constexpr uint32_t SH_SLOTS = 2048;      // bricks that such a block counts in LDS
 constexpr uint32_t SH_NONE = 0xFFFFFFFFu;
 
 struct SensorGeom {
@@ -676,39 +678,132 @@ __device__ __forceinline__ void sensor_target(const SensorGeom& g, uint64_t v, u
   t[2] = g.dyd.div(g.dxd.div((uint32_t)v, t[0]), t[1]);  // a map has at most 2^32 voxels
 }
 
-// emit(brick, cell inside it) for every brick that the ray from the sensor to t enters
-template <typename Emit>
-__device__ __forceinline__ void sensor_bricks(const SensorGeom& g, const uint32_t (&t)[3], Emit&& emit)
+// floor(n / d) for n < 2^26 and quotients below 2^13 (edges up to SB_EDGE): the float
+// quotient is within 1 of it (relative errors of 2^-24 and 2^-22), one step corrects it
+__device__ __forceinline__ uint32_t sensor_div(uint32_t n, uint32_t d, float rcp)
 {
-  uint32_t d[3], e[3], c[3];  // steps per axis, index of the step into the next brick, current cell
+  const uint32_t q = (uint32_t)((float)n * rcp);
+  const int32_t r = (int32_t)(n - q * d);
+  return r < 0 ? q - 1 : (uint32_t)r >= d ? q + 1 : q;
+}
+
+// a ray's steps per axis, and the step that leaves the sensor's brick along each
+struct SensorRay {
+  uint32_t d[3], e[3];
   bool up[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    up[a] = t[a] > g.s[a];
-    d[a] = up[a] ? t[a] - g.s[a] : g.s[a] - t[a];
-    e[a] = up[a] ? SB - 1 - g.s[a] % SB : g.s[a] % SB;
-    c[a] = g.s[a];
-  }
-  for (;;) {
-    emit(((c[2] / SB) * g.by + c[1] / SB) * g.bx + c[0] / SB, ((c[2] % SB) * SB + c[1] % SB) * SB + c[0] % SB);
-    const bool h0 = e[0] < d[0], h1 = e[1] < d[1], h2 = e[2] < d[2];
-    if (!(h0 || h1 || h2)) return;
-    const uint32_t u0 = 2 * e[0] + 1, u1 = 2 * e[1] + 1, u2 = 2 * e[2] + 1;
-    const bool xy = h0 && (!h1 || u0 * d[1] < u1 * d[0]), xz = h0 && (!h2 || u0 * d[2] < u2 * d[0]);
-    const bool yz = h1 && (!h2 || u1 * d[2] < u2 * d[1]);
-    const int ax = xy && xz ? 0 : yz ? 1 : 2;
-    const uint32_t ua = ax == 0 ? u0 : ax == 1 ? u1 : u2, da = ax == 0 ? d[0] : ax == 1 ? d[1] : d[2];
+  __device__ __forceinline__ SensorRay(const SensorGeom& g, const uint32_t (&t)[3])
+  {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      uint32_t k;  // steps of axis a up to and with this one
-      if (a == ax) {
-        k = e[a] + 1;
-        e[a] += SB;
-      } else {  // (2j + 1) / d[a] before ua / da, or with it when a comes first (a > ax)
-        k = d[a] == 0u ? 0u : ((ua * d[a] - (a > ax ? 0u : 1u)) / da + 1) / 2;
-      }
-      c[a] = up[a] ? g.s[a] + k : g.s[a] - k;
+      up[a] = t[a] > g.s[a];
+      d[a] = up[a] ? t[a] - g.s[a] : g.s[a] - t[a];
+      e[a] = up[a] ? SB - 1 - g.s[a] % SB : g.s[a] % SB;
     }
+  }
+  // brick faces crossed along axis a: steps e[a], e[a] + SB, ... below d[a]
+  __device__ __forceinline__ uint32_t faces(int a) const { return e[a] < d[a] ? (d[a] - 1 - e[a]) / SB + 1 : 0u; }
+  // k[] = steps of every axis up to and with axis ax's step i: those with a time (2j + 1) /
+  // d[a] before (2i + 1) / d[ax], or equal to it when a comes first (a > ax)
+  __device__ __forceinline__ void steps(int ax, uint32_t i, uint32_t (&k)[3]) const
+  {
+    const uint32_t ua = 2 * i + 1, da = ax == 0 ? d[0] : ax == 1 ? d[1] : d[2];
+    const float rcp = __builtin_amdgcn_rcpf((float)da);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      k[a] = a == ax ? i + 1 : d[a] == 0u ? 0u : (sensor_div(ua * d[a] - (a > ax ? 0u : 1u), da, rcp) + 1) / 2;
+  }
+  // the ray's f-th entry into a brick in no particular order (0: the sensor's), f below
+  // 1 + the faces of all axes: steps taken by then
+  __device__ __forceinline__ void entry(uint32_t f, uint32_t f0, uint32_t f1, uint32_t (&k)[3]) const
+  {
+    if (f == 0u) {
+      k[0] = k[1] = k[2] = 0u;
+      return;
+    }
+    --f;
+    const int ax = f < f0 ? 0 : f < f0 + f1 ? 1 : 2;
+    const uint32_t q = ax == 0 ? f : ax == 1 ? f - f0 : f - f0 - f1;
+    steps(ax, (ax == 0 ? e[0] : ax == 1 ? e[1] : e[2]) + q * SB, k);
+  }
+  // cells from the one after k[] steps to the last one in its brick (both included): up to
+  // the earliest of the three next faces, or the target
+  __device__ __forceinline__ uint32_t stretch(const uint32_t (&k)[3]) const
+  {
+    uint32_t n[3];  // each axis's next step that crosses a face
+    bool h[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      n[a] = k[a] <= e[a] ? e[a] : e[a] + (k[a] - e[a] + SB - 1) / SB * SB;
+      h[a] = n[a] < d[a];
+    }
+    if (!(h[0] || h[1] || h[2])) return d[0] - k[0] + d[1] - k[1] + d[2] - k[2] + 1;
+    const uint32_t u0 = 2 * n[0] + 1, u1 = 2 * n[1] + 1, u2 = 2 * n[2] + 1;
+    const bool xy = h[0] && (!h[1] || u0 * d[1] < u1 * d[0]), xz = h[0] && (!h[2] || u0 * d[2] < u2 * d[0]);
+    const bool yz = h[1] && (!h[2] || u1 * d[2] < u2 * d[1]);
+    const int ax = xy && xz ? 0 : yz ? 1 : 2;
+    uint32_t m[3];
+    steps(ax, ax == 0 ? n[0] : ax == 1 ? n[1] : n[2], m);
+    return m[0] - k[0] + m[1] - k[1] + m[2] - k[2];
+  }
+  __device__ __forceinline__ void cell(const SensorGeom& g, const uint32_t (&k)[3], uint32_t& brick, uint32_t& at) const
+  {
+    uint32_t c[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c[a] = up[a] ? g.s[a] + k[a] : g.s[a] - k[a];
+    brick = ((c[2] / SB) * g.by + c[1] / SB) * g.bx + c[0] / SB;
+    at = ((c[2] % SB) * SB + c[1] % SB) * SB + c[0] % SB;
+  }
+};
+
+// The entries of a block's rays, one thread each: the rays' targets and the prefix of
+// their entry counts in LDS.  (A thread per ray, face after face, took as long as the
+// longest ray: 43 + 77 us for the two kernels below, against 27 + 60 us.)
+struct SensorCut {
+  uint32_t t[3][SR_RAYS], pre[SR_RAYS + 1];
+};
+__device__ __forceinline__ void sensor_cut(const SensorGeom& g, const uint64_t* __restrict__ list, uint32_t m,
+                                           SensorCut& c)
+{
+  const uint32_t r = threadIdx.x, k = blockIdx.x * SR_RAYS + r;
+  uint32_t n = 0;
+  if (r < SR_RAYS && k < m) {
+    uint32_t t[3];
+    sensor_target(g, list[k], t);
+    const SensorRay ray(g, t);
+    n = 1 + ray.faces(0) + ray.faces(1) + ray.faces(2);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) c.t[a][r] = t[a];
+  }
+  static_assert(SR_RAYS == 128, "two waves");
+  uint32_t incl = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o);
+    if ((threadIdx.x & 63) >= (uint32_t)o) incl += y;
+  }
+  if (r < SR_RAYS) c.pre[r + 1] = incl;
+  if (r == 0) c.pre[0] = 0u;
+  __syncthreads();
+  const uint32_t first = c.pre[64];
+  __syncthreads();
+  if (r >= 64 && r < SR_RAYS) c.pre[r + 1] += first;
+  __syncthreads();
+}
+// f(ray of the block, its SensorRay, steps at the entry) for every entry, all threads
+template <typename F>
+__device__ __forceinline__ void sensor_entries(const SensorGeom& g, const SensorCut& c, F&& f)
+{
+  for (uint32_t i = threadIdx.x; i < c.pre[SR_RAYS]; i += SR_THREADS) {
+    uint32_t lo = 0, hi = SR_RAYS;  // the last ray whose prefix is at most i (rays without entries come last)
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (c.pre[mid] <= i) lo = mid; else hi = mid;
+    }
+    const uint32_t t[3] = {c.t[0][lo], c.t[1][lo], c.t[2][lo]};
+    const SensorRay ray(g, t);
+    uint32_t k[3];
+    ray.entry(i - c.pre[lo], ray.faces(0), ray.faces(1), k);
+    f(lo, ray, k);
   }
 }
 
@@ -728,33 +823,31 @@ __device__ __forceinline__ uint32_t sensor_slot(uint32_t* keys, uint32_t b)
   return SH_NONE;
 }
 
-// pairs per brick: counted per block of 256 rays first (neighbouring rays share bricks).
-// Also clears the targets' tags.
-__global__ void __launch_bounds__(256) k_sensor_count(const SensorGeom g, const SensorState* __restrict__ st,
-                                                      const uint64_t* __restrict__ list, uint32_t* __restrict__ hits,
-                                                      uint32_t* __restrict__ cnt)
+// pairs per brick: counted per block first (neighbouring rays share bricks).  Also clears
+// the targets' tags.
+__global__ void __launch_bounds__(SR_THREADS) k_sensor_count(const SensorGeom g, const SensorState* __restrict__ st,
+                                                             const uint64_t* __restrict__ list,
+                                                             uint32_t* __restrict__ hits, uint32_t* __restrict__ cnt)
 {
   __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
-  const uint32_t m = st->targets, k = blockIdx.x * 256 + threadIdx.x;
-  if (blockIdx.x * 256 >= m) return;  // uniform
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256) {
+  __shared__ SensorCut cut;
+  const uint32_t m = st->targets;
+  if (blockIdx.x * SR_RAYS >= m) return;  // uniform
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS) {
     keys[i] = SH_NONE;
     num[i] = 0u;
   }
+  if (threadIdx.x < SR_RAYS && blockIdx.x * SR_RAYS + threadIdx.x < m) hits[list[blockIdx.x * SR_RAYS + threadIdx.x]] = 0u;
+  sensor_cut(g, list, m, cut);
+  sensor_entries(g, cut, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
+    uint32_t b, at;
+    ray.cell(g, k, b, at);
+    const uint32_t h = sensor_slot(keys, b);
+    if (h != SH_NONE) atomicAdd(&num[h], 1u);
+    else atomicAdd(cnt + b, 1u);
+  });
   __syncthreads();
-  if (k < m) {
-    const uint64_t v = list[k];
-    hits[v] = 0u;
-    uint32_t t[3];
-    sensor_target(g, v, t);
-    sensor_bricks(g, t, [&](uint32_t b, uint32_t) {
-      const uint32_t h = sensor_slot(keys, b);
-      if (h != SH_NONE) atomicAdd(&num[h], 1u);
-      else atomicAdd(cnt + b, 1u);
-    });
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256)
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
     if (num[i]) atomicAdd(cnt + keys[i], num[i]);
 }
 
@@ -789,42 +882,43 @@ __global__ void __launch_bounds__(256) k_sensor_place(uint32_t nb, SensorState* 
   if (cc > 1) split[atomicAdd(&st->split, 1u)] = b;
 }
 
-// the pairs, sorted by brick: a block takes a stretch per brick, its rays fill it
-__global__ void __launch_bounds__(256) k_sensor_pairs(const SensorGeom g, const SensorState* __restrict__ st,
-                                                      const uint64_t* __restrict__ list, uint32_t* __restrict__ cursor,
-                                                      uint2* __restrict__ pairs)
+// the pairs (ray; entry cell and number of cells), sorted by brick: a block takes a stretch
+// per brick, its rays fill it
+__global__ void __launch_bounds__(SR_THREADS) k_sensor_pairs(const SensorGeom g, const SensorState* __restrict__ st,
+                                                             const uint64_t* __restrict__ list,
+                                                             uint32_t* __restrict__ cursor, uint2* __restrict__ pairs)
 {
   __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
-  const uint32_t m = st->targets, k = blockIdx.x * 256 + threadIdx.x;
-  if (blockIdx.x * 256 >= m) return;  // uniform
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256) {
+  __shared__ SensorCut cut;
+  const uint32_t m = st->targets;
+  if (blockIdx.x * SR_RAYS >= m) return;  // uniform
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS) {
     keys[i] = SH_NONE;
     num[i] = 0u;
   }
+  sensor_cut(g, list, m, cut);
+  sensor_entries(g, cut, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
+    uint32_t b, at;
+    ray.cell(g, k, b, at);
+    const uint32_t h = sensor_slot(keys, b);
+    if (h != SH_NONE) atomicAdd(&num[h], 1u);
+  });
   __syncthreads();
-  uint32_t t[3];
-  if (k < m) {
-    sensor_target(g, list[k], t);
-    sensor_bricks(g, t, [&](uint32_t b, uint32_t) {
-      const uint32_t h = sensor_slot(keys, b);
-      if (h != SH_NONE) atomicAdd(&num[h], 1u);
-    });
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += 256)
+  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
     if (num[i]) num[i] = atomicAdd(cursor + keys[i], num[i]);
   __syncthreads();
-  if (k < m)
-    sensor_bricks(g, t, [&](uint32_t b, uint32_t cell) {
-      // the keys are complete: the same slot as before, or none where there was none
-      uint32_t h = (b * 2654435761u) >> 21, at = SH_NONE;
-      for (int probe = 0; probe < 16 && at == SH_NONE; ++probe) {
-        if (keys[h] == b) at = h;
-        h = (h + 1) % SH_SLOTS;
-      }
-      const uint32_t i = at != SH_NONE ? atomicAdd(&num[at], 1u) : atomicAdd(cursor + b, 1u);
-      pairs[i] = make_uint2(k, cell);
-    });
+  sensor_entries(g, cut, [&](uint32_t r, const SensorRay& ray, const uint32_t (&k)[3]) {
+    uint32_t b, at;
+    ray.cell(g, k, b, at);
+    // the keys are complete: the same slot as before, or none where there was none
+    uint32_t h = (b * 2654435761u) >> 21, slot = SH_NONE;
+    for (int probe = 0; probe < 16 && slot == SH_NONE; ++probe) {
+      if (keys[h] == b) slot = h;
+      h = (h + 1) % SH_SLOTS;
+    }
+    const uint32_t i = slot != SH_NONE ? atomicAdd(&num[slot], 1u) : atomicAdd(cursor + b, 1u);
+    pairs[i] = make_uint2(blockIdx.x * SR_RAYS + r, at | ray.stretch(k) << 12);  // at most 46 cells
+  });
 }
 
 // F free updates in a row on one voxel = max((unknown ? 0 : v) - 10 F, -127)
@@ -856,50 +950,46 @@ __global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const 
     const uint4 ch = chunks[c];
     for (uint32_t i = threadIdx.x; i < SB_CELLS / 4; i += 256) num4[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
-    const uint32_t o[3] = {ch.x % g.bx * SB, ch.x / g.bx % g.by * SB, ch.x / (g.bx * g.by) * SB};
+    const uint32_t o[3] = {ch.x % g.bx * SB, ch.x / g.bx % g.by * SB, ch.x / (g.bx * g.by) * SB};  // first voxel
     for (uint32_t i = threadIdx.x; i < ch.z; i += 256) {
       const uint2 pr = pairs[ch.y + i];
       const uint32_t wgt = weight[pr.x];
       uint32_t t[3];
       sensor_target(g, list[pr.x], t);
-      uint32_t cell = pr.y;
+      const SensorRay ray(g, t);
+      uint32_t cell = pr.y % SB_CELLS, len = pr.y / SB_CELLS;
+      // The axes' next times as integers, (2k + 1) d[b] d[c] for steps k taken and the other
+      // axes' lengths (1 for 0), less the earliest so that they and the at most 46
+      // increments 2 d[b] d[c] after it stay below 2^32 (differences are exact modulo 2^32).
+      // An axis without steps never comes.
+      uint32_t k[3], T[3], inc[3];
       const uint32_t l[3] = {cell % SB, cell / SB % SB, cell / (SB * SB)};
-      uint32_t d[3], k[3], room[3];  // steps per axis, taken so far, left before the brick's face
-      bool up[3];
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        up[a] = t[a] > g.s[a];
-        d[a] = up[a] ? t[a] - g.s[a] : g.s[a] - t[a];
-        const uint32_t at = o[a] + l[a];
-        k[a] = up[a] ? at - g.s[a] : g.s[a] - at;
-        room[a] = up[a] ? SB - 1 - l[a] : l[a];
+        const uint32_t at = o[a] + l[a], p = max(ray.d[(a + 1) % 3], 1u) * max(ray.d[(a + 2) % 3], 1u);
+        k[a] = ray.up[a] ? at - g.s[a] : g.s[a] - at;
+        T[a] = (2 * k[a] + 1) * p;
+        inc[a] = 2 * p;
       }
-      // the walk's errors at this cell (exact modulo 2^32, and small)
-      int32_t exy = (int32_t)(d[0] - d[1] - 2 * k[0] * d[1] + 2 * k[1] * d[0]);
-      int32_t exz = (int32_t)(d[0] - d[2] - 2 * k[0] * d[2] + 2 * k[2] * d[0]);
-      int32_t eyz = (int32_t)(d[1] - d[2] - 2 * k[1] * d[2] + 2 * k[2] * d[1]);
-      const int32_t d0 = (int32_t)(2 * d[0]), d1 = (int32_t)(2 * d[1]), d2 = (int32_t)(2 * d[2]);
-      uint32_t left = d[0] - k[0] + d[1] - k[1] + d[2] - k[2];
-      const uint32_t sx = up[0] ? 1u : 0u - 1u, sy = up[1] ? SB : 0u - SB, sz = up[2] ? SB * SB : 0u - SB * SB;
+      uint32_t t0 = 0;
+      bool none = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        if (ray.d[a] != 0u && (none || (int32_t)(T[a] - t0) < 0)) {
+          t0 = T[a];
+          none = false;
+        }
+      uint32_t tx = ray.d[0] ? T[0] - t0 : 0xFFFFFFFFu, ty = ray.d[1] ? T[1] - t0 : 0xFFFFFFFFu,
+               tz = ray.d[2] ? T[2] - t0 : 0xFFFFFFFFu;
+      const uint32_t sx = ray.up[0] ? 1u : 0u - 1u, sy = ray.up[1] ? SB : 0u - SB, sz = ray.up[2] ? SB * SB : 0u - SB * SB;
       for (;;) {
         atomicAdd(&num[cell], wgt);
-        if (left-- == 0u) break;
-        if (exy > 0 && exz > 0) {
-          if (room[0]-- == 0u) break;
-          cell += sx;
-          exy -= d1;
-          exz -= d2;
-        } else if (eyz > 0) {
-          if (room[1]-- == 0u) break;
-          cell += sy;
-          exy += d0;
-          eyz -= d2;
-        } else {
-          if (room[2]-- == 0u) break;
-          cell += sz;
-          exz += d0;
-          eyz += d1;
-        }
+        if (--len == 0u) break;
+        const bool x = tx < ty && tx < tz, y = !x && ty < tz;
+        cell += x ? sx : y ? sy : sz;
+        tx += x ? inc[0] : 0u;
+        ty += y ? inc[1] : 0u;
+        tz += x || y ? 0u : inc[2];
       }
     }
     __syncthreads();
@@ -917,7 +1007,7 @@ __global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const 
 }
 
 // bricks whose pairs were cut into several chunks
-__global__ void __launch_bounds__(256) k_sensor_split(const SensorGeom g, const SensorState* __restrict__ st,
+__global__ void __launch_bounds__(1024) k_sensor_split(const SensorGeom g, const SensorState* __restrict__ st,
                                                       const uint32_t* __restrict__ split, uint32_t dz,
                                                       uint8_t* __restrict__ map, uint32_t* __restrict__ hits)
 {
@@ -925,7 +1015,7 @@ __global__ void __launch_bounds__(256) k_sensor_split(const SensorGeom g, const 
   for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
     const uint32_t brick = split[b];
     const uint32_t x0 = brick % g.bx * SB, y0 = brick / g.bx % g.by * SB, z0 = brick / (g.bx * g.by) * SB;
-    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += 256) {
+    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += 1024) {
       if (x0 + i % SB >= g.dxd.d || y0 + i / SB % SB >= g.dyd.d || z0 + i / (SB * SB) >= dz) continue;
       const uint64_t v = sensor_voxel(g, brick, i);
       const uint32_t f = hits[v];
@@ -1439,15 +1529,15 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
   }
   if (enable_raycasting && bricks) {
     ProfScope ps("sensor_rays");
-    const unsigned gr = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_sensor_count, dim3(gr), dim3(256), 0, s, geom, P.st, P.list, hits, B.cnt);
+    const unsigned gr = (unsigned)((n + SR_RAYS - 1) / SR_RAYS);
+    hipLaunchKernelGGL(k_sensor_count, dim3(gr), dim3(SR_THREADS), 0, s, geom, P.st, P.list, hits, B.cnt);
     hipLaunchKernelGGL(k_sensor_place, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, (uint32_t)nb, P.st, B.cnt,
                        B.cursor, B.chunks, B.split);
-    hipLaunchKernelGGL(k_sensor_pairs, dim3(gr), dim3(256), 0, s, geom, P.st, P.list, B.cursor, B.pairs);
+    hipLaunchKernelGGL(k_sensor_pairs, dim3(gr), dim3(SR_THREADS), 0, s, geom, P.st, P.list, B.cursor, B.pairs);
     const unsigned gc = (unsigned)(rt().num_cus > 0 ? rt().num_cus : 256) * 8;
     hipLaunchKernelGGL(k_sensor_cells, dim3(gc), dim3(256), 0, s, geom, P.st, B.chunks, B.pairs, P.list, P.weight,
                        (uint8_t*)m->data, hits);
-    hipLaunchKernelGGL(k_sensor_split, dim3(256), dim3(256), 0, s, geom, P.st, B.split, dz, (uint8_t*)m->data, hits);
+    hipLaunchKernelGGL(k_sensor_split, dim3(256), dim3(1024), 0, s, geom, P.st, B.split, dz, (uint8_t*)m->data, hits);
     GVX_HIP(hipGetLastError());
   } else if (enable_raycasting) {
     {
