@@ -82,6 +82,7 @@ def lib():
             "gvx_batch_last_stats": [P, P, P, P],
             "gvx_cost_create": [P, P, f32, P, u32, P, P, u32, f32, f32, P], "gvx_cost_destroy": [P],
             "gvx_cost_forward": [P, P, u32, u32, P], "gvx_cost_backward": [P, P, u32, u32, P, P, P],
+            "gvx_cost_forward_grad": [P, P, u32, u32, P, P],
             "gvx_list_info": [P, P, P],
             "gvx_map_insert_sensor": [P, P, u64, P, i32, P, u32, i32],
             "gvx_map_collide_sv": [P, P, f32, u32, u32, P, P], "gvx_map_shift_sv": [P, u32],
@@ -626,6 +627,14 @@ class Cost:
         self._check("out", out, (q.shape[0],))
         check(lib().gvx_cost_forward(self.h, _p(q), q.shape[0], q.shape[1], _p(out)))
         return out
+
+    def forward_grad(self, q, out, dq):
+        """out (T,) as forward writes it and dq (T, W, L) as backward does, in one pass over the grid"""
+        self._check("q", q, (q.shape[0], q.shape[1], self.n_links) if q.dim() == 3 else (-1,))
+        self._check("out", out, (q.shape[0],))
+        self._check("dq", dq, q.shape)
+        check(lib().gvx_cost_forward_grad(self.h, _p(q), q.shape[0], q.shape[1], _p(out), _p(dq)))
+        return out, dq
 
     def backward(self, q, dq, dx=None, upstream=None):
         """dq: (T, W, L); dx (optional): (T, W, L, spheres per link, 3); upstream (optional): (T,)"""

@@ -282,6 +282,11 @@ int gvx_cost_forward(gvx_cost c, const float* q_dev, uint32_t n_traj, uint32_t n
    n_traj x n_wp x n_links x spheres_per_link x 3; upstream: device n_traj (dL/dc) or NULL for ones */
 int gvx_cost_backward(gvx_cost c, const float* q_dev, uint32_t n_traj, uint32_t n_wp,
                       const float* upstream_dev, float* dq_out_dev, float* dx_out_dev);
+/* both in one pass over the grid: cost_out as gvx_cost_forward writes it, dq_out as
+   gvx_cost_backward does for an upstream of ones.  The upstream factor is the last one applied
+   (dq = upstream * dq_out, the same bits as gvx_cost_backward). */
+int gvx_cost_forward_grad(gvx_cost c, const float* q_dev, uint32_t n_traj, uint32_t n_wp, float* cost_out_dev,
+                          float* dq_out_dev);
 
 /* BitVoxelList::shiftLeftSweptVolumeIDs (voxellist/BitVoxelList.hpp:641-664) */
 int gvx_list_shift_sv(gvx_list list, uint32_t shift);

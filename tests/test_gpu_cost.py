@@ -307,3 +307,71 @@ def test_autograd_function(gvx_lib, edt_512):
         cost.backward(q.detach(), torch.empty(32, 32, 7, device="cuda"), torch.empty(32, 32, 7, 3, device="cuda"))
     with pytest.raises(ValueError):
         gvx.Cost(grid[:1000], d, SIDE, c5["dh"], c5["spheres"], c5["eps"], c5["w"], c5["base"])
+
+
+@pytest.mark.parametrize("nl,spl,ntraj,nwp,dims", [
+    (1, 1, 1, 1, (24, 20, 16)),            # one lane
+    (7, 64, 3, 5, (24, 20, 16)),           # a wave per link
+    (3, 65, 2, 3, (24, 20, 16)),           # two rounds of a wave
+    (5, 17, 4, 70, (24, 20, 16)),          # half waves; more waypoints than lanes in a trajectory
+    (9, 32, 4, 3, (24, 20, 16)),
+    (33, 16, 2, 3, (24, 20, 16)),          # quarter waves, the last wave with one link
+    (64, 40, 1, 3, (24, 20, 16)),          # more waves of links than waves in a block
+    (3, 5, 17, 241, (24, 20, 16)),         # 4097 waypoints: 2 in a block, the last block with 1
+    (3, 5, 3, 2731, (24, 20, 16)),         # 8193: 4 in a block
+    (3, 5, 7, 2341, (24, 20, 16)),         # 16387: 8 in a block, the last with 3
+    (7, 64, 2, 3, (1024, 1024, 1152)),     # samples beyond 32-bit byte offsets
+])
+def test_cost_layouts(gvx_lib, nl, spl, ntraj, nwp, dims):
+    """Every layout of links on lanes, of waypoints on blocks and both address widths against the FP64
+    oracle; the one-pass form gives the bits of the two passes.
+
+    The field is a multilinear polynomial (one cell or the next: the same values) and every hinge is
+    active with h >= 1, so float32 centres, good to 4 ulp(12 m) = 4e-6 m, change a sphere's term by
+    about 1e-5 of it at most (|grad d| <= 1.1); sums of up to 2560 terms add 12 roundings."""
+    import torch
+    gvx = gvx_lib
+    rng = np.random.default_rng(nl * 1000 + spl)
+    big = dims[0] > 24
+    side = 0.01 if big else 0.1
+    i, j, k = (torch.arange(n, device="cuda", dtype=torch.float32) for n in dims)
+    if big:  # small values where the arm is: the gradient is a difference of samples
+        i, j, k = i - 512, j - 512, k - 1056
+    plane = 2 * i[None, :] - j[:, None] + (0 if big else 1) * i[None, :] * j[:, None]
+    scale = 2.0 ** -10 if big else 2.0 ** -8
+    grid = ((plane[None] + 3 * k[:, None, None]) * scale).reshape(-1)  # exact in float32
+    dh = np.zeros((nl, 5), np.float32)
+    dh[:, 1:3] = rng.uniform(0.05, 0.2, size=(nl, 2)) / nl
+    dh[:, 3] = rng.choice([-np.pi / 2, 0, np.pi / 2], nl)
+    dh[nl // 2, 4] = nl > 2  # one prismatic joint
+    sph = np.zeros((nl, spl, 4), np.float32)
+    sph[:, :, :3] = rng.uniform(-0.02, 0.02, size=(nl, spl, 3))
+    sph[:, :, 3] = rng.uniform(0.01, 0.05, size=(nl, spl))
+    q = rng.uniform(-1, 1, size=(ntraj, nwp, nl)).astype(np.float32)
+    if nl > 2:
+        q[:, :, nl // 2] *= 0.02
+    pos = np.array([dims[0] * side / 2, dims[1] * side / 2, 10.6 if big else 0.8], np.float32)
+    base = np.array([1, 0, 0, pos[0], 0, 1, 0, pos[1], 0, 0, 1, pos[2]], np.float32)
+    eps, w = 4.0, 0.5
+    cost = gvx.Cost(grid, dims, side, dh, sph, eps, w, base)
+    qd = torch.from_numpy(q).cuda()
+    up = torch.from_numpy(rng.uniform(0.3, 2, ntraj).astype(np.float32)).cuda()
+    out, one = torch.empty(ntraj, device="cuda"), torch.empty(ntraj, device="cuda")
+    dq, dq1, dqu = (torch.empty_like(qd) for _ in range(3))
+    dx = torch.empty((ntraj, nwp, nl, spl, 3), device="cuda")
+    torch.cuda.synchronize()
+    cost.forward(qd, out)
+    cost.backward(qd, dq)
+    cost.backward(qd, dqu, dx, up)
+    cost.forward_grad(qd, one, dq1)
+    assert torch.equal(out, one) and torch.equal(dq, dq1)
+    assert torch.equal(dqu, dq * up[:, None, None])
+    oc, odq, odx = O.cost_d(grid.cpu().numpy(), dims, float(np.float32(side)), dh, base.astype(np.float64), sph,
+                            q.astype(np.float64), eps, w)
+    assert np.allclose(out.cpu().numpy(), oc, rtol=3e-5, atol=0)
+    odx, odq = odx.reshape(dx.shape), odq.reshape(q.shape)
+    size = np.linalg.norm(odx, axis=-1)
+    err = np.linalg.norm(dx.cpu().numpy() / up.cpu().numpy()[:, None, None, None, None] - odx, axis=-1)
+    assert np.all(err <= 3e-5 * size)
+    # a joint's term: |dc/dx| times a lever of at most the arm's reach
+    assert np.all(np.abs(dq.cpu().numpy() - odq) <= 3e-5 * 0.5 * size.sum(axis=(2, 3))[:, :, None])
