@@ -258,3 +258,74 @@ def test_batch_dense_environment(gvx_lib):
             c, m = b.collide(q)
             assert np.array_equal(c, oc), (sched, sl)
             assert np.array_equal(m, om), (sched, sl)
+
+
+@pytest.mark.parametrize("case", ["faces", "remainders", "many_runs", "many_links", "overflow"])
+def test_batch_pose_blocks(gvx_lib, case):
+    """A block per pose against the oracle and against the chunk kernels (schedule 1), host and device
+    buffers, directly and replayed: points on voxel faces (the reciprocal's product does not decide),
+    links of 1 to 4097 points (chunks of 64, runs of 4096), more than 64 runs, a solid environment
+    where a pose has more voxels than its hash table has slots; the chunk kernels run in between, on
+    the hit matrix that such poses borrow."""
+    import torch
+    gvx = gvx_lib
+    rng = np.random.default_rng(61)
+    d, side = (72, 64, 80), 0.01
+    ext = np.array(d, np.float32) * side
+    env_pts = rng.uniform(0, 1, (20000, 3)).astype(np.float32) * ext
+    nl, n = 3, 40
+    dh = np.stack([np.zeros(nl), rng.uniform(0.05, 0.2, nl), rng.uniform(0.05, 0.2, nl),
+                   rng.choice([-np.pi / 2, np.pi / 2], nl), np.zeros(nl)], axis=1).astype(np.float32)
+    q = rng.uniform(-np.pi, np.pi, (n, nl)).astype(np.float32)
+    box = 0.12
+    if case == "faces":  # a lattice of multiples of the side, moved by whole sides along the axes
+        dh = np.zeros((nl, 5), np.float32)
+        dh[:, 4] = 1.0  # prismatic along z
+        q = (rng.integers(-3, 9, (n, nl)) * np.float32(side)).astype(np.float32)
+        pts = (rng.integers(-2, 60, (9000, 3)) * np.float32(side)).astype(np.float32)
+        sizes = np.array([3000, 3000, 3000], np.uint32)
+        base = np.eye(3, 4, dtype=np.float32).ravel()
+    else:
+        if case == "remainders":
+            nl = 8
+            sizes = np.array([1, 63, 64, 65, 4095, 4096, 4097, 0], np.uint32)
+        elif case == "many_runs":
+            sizes = np.array([270000, 100, 5000], np.uint32)
+        elif case == "many_links":
+            nl = 130
+            sizes = rng.integers(1, 90, nl).astype(np.uint32)
+            box = 0.05
+        else:
+            sizes = np.array([20000, 30000, 10000], np.uint32)
+            box = 0.25
+            env_pts = (np.stack(np.meshgrid(*[np.arange(k) for k in d], indexing="ij"), -1).reshape(-1, 3) + 0.5) * side
+            env_pts = env_pts.astype(np.float32)
+        if nl > 3:
+            dh = np.stack([np.zeros(nl), rng.uniform(0, 0.6 / nl, nl), rng.uniform(0, 0.6 / nl, nl),
+                           rng.choice([-np.pi / 2, 0, np.pi / 2], nl), np.zeros(nl)], axis=1).astype(np.float32)
+            q = rng.uniform(-np.pi, np.pi, (n, nl)).astype(np.float32)
+        pts = rng.uniform(-box, box, (int(sizes.sum()), 3)).astype(np.float32)
+        base = np.array([1, 0, 0, 0.3, 0, 1, 0, 0.3, 0, 0, 1, 0.4], np.float32)
+    oenv = O.new_map(O.BITVECTOR_MAP, d)
+    O.map_insert_points(O.BITVECTOR_MAP, oenv, d, side, env_pts, 1)
+    env = gvx.Map(O.BITVECTOR_MAP, d, side)
+    env.write(oenv)
+    b = gvx.Batch(env, pts, sizes, dh, base, max_poses=64)
+    oc, om = O.batch_collide(O.occupancy_bits(oenv), d, side, pts, sizes, dh, base, q)
+    assert (oc > 0).sum() > n // 2 and (case != "overflow" or (oc > 8000).sum() > 3)
+    qd = torch.from_numpy(q).cuda()
+    cd = torch.empty(n, dtype=torch.int32, device="cuda")
+    md = torch.empty((n, 32), dtype=torch.uint8, device="cuda")
+    for s in (7, 6, 1, 15, 6, 0, 1, 14, 7):
+        b.set_schedule(s)
+        c, m = b.collide(q)
+        assert np.array_equal(c, oc) and np.array_equal(m, om), s
+        cd.fill_(9)
+        md.fill_(9)
+        torch.cuda.synchronize()
+        b.collide(qd, cd, md)
+        assert np.array_equal(cd.cpu().numpy().astype(np.uint32), oc) and np.array_equal(md.cpu().numpy(), om), s
+    b.collide(q)
+    assert 0 <= b.autotune(n) < 16
+    c, m = b.collide(q[:7])
+    assert np.array_equal(c, oc[:7]) and np.array_equal(m, om[:7])
