@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256) k_pba_z_long(const uint32_t* __restrict__
 // at position p exactly when p * D <= N with N = (pb^2 - pa^2) + cb - ca and
 // D = 2 (pb - pa) > 0.  Positions are < 1024 and costs < 2^21, so N < 2^23 and
 // p * D < 2^21 fit int32; phase 2's comparison N_ab * D_bc >= N_bc * D_ab (pop b,
-// also on equality) has products < 2^35, exact in double precision.
+// also on equality) has products < 2^34 (middle_empty).
 #ifndef GVX_PBA_TYR
 #define GVX_PBA_TYR 32
 #endif
@@ -223,20 +223,26 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t slice_rsrc(const void* base, u
                                            __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
 }
 
-// bisector of sites a < b: a is at least as close as b at p  <=>  p * D <= N
+// bisector of sites a < b: a is at least as close as b at p  <=>  2 p D <= N.  Whole numbers
+// below 2^24 in floats, each step exact.
 struct Bis {
-  int32_t N, D;
-  __device__ __forceinline__ void set(int32_t pa, int32_t ca, int32_t pb, int32_t cb)
+  float N, D;
+  __device__ __forceinline__ void set(float pa, float ca, float pb, float cb)
   {
-    D = 2 * (pb - pa);
-    N = __mul24(pb - pa, pb + pa) + (cb - ca);
+    D = pb - pa;
+    N = fmaf(D, pb + pa, cb - ca);
   }
-  __device__ __forceinline__ bool a_wins(int32_t p) const { return __mul24(p, D) <= N; }
+  __device__ __forceinline__ bool a_wins(float p) const { return 2.0f * p * D <= N; }
 };
-// b (the middle of a < b < c) owns no position: bisector(a, b) >= bisector(b, c)
+// b (the middle of a < b < c) owns no position: bisector(a, b) >= bisector(b, c), N_ab D_bc >=
+// N_bc D_ab.  With p the rounded right side, its error is a whole number below 2^9 and a
+// float, and the left side less p is a whole number that rounds only above 2^24: the two
+// compare as the products do.  (In double precision the stack kernels of a 512^3 room took
+// 313 and 112 us, this way 309 and 106: the chain of a line and its LDS round trips are longer.)
 __device__ __forceinline__ bool middle_empty(const Bis& ab, const Bis& bc)
 {
-  return (double)ab.N * (double)bc.D >= (double)bc.N * (double)ab.D;
+  const float p = bc.N * ab.D;
+  return fmaf(ab.N, bc.D, -p) >= fmaf(bc.N, ab.D, -p);
 }
 
 // Per-lane stack of 32-bit entries: ring[depth % RK][lane] holds depths [lo, n);
@@ -317,21 +323,22 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
   if (x >= dx) return;
   const int32_t zi = (int32_t)z;
   LineStack st{ring, stk + ((uint64_t)z * dx + x) * dy, lane, 0, 0};
-  // top (ty, tz, tc), second (sy, sz, sc) and third (entry e3) of the stack;
+  // top, second and third of the stack (entries; positions and costs of the first two);
   // bst = bisector(second, top)
-  int32_t ty = 0, tz = 0, tc = 0, sy = 0, sz = 0, sc = 0;
-  uint32_t e3 = 0;
-  Bis bst{0, 1};
+  float ty = 0.f, tc = 0.f, sy = 0.f, sc = 0.f;
+  uint32_t te = 0, se = 0, e3 = 0;
+  Bis bst{0.f, 1.f};
+  auto cost = [&](int32_t s) -> float { const float d = (float)(s - zi); return d * d; };
   // pop the top: second and third move up, the new third is fetched (when fewer
   // than two entries remain the moved values are never read)
   auto pop_y = [&]() {
     st.pop();
     ty = sy;
-    tz = sz;
     tc = sc;
-    sy = (int32_t)(e3 & 0x3FFu);
-    sz = (int32_t)(e3 >> 10);
-    sc = sq24(sz - zi);
+    te = se;
+    se = e3;
+    sy = (float)(e3 & 0x3FFu);
+    sc = cost((int32_t)(e3 >> 10));
     bst.set(sy, sc, ty, tc);
     e3 = st.at3(st.n >= 3 ? st.n - 3 : 0);
   };
@@ -377,7 +384,7 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
       m &= m - 1u;
       const uint32_t rn = m ? (uint32_t)__builtin_ctz(m) : r;
       const int32_t sn = ztile[rn][lane];
-      const int32_t y = (int32_t)(y0 + r), c = sq24(s - zi);
+      const float y = (float)(y0 + r), c = cost(s);
       if (st.n >= 1) {
         Bis btn;
         btn.set(ty, tc, y, c);
@@ -387,13 +394,13 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
         }
         bst = btn;
       }
-      st.push((uint32_t)y | ((uint32_t)s << 10));
-      e3 = (uint32_t)sy | ((uint32_t)sz << 10);
+      e3 = se;
+      se = te;
+      te = (y0 + r) | ((uint32_t)s << 10);
+      st.push(te);
       sy = ty;
-      sz = tz;
       sc = tc;
       ty = y;
-      tz = s;
       tc = c;
       r = rn;
       s = sn;
@@ -419,10 +426,10 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
     return;
   }
   for (int32_t yy = (int32_t)dy - 1; yy >= 0; --yy) {
-    while (st.n >= 2 && bst.a_wins(yy)) {
+    while (st.n >= 2 && bst.a_wins((float)yy)) {
       pop_y();
     }
-    __builtin_amdgcn_raw_buffer_store_b32(x | ((uint32_t)ty << 10) | ((uint32_t)tz << 20), orr, (int)(x * 4),
+    __builtin_amdgcn_raw_buffer_store_b32(x | te << 10, orr, (int)(x * 4),
                                           (int)((uint32_t)yy * dx * 4), 0);
   }
 }
@@ -962,14 +969,16 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
   const uint32_t lane = threadIdx.x, y = y0 + lane;
   const bool active = y < dy;
   const int32_t yi = (int32_t)y, zi = (int32_t)z;
-  auto cost = [&](uint32_t yz) -> int32_t { return sq24((int32_t)(yz & 0x3FFu) - yi) + sq24((int32_t)(yz >> 10) - zi); };
+  auto cost = [&](uint32_t e) -> float {
+    return (float)(sq24((int32_t)((e >> 10) & 0x3FFu) - yi) + sq24((int32_t)(e >> 20) - zi));
+  };
   // loader mapping: pass k covers rows LPR k + lane / TX, column lane % TX
   const uint32_t lr = lane / TX, lc = lane % TX;
   const uint32_t ntiles = (dx + TX - 1) / TX;
   LineStack st{ring, stk + ((uint64_t)z * dy + (active ? y : 0)) * dx, lane, 0, 0};
-  int32_t tx = 0, tc = 0, sx = 0, sc = 0;
-  uint32_t tyz = 0, syz = 0, e3 = 0;  // top, second, third (entry) of the stack
-  Bis bst{0, 1};
+  float tx = 0.f, tc = 0.f, sx = 0.f, sc = 0.f;
+  uint32_t te = 0, se = 0, e3 = 0;  // top, second, third entry of the stack
+  Bis bst{0.f, 1.f};
   uint32_t pre[NLD];
   const uint32_t* __restrict__ slice = map + (uint64_t)z * dy * dx;
   const uint16_t* __restrict__ rslice = yr + (uint64_t)z * dy * dx;
@@ -1029,9 +1038,7 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
         m &= m - 1u;
         const uint32_t lxn = m ? (uint32_t)__builtin_ctz(m) : lx;
         const uint32_t en = tile[lane][lxn];
-        const int32_t x = (int32_t)(x0 + lx);
-        const uint32_t yz = e >> 10;
-        const int32_t c = cost(yz);
+        const float x = (float)(x0 + lx), c = cost(e);
         if (st.n >= 1) {
           Bis btn;
           btn.set(tx, tc, x, c);
@@ -1039,24 +1046,24 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
             // pop the top: second and third move up, the new third is fetched
             st.pop();
             tx = sx;
-            tyz = syz;
             tc = sc;
-            sx = (int32_t)(e3 & 0x3FFu);
-            syz = e3 >> 10;
-            sc = cost(syz);
+            te = se;
+            se = e3;
+            sx = (float)(e3 & 0x3FFu);
+            sc = cost(e3);
             bst.set(sx, sc, tx, tc);
             e3 = st.at3(st.n >= 3 ? st.n - 3 : 0);
             btn.set(tx, tc, x, c);
           }
           bst = btn;
         }
-        st.push((uint32_t)x | (yz << 10));
-        e3 = (uint32_t)sx | (syz << 10);
+        e3 = se;
+        se = te;
+        te = (x0 + lx) | (e & ~0x3FFu);
+        st.push(te);
         sx = tx;
-        syz = tyz;
         sc = tc;
         tx = x;
-        tyz = yz;
         tc = c;
         lx = lxn;
         e = en;
@@ -1175,9 +1182,8 @@ __global__ void __launch_bounds__(TB * XC_LINES) k_pba_x_colour(uint32_t* __rest
         ent[k] = e;
         if (k >= 1) {
           const uint32_t a = k == lane ? a0 : s[k - 1];
-          Bis b;
-          b.set((int32_t)(a & 0x3FFu), cost(a), (int32_t)(e & 0x3FFu), cost(e));
-          const int32_t st = floor_div(b.N, b.D) + 1;
+          const int32_t pa = (int32_t)(a & 0x3FFu), pb = (int32_t)(e & 0x3FFu);
+          const int32_t st = floor_div(__mul24(pb - pa, pb + pa) + cost(e) - cost(a), 2 * (pb - pa)) + 1;
           if (st < (int32_t)dx) atomicMax(&mark[st > 0 ? st : 0], k);
         }
       }
