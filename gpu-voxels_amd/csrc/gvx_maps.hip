@@ -651,8 +651,10 @@ __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hit
 // a block walks a brick's pairs with the 4096 counters in LDS and updates the brick's
 // voxels itself.  Bricks near the sensor hold most rays: their pairs are cut into chunks of
 // SB_CHUNK, whose counters meet in memory (hits, zero at rest) before the voxels are
-// updated.  That frame: count 27, place 7, pairs 60, cells 72, split 6 us; all of them
-// half bound by instruction issue, half by latency.
+// updated.  That frame: count 24, place 6, pairs 41, cells 49, split 10 us; all of them
+// half bound by instruction issue, half by latency.  Chunks of 1024 pairs, 512 threads
+// each and 16 blocks per CU end more evenly than 2048, 256 and 8: cells 69 + split 6 us
+// then (4096: 94 + 5; 1024 with 1024 threads 56).
 //
 // The line steps along x when tx < ty and tx < tz, else along y when ty < tz, else along z,
 // where the i-th step of an axis of length d has the time t = (2i + 1) / (2d): the errors of
@@ -661,9 +663,9 @@ __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hit
 // earliest of three steps) and the position on the other axes at that moment (steps earlier
 // than it) have closed forms.
 constexpr uint32_t SB = 16, SB_CELLS = SB * SB * SB;
-constexpr uint32_t SB_CHUNK = 2048;      // pairs per block at a time
+constexpr uint32_t SB_CHUNK = 1024, SC_THREADS = 512;  // pairs per block at a time, its threads
 constexpr uint32_t SB_EDGE = 4095;       // longest map edge: keeps products of step numbers and times in 32 bits
-constexpr uint32_t SR_RAYS = 128, SR_THREADS = 512;  // rays and threads of a block that cuts rays
+constexpr uint32_t SR_RAYS = 128, SR_THREADS = 1024;  // rays and threads of a block that cuts rays
 constexpr uint32_t SH_SLOTS = 2048;      // bricks that such a block counts in LDS
 constexpr uint32_t SH_NONE = 0xFFFFFFFFu;
 
@@ -757,7 +759,7 @@ struct SensorRay {
 
 // The entries of a block's rays, one thread each: the rays' targets and the prefix of
 // their entry counts in LDS.  (A thread per ray, face after face, took as long as the
-// longest ray: 43 + 77 us for the two kernels below, against 27 + 60 us.)
+// longest ray: 43 + 77 us for the two kernels below, against 24 + 41 us.)
 struct SensorCut {
   uint32_t t[3][SR_RAYS], pre[SR_RAYS + 1];
 };
@@ -789,22 +791,20 @@ __device__ __forceinline__ void sensor_cut(const SensorGeom& g, const uint64_t* 
   if (r >= 64 && r < SR_RAYS) c.pre[r + 1] += first;
   __syncthreads();
 }
-// f(ray of the block, its SensorRay, steps at the entry) for every entry, all threads
+// entry i of the block: f(ray of the block, its SensorRay, steps at the entry)
 template <typename F>
-__device__ __forceinline__ void sensor_entries(const SensorGeom& g, const SensorCut& c, F&& f)
+__device__ __forceinline__ void sensor_entry(const SensorGeom& g, const SensorCut& c, uint32_t i, F&& f)
 {
-  for (uint32_t i = threadIdx.x; i < c.pre[SR_RAYS]; i += SR_THREADS) {
-    uint32_t lo = 0, hi = SR_RAYS;  // the last ray whose prefix is at most i (rays without entries come last)
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (c.pre[mid] <= i) lo = mid; else hi = mid;
-    }
-    const uint32_t t[3] = {c.t[0][lo], c.t[1][lo], c.t[2][lo]};
-    const SensorRay ray(g, t);
-    uint32_t k[3];
-    ray.entry(i - c.pre[lo], ray.faces(0), ray.faces(1), k);
-    f(lo, ray, k);
+  uint32_t lo = 0, hi = SR_RAYS;  // the last ray whose prefix is at most i (rays without entries come last)
+  while (hi - lo > 1) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (c.pre[mid] <= i) lo = mid; else hi = mid;
   }
+  const uint32_t t[3] = {c.t[0][lo], c.t[1][lo], c.t[2][lo]};
+  const SensorRay ray(g, t);
+  uint32_t k[3];
+  ray.entry(i - c.pre[lo], ray.faces(0), ray.faces(1), k);
+  f(lo, ray, k);
 }
 
 // a block's bricks with their pairs: slot of brick b, or SH_NONE when the table is full
@@ -839,24 +839,28 @@ __global__ void __launch_bounds__(SR_THREADS) k_sensor_count(const SensorGeom g,
   }
   if (threadIdx.x < SR_RAYS && blockIdx.x * SR_RAYS + threadIdx.x < m) hits[list[blockIdx.x * SR_RAYS + threadIdx.x]] = 0u;
   sensor_cut(g, list, m, cut);
-  sensor_entries(g, cut, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
-    uint32_t b, at;
-    ray.cell(g, k, b, at);
-    const uint32_t h = sensor_slot(keys, b);
-    if (h != SH_NONE) atomicAdd(&num[h], 1u);
-    else atomicAdd(cnt + b, 1u);
-  });
+  for (uint32_t i = threadIdx.x; i < cut.pre[SR_RAYS]; i += SR_THREADS)
+    sensor_entry(g, cut, i, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
+      uint32_t b, at;
+      ray.cell(g, k, b, at);
+      const uint32_t h = sensor_slot(keys, b);
+      if (h != SH_NONE) atomicAdd(&num[h], 1u);
+      else atomicAdd(cnt + b, 1u);
+    });
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
     if (num[i]) atomicAdd(cnt + keys[i], num[i]);
 }
 
-// places of the bricks' pairs (any order of bricks serves) and their chunks; counts back to zero
-__global__ void __launch_bounds__(256) k_sensor_place(uint32_t nb, SensorState* __restrict__ st, uint32_t* __restrict__ cnt,
-                                                      uint32_t* __restrict__ cursor, uint4* __restrict__ chunks,
-                                                      uint32_t* __restrict__ split)
+// places of the bricks' pairs (any order of bricks serves) and their chunks; counts back to
+// zero.  Two device atomics per block of 1024 bricks: per wave they were 7.2 us of one address
+// after the other (32768 bricks; 5.0 with the same chunks now).
+__global__ void __launch_bounds__(1024) k_sensor_place(uint32_t nb, SensorState* __restrict__ st, uint32_t* __restrict__ cnt,
+                                                       uint32_t* __restrict__ cursor, uint4* __restrict__ chunks,
+                                                       uint32_t* __restrict__ split)
 {
-  const uint32_t b = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+  __shared__ uint32_t wp[17], wk[17];
+  const uint32_t b = blockIdx.x * 1024 + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint32_t c = b < nb ? cnt[b] : 0u, cc = (c + SB_CHUNK - 1) / SB_CHUNK;
   uint32_t pc = c, pk = cc;
 #pragma unroll
@@ -867,14 +871,21 @@ __global__ void __launch_bounds__(256) k_sensor_place(uint32_t nb, SensorState* 
       pk += y1;
     }
   }
-  uint32_t base = 0, kbase = 0;
-  if (lane == 63 && pc) {
-    base = atomicAdd(&st->pairs, pc);
-    kbase = atomicAdd(&st->chunks, pk);
+  if (lane == 63) {
+    wp[w + 1] = pc;
+    wk[w + 1] = pk;
   }
-  base = __shfl(base, 63) + pc - c;
-  kbase = __shfl(kbase, 63) + pk - cc;
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    uint32_t* s = threadIdx.x ? wk : wp;
+    uint32_t sum = 0;
+    for (int i = 1; i <= 16; ++i) sum += s[i];
+    s[0] = sum ? atomicAdd(threadIdx.x ? &st->chunks : &st->pairs, sum) : 0u;
+    for (int i = 1; i < 16; ++i) s[i] += s[i - 1];
+  }
+  __syncthreads();
   if (c == 0u) return;
+  const uint32_t base = wp[w] + pc - c, kbase = wk[w] + pk - cc;
   cnt[b] = 0u;
   cursor[b] = base;
   for (uint32_t k = 0; k < cc; ++k)
@@ -882,8 +893,11 @@ __global__ void __launch_bounds__(256) k_sensor_place(uint32_t nb, SensorState* 
   if (cc > 1) split[atomicAdd(&st->split, 1u)] = b;
 }
 
-// the pairs (ray; entry cell and number of cells), sorted by brick: a block takes a stretch
-// per brick, its rays fill it
+// the pairs (ray; entry cell and number of cells), sorted by brick: a block takes SP_HELD
+// entries per thread at a time, counts them per brick, takes a stretch per brick and fills
+// it.  An entry's pair and place wait in registers for the stretch (cut twice instead: 60 us,
+// 41 now; 512 threads 50).
+constexpr uint32_t SP_HELD = 4;
 __global__ void __launch_bounds__(SR_THREADS) k_sensor_pairs(const SensorGeom g, const SensorState* __restrict__ st,
                                                              const uint64_t* __restrict__ list,
                                                              uint32_t* __restrict__ cursor, uint2* __restrict__ pairs)
@@ -892,33 +906,39 @@ __global__ void __launch_bounds__(SR_THREADS) k_sensor_pairs(const SensorGeom g,
   __shared__ SensorCut cut;
   const uint32_t m = st->targets;
   if (blockIdx.x * SR_RAYS >= m) return;  // uniform
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS) {
-    keys[i] = SH_NONE;
-    num[i] = 0u;
-  }
   sensor_cut(g, list, m, cut);
-  sensor_entries(g, cut, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
-    uint32_t b, at;
-    ray.cell(g, k, b, at);
-    const uint32_t h = sensor_slot(keys, b);
-    if (h != SH_NONE) atomicAdd(&num[h], 1u);
-  });
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
-    if (num[i]) num[i] = atomicAdd(cursor + keys[i], num[i]);
-  __syncthreads();
-  sensor_entries(g, cut, [&](uint32_t r, const SensorRay& ray, const uint32_t (&k)[3]) {
-    uint32_t b, at;
-    ray.cell(g, k, b, at);
-    // the keys are complete: the same slot as before, or none where there was none
-    uint32_t h = (b * 2654435761u) >> 21, slot = SH_NONE;
-    for (int probe = 0; probe < 16 && slot == SH_NONE; ++probe) {
-      if (keys[h] == b) slot = h;
-      h = (h + 1) % SH_SLOTS;
+  const uint32_t total = cut.pre[SR_RAYS];
+  for (uint32_t i0 = 0; i0 < total; i0 += SP_HELD * SR_THREADS) {  // uniform
+    for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS) {
+      keys[i] = SH_NONE;
+      num[i] = 0u;
     }
-    const uint32_t i = slot != SH_NONE ? atomicAdd(&num[slot], 1u) : atomicAdd(cursor + b, 1u);
-    pairs[i] = make_uint2(blockIdx.x * SR_RAYS + r, at | ray.stretch(k) << 12);  // at most 46 cells
-  });
+    __syncthreads();
+    uint32_t what[SP_HELD], slot[SP_HELD], nth[SP_HELD];
+#pragma unroll
+    for (uint32_t j = 0; j < SP_HELD; ++j) {
+      const uint32_t i = i0 + j * SR_THREADS + threadIdx.x;
+      slot[j] = SH_NONE;
+      if (i < total)
+        sensor_entry(g, cut, i, [&](uint32_t r, const SensorRay& ray, const uint32_t (&k)[3]) {
+          uint32_t b, at;
+          ray.cell(g, k, b, at);
+          what[j] = at | ray.stretch(k) << 12 | r << 18;  // at most 46 cells
+          slot[j] = sensor_slot(keys, b);
+          if (slot[j] != SH_NONE) nth[j] = atomicAdd(&num[slot[j]], 1u);
+          else pairs[atomicAdd(cursor + b, 1u)] = make_uint2(blockIdx.x * SR_RAYS + r, what[j] & 0x3FFFFu);
+        });
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
+      if (num[i]) num[i] = atomicAdd(cursor + keys[i], num[i]);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < SP_HELD; ++j)
+      if (slot[j] != SH_NONE)
+        pairs[num[slot[j]] + nth[j]] = make_uint2(blockIdx.x * SR_RAYS + (what[j] >> 18), what[j] & 0x3FFFFu);
+    __syncthreads();
+  }
 }
 
 // F free updates in a row on one voxel = max((unknown ? 0 : v) - 10 F, -127)
@@ -937,7 +957,7 @@ __device__ __forceinline__ uint64_t sensor_voxel(const SensorGeom& g, uint32_t b
   return ((uint64_t)z * g.dyd.d + y) * g.dxd.d + x;
 }
 
-__global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const SensorState* __restrict__ st,
+__global__ void __launch_bounds__(SC_THREADS) k_sensor_cells(const SensorGeom g, const SensorState* __restrict__ st,
                                                       const uint4* __restrict__ chunks, const uint2* __restrict__ pairs,
                                                       const uint64_t* __restrict__ list,
                                                       const uint32_t* __restrict__ weight, uint8_t* __restrict__ map,
@@ -948,10 +968,10 @@ __global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const 
   const uint32_t nc = st->chunks;
   for (uint32_t c = blockIdx.x; c < nc; c += gridDim.x) {  // uniform over the block
     const uint4 ch = chunks[c];
-    for (uint32_t i = threadIdx.x; i < SB_CELLS / 4; i += 256) num4[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (uint32_t i = threadIdx.x; i < SB_CELLS / 4; i += SC_THREADS) num4[i] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     const uint32_t o[3] = {ch.x % g.bx * SB, ch.x / g.bx % g.by * SB, ch.x / (g.bx * g.by) * SB};  // first voxel
-    for (uint32_t i = threadIdx.x; i < ch.z; i += 256) {
+    for (uint32_t i = threadIdx.x; i < ch.z; i += SC_THREADS) {
       const uint2 pr = pairs[ch.y + i];
       const uint32_t wgt = weight[pr.x];
       uint32_t t[3];
@@ -995,7 +1015,7 @@ __global__ void __launch_bounds__(256) k_sensor_cells(const SensorGeom g, const 
     __syncthreads();
     // 16 neighbouring lanes are 16 neighbouring voxels; bytes, since a word may belong to
     // two bricks
-    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += 256) {
+    for (uint32_t i = threadIdx.x; i < SB_CELLS; i += SC_THREADS) {
       const uint32_t f = num[i];
       if (!f) continue;
       const uint64_t v = sensor_voxel(g, ch.x, i);
@@ -1531,13 +1551,13 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
     ProfScope ps("sensor_rays");
     const unsigned gr = (unsigned)((n + SR_RAYS - 1) / SR_RAYS);
     hipLaunchKernelGGL(k_sensor_count, dim3(gr), dim3(SR_THREADS), 0, s, geom, P.st, P.list, hits, B.cnt);
-    hipLaunchKernelGGL(k_sensor_place, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, (uint32_t)nb, P.st, B.cnt,
+    hipLaunchKernelGGL(k_sensor_place, dim3((unsigned)((nb + 1023) / 1024)), dim3(1024), 0, s, (uint32_t)nb, P.st, B.cnt,
                        B.cursor, B.chunks, B.split);
     hipLaunchKernelGGL(k_sensor_pairs, dim3(gr), dim3(SR_THREADS), 0, s, geom, P.st, P.list, B.cursor, B.pairs);
-    const unsigned gc = (unsigned)(rt().num_cus > 0 ? rt().num_cus : 256) * 8;
-    hipLaunchKernelGGL(k_sensor_cells, dim3(gc), dim3(256), 0, s, geom, P.st, B.chunks, B.pairs, P.list, P.weight,
+    const unsigned gc = (unsigned)(rt().num_cus > 0 ? rt().num_cus : 256) * 16;
+    hipLaunchKernelGGL(k_sensor_cells, dim3(gc), dim3(SC_THREADS), 0, s, geom, P.st, B.chunks, B.pairs, P.list, P.weight,
                        (uint8_t*)m->data, hits);
-    hipLaunchKernelGGL(k_sensor_split, dim3(256), dim3(1024), 0, s, geom, P.st, B.split, dz, (uint8_t*)m->data, hits);
+    hipLaunchKernelGGL(k_sensor_split, dim3(512), dim3(1024), 0, s, geom, P.st, B.split, dz, (uint8_t*)m->data, hits);
     GVX_HIP(hipGetLastError());
   } else if (enable_raycasting) {
     {
