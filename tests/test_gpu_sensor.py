@@ -113,3 +113,21 @@ def test_sensor_bricks(gvx_lib, dims, n):
             g.insert_sensor_data(pts, sensor)
             O.prob_insert_sensor(o, dims, side, sensor, pts)
             assert np.array_equal(g.read(), o)
+
+
+@pytest.mark.parametrize("dims", [(4000, 20, 18), (640, 512, 384)])
+def test_sensor_long_rays(gvx_lib, dims):
+    """Rays that enter so many bricks that a block cuts its rays in several batches, and (the second
+    map, targets all around) more bricks in a batch than its table has slots."""
+    gvx = gvx_lib
+    side = 0.05
+    rng = np.random.default_rng(sum(dims))
+    for at in (0.02, 0.45):
+        sensor = (np.array(dims) * side * at).astype(np.float32)
+        pts = (rng.uniform(0, 1, (3000, 3)) * np.array(dims) * side).astype(np.float32)
+        pts[::2, 0] = rng.choice([0.01, dims[0] * side - 0.01], 1500).astype(np.float32)
+        g = gvx.Map(gvx.PROBAB_VOXELMAP, dims, side)
+        g.insert_sensor_data(pts, sensor)
+        o = O.new_map(O.PROB_MAP, dims)
+        O.prob_insert_sensor(o, dims, side, sensor, pts)
+        assert np.array_equal(g.read(), o)
