@@ -692,10 +692,12 @@ struct PoseArgs {
 // costs 5 us before its first point.  Calls, a prologue and work items of 128 points x 512
 // poses before: 64 poses of 40k points from host memory 66 -> 33 us, the 1024 poses 103 ->
 // 90, an environment with a tenth of all voxels occupied 1274 -> 514 (96 poses 375 -> 122); the
-// first call on new buffers 286 -> 86.  Tried: a bit per occupied voxel in LDS (one block per
-// CU, 88), a line per occupied brick instead of the whole bitmap (the same), a second box test
-// against single voxels (10 % fewer chunks, no faster), two chunks at a time in 64 registers
-// (105).
+// first call on new buffers 286 -> 86.  Four chunks at a time with 1024 threads, a block per
+// CU; three with 512, three blocks in 80 registers (1024 poses of 150k points 83 us, with four
+// and two blocks 88).  Tried: a bit per occupied voxel in LDS, a line per occupied brick
+// instead of the whole bitmap (both the same), a second box test against single voxels
+// (10 % fewer chunks, no faster), two chunks at a time in 64 registers (a tenth slower, they
+// spill).
 constexpr uint32_t PB_RUNS = 64;    // runs per round of broad and narrow phase
 constexpr uint32_t PB_HASH = 4096;  // slots
 constexpr uint32_t PB_PROBES = 16;
@@ -760,7 +762,7 @@ __device__ __forceinline__ void pose_unmark(const PoseArgs& a, const uint32_t* s
 }
 
 template <int TB>
-__global__ void __launch_bounds__(TB) k_batch_pose(const PoseArgs a)
+__global__ void __launch_bounds__(TB, TB == 512 ? 6 : 4) k_batch_pose(const PoseArgs a)
 {
   extern __shared__ float4 pose_lds_mem[];
   float* sT = reinterpret_cast<float*>(pose_lds_mem);                        // nl x 12
@@ -769,7 +771,7 @@ __global__ void __launch_bounds__(TB) k_batch_pose(const PoseArgs a)
   uint32_t* sH = reinterpret_cast<uint32_t*>(sL + PB_RUNS * kRun);           // PB_HASH slots: key + 1, 0: free
   float* sA = reinterpret_cast<float*>(sH);                                  // before that: nl x 12 DH matrices
   __shared__ uint32_t s_n, s_live, s_count, s_mask[8], s_stat[2], s_over;
-  constexpr int U = 4, NW = TB / 64;
+  constexpr int U = TB == 512 ? 3 : 4, NW = TB / 64;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t pose = blockIdx.x;
   // the first runs' boxes are on their way while the link frames are built
@@ -861,14 +863,10 @@ __global__ void __launch_bounds__(TB) k_batch_pose(const PoseArgs a)
         p[u] = *reinterpret_cast<const Point*>(base + lane * 12);
       }
       float c[U][3], off[U], most = 0.f;  // voxel coordinates by the reciprocal; the distance from a voxel's middle
-      uint32_t have = ~0u;
       float m[12];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (link[u] != have) {  // uniform, and rare after the first: the list holds run after run
-          load_frame(sT + 12 * link[u], m);
-          have = link[u];
-        }
+        load_frame(sT + 12 * link[u], m);  // one address per wave (kept while the link is the same: 5 % slower)
         transform(m, p[u].x, p[u].y, p[u].z, c[u][0], c[u][1], c[u][2]);
         off[u] = 0.f;
 #pragma unroll
@@ -1105,11 +1103,11 @@ static bool pose_blocks_suit(const BatchS* b)
 // The kernel a schedule takes for n poses.  Schedule 0 takes a block per pose unless the poses
 // are few for their points: one CU then walks what 128-point chunks spread over the chip.
 // Call times, device memory, pose blocks against 128-point chunks, links of 150k points in
-// 512^3: 4 poses 34 / 26 us, 16: 39 / 37, 64: 40 / 43, 256: 45 / 63, 1024: 94 / 106;
-// 60k points in 256^3: 4: 28 / 26, 16: 31 / 34, 64: 31 / 43, 1024: 64 / 135; 20k points: 4: 23 / 23,
-// 64: 23 / 33, 1024: 43 / 89.  A pose takes 1024 threads while a CU has at most three poses
-// (150k points, 64 poses: 47 us with 512), and 512 beyond, where two blocks share a CU (1024
-// poses: 104 us with 1024; 20k points 53).
+// 512^3: 4 poses 34 / 26 us, 16: 39 / 37, 64: 38 / 43, 256: 45 / 63, 1024: 83 / 106;
+// 60k points in 256^3: 4: 28 / 26, 16: 31 / 34, 64: 30 / 43, 1024: 58 / 135; 20k points: 4: 23 / 23,
+// 64: 23 / 33, 1024: 39 / 89.  A pose takes 1024 threads while a CU has at most three poses
+// (150k points, 64 poses: 47 us with 512; 512 poses 62 and 65), and 512 beyond, where three
+// blocks share a CU (1024 poses: 98 us with 1024; 20k points 52).
 static int kernel_schedule(const BatchS* b, uint32_t n, int ks)
 {
   const uint32_t cus = (uint32_t)(rt().num_cus > 0 ? rt().num_cus : 256);
