@@ -35,23 +35,24 @@ __device__ __forceinline__ void voxel_insert(uint8_t* map, uint64_t idx, uint32_
   }
 }
 
-// `count` ProbabilisticVoxel::insert(meaning) updates in a row on voxel idx, one CAS
-// (identical updates: any order gives the same byte)
-__device__ __forceinline__ void prob_insert_n(uint8_t* map, uint64_t idx, uint32_t meaning, uint32_t count)
+// ProbabilisticVoxel::insert(meaning) updates on the four voxels of a 32-bit word, counts byte
+// by byte, with one CAS (identical updates: any order gives the same byte)
+__device__ __forceinline__ void prob_insert_word(uint32_t* w, uint32_t meaning, uint32_t counts)
 {
-  uint32_t* w = reinterpret_cast<uint32_t*>(map + (idx & ~(uint64_t)3));
-  const uint32_t sh = (uint32_t)(idx & 3) * 8;
   uint32_t old = __atomic_load_n(w, __ATOMIC_RELAXED);
   for (;;) {
-    const int cur = (int)(int8_t)((old >> sh) & 0xFF);
-    int nv = cur;
-    for (uint32_t k = 0; k < count; ++k) {
-      const int n2 = prob_insert(nv, meaning);
-      if (n2 == nv) break;
-      nv = n2;
+    uint32_t neu = 0;
+#pragma unroll
+    for (int b = 0; b < 32; b += 8) {
+      int v = (int)(int8_t)(old >> b);
+      for (uint32_t k = (counts >> b) & 0xFFu; k; --k) {
+        const int n = prob_insert(v, meaning);
+        if (n == v) break;
+        v = n;
+      }
+      neu |= (uint32_t)(uint8_t)(int8_t)v << b;
     }
-    if (nv == cur) return;
-    const uint32_t neu = (old & ~(0xFFu << sh)) | ((uint32_t)(uint8_t)(int8_t)nv << sh);
+    if (neu == old) return;
     const uint32_t prev = atomicCAS(w, old, neu);
     if (prev == old) return;
     old = prev;
@@ -82,11 +83,21 @@ __global__ void __launch_bounds__(256) k_insert_points(uint8_t* __restrict__ map
                    z = quantize(pts[3 * i + 2], side);
     const bool in = (x < dx) && (y < dy) && (z < dz);
     if constexpr (T == TPROB) {
-      // neighbouring points often share a voxel: a run of lanes on one voxel
-      // updates it with one CAS (identical updates commute)
+      // neighbouring points often share a voxel or the word of four: a run of lanes on one
+      // word updates it with one CAS, its points per voxel counted in the word's bytes (at
+      // most 64).  A CAS per voxel had the lanes of a word wait for each other (304k points
+      // of a depth image into 512^3, by scene: 16.5 -> 15.9 us, clear and insert 68 -> 63)
       const uint64_t idx = in ? ((uint64_t)z * dy + y) * dx + x : 0ull;
-      const uint32_t run = wave_run_head(in, idx, m);
-      if (run) prob_insert_n(map, idx, m, run);
+      const uint32_t lane = threadIdx.x & 63, own = in ? 1u << (8 * (uint32_t)(idx & 3)) : 0u;
+      const uint32_t run = wave_run_head(in, idx >> 2, m);
+      uint32_t sum = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t below = __shfl_up(sum, o);
+        if (lane >= (uint32_t)o) sum += below;
+      }
+      const uint32_t counts = __shfl(sum, (int)(run ? lane + run - 1 : lane)) - (sum - own);
+      if (run) prob_insert_word(reinterpret_cast<uint32_t*>(map) + (idx >> 2), m, counts);
     } else if constexpr (T == TBIT) {
       // setting a bit is idempotent: one lane per run on one (voxel, meaning) sets it
       const uint64_t idx = in ? ((uint64_t)z * dy + y) * dx + x : 0ull;

@@ -279,3 +279,37 @@ def test_cfg2_scene(gvx_lib):
     n2, mask2 = O.map_collide_types(O.BITVECTOR_MAP, orob, O.PROB_MAP, oenv, d, 1.0)
     assert n == n2 and np.array_equal(mask, mask2)
     assert robot.collide(env, 1.0) == O.map_collide(O.BITVECTOR_MAP, orob, O.PROB_MAP, oenv, d, 1.0)
+
+
+@pytest.mark.parametrize("dims", [(13, 7, 5), (64, 3, 2), (1, 1, 1)])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 5000])
+def test_insert_prob_words(gvx_lib, dims, n):
+    """Runs of points on one 32-bit word of a Prob map: sorted points that fill a word's four voxels,
+    zigzag inside a word, a whole wave on one voxel, rows that do not end with a word, points outside
+    in between; every kind of meaning, from an unknown and from a filled map, one and several clouds."""
+    gvx = gvx_lib
+    side = 0.25  # exact
+    rng = np.random.default_rng(sum(dims) * 100 + n)
+    d = np.array(dims)
+    cell = np.sort(rng.integers(0, int(d.prod()), n))
+    cell[n // 2:n // 2 + 64] = cell[n // 2]
+    cell[:32] ^= (np.arange(n)[:32] * 3) % 4
+    cell = np.minimum(cell, int(d.prod()) - 1)
+    v = np.stack([cell % dims[0], cell // dims[0] % dims[1], cell // (dims[0] * dims[1])], 1)
+    v[rng.random(n) < 0.05] += d
+    p = ((v + 0.5) * side).astype(np.float32)
+    g, o = _map(gvx, O.PROB_MAP, dims, side), O.new_map(O.PROB_MAP, dims)
+    for m in (1, 0, 60, 2, 255, 1, 3, 1, 1):
+        assert g.insert_points(p, m) == O.map_insert_points(O.PROB_MAP, o, dims, side, p, m)
+        assert np.array_equal(g.read(), o), m
+    sizes = np.array([n // 3, n - n // 3], np.uint32)
+    for meanings in ([1, 1], [0, 1], [40, 90]):
+        # meanings that differ on one voxel do not commute: the clouds lie in different rows of words
+        q = p.copy()
+        if meanings[0] != meanings[1]:
+            q[:n // 3, 2], q[n // 3:, 2] = side / 2, (dims[2] - 0.5) * side
+            if dims[2] == 1:
+                continue
+        mn = np.array(meanings, np.uint32)
+        assert g.insert_meta(q, sizes, mn) == O.map_insert_meta(O.PROB_MAP, o, dims, side, q, sizes, mn)
+        assert np.array_equal(g.read(), o), meanings
