@@ -433,8 +433,15 @@ static unsigned stream_grid(uint64_t n)
 
 // kernels that stream a ProbVoxelMap: one round of kLoadsInFlight chunks per lane, so that
 // waves that wait for memory are replaced by others instead of looping (512^3: 31 us with
-// 8 blocks per CU and 4 rounds each, 24 us)
-static unsigned prob_grid(uint64_t chunks) { return grid_for((chunks + kLoadsInFlight - 1) / kLoadsInFlight, 256, 1u << 16); }
+// 8 blocks per CU and 4 rounds each, 24 us).  Below 4 blocks per CU a lane takes fewer
+// chunks, since a wave visits the passing voxels of its chunks one after another (a call on
+// 64^3 21.2 -> 17.4 us, 128^3 20.9 -> 17.2, 200 x 200 x 150 19.2 -> 17.6, 256^3 equal; with 1
+// or 2 blocks per CU the middle ones 18.5 to 19.2).
+static unsigned prob_grid(uint64_t chunks)
+{
+  const unsigned rounds = grid_for((chunks + kLoadsInFlight - 1) / kLoadsInFlight, 256, 1u << 16);
+  return std::max(rounds, grid_for(chunks, 256, (unsigned)(rt().num_cus > 0 ? rt().num_cus : 256) * 4));
+}
 
 // scan_bit_voxels: a block reads 32 kHalves x 4 voxels per iteration
 static unsigned bits_grid(uint64_t voxels) { return grid_for((voxels + 32 * kHalves - 1) / (32 * kHalves) * 64, 256, 1u << 16); }
