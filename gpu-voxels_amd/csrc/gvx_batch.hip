@@ -1106,14 +1106,16 @@ static bool pose_blocks_suit(const BatchS* b)
 // 512^3: 4 poses 34 / 26 us, 16: 39 / 37, 64: 38 / 43, 256: 45 / 63, 1024: 83 / 106;
 // 60k points in 256^3: 4: 28 / 26, 16: 31 / 34, 64: 30 / 43, 1024: 58 / 135; 20k points: 4: 23 / 23,
 // 64: 23 / 33, 1024: 39 / 89.  A pose takes 1024 threads while a CU has at most three poses
-// (150k points, 64 poses: 47 us with 512; 512 poses 62 and 65), and 512 beyond, where three
-// blocks share a CU (1024 poses: 98 us with 1024; 20k points 52).
+// (150k points, 64 poses: 38 us, with 512 47; 512 poses 62 and 65), and 512 beyond, where
+// three blocks share a CU (1024 poses of 40k points in eight scenes: 44 to 61 us with 1024, 35
+// to 52 with 512) -- but not for many points, whose longest pose then lasts longest (150k
+// points: 61 to 107 us with 1024, 55 to 112 with 512).
 static int kernel_schedule(const BatchS* b, uint32_t n, int ks)
 {
   const uint32_t cus = (uint32_t)(rt().num_cus > 0 ? rt().num_cus : 256);
   if (ks == 0 && b->n_pts > 4096ull * n) return 1;
   if (kSchedules[ks].chunk == 0 && !pose_blocks_suit(b)) return 1;
-  return ks == 0 ? (n > 3 * cus ? 6 : 7) : ks;
+  return ks == 0 ? (n > 3 * cus && b->n_pts <= 1u << 17 ? 6 : 7) : ks;
 }
 
 // chunks of `block` consecutive points of one link (the last one of a link may be
