@@ -110,7 +110,7 @@ struct BatchS {
   uint32_t tcap = 0;
   bool touched = false;  // the last call listed words that are still set
   // pinned host memory that pose blocks read joint values from and write results to: q, then
-  // max_poses x (8 mask words), then counts; null: too many poses
+  // max_poses x (8 mask words), then counts; null: too many poses, or no such memory
   uint32_t* io = nullptr;
   uint32_t io_q = 0;           // poses in it, if the last joint values from the host went there
   uint32_t* counts = nullptr;  // max_poses
@@ -1379,8 +1379,10 @@ int gvx_batch_create(gvx_map env, float threshold, const float* link_pts, const 
     return bail(s);
   if ((s = dalloc((void**)&b->tcnt, kTouchSlots * kTouchStride * 4)) != GVX_OK) return bail(s);
   const uint64_t io_bytes = (uint64_t)max_poses * (n_links + 9) * 4;
-  if (io_bytes <= kIoMax && hipHostMalloc((void**)&b->io, io_bytes, hipHostMallocCoherent) != hipSuccess)
-    return bail(fail(GVX_ERR_OOM, "pinned memory"));
+  if (io_bytes <= kIoMax && hipHostMalloc((void**)&b->io, io_bytes, hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    b->io = nullptr;  // calls copy instead
+  }
   b->lwords = (max_poses + 31) / 32;
   if ((s = dalloc((void**)&b->llive, (uint64_t)n_links * b->lwords * 4)) != GVX_OK) return bail(s);
   if ((s = dalloc((void**)&b->lbox, (uint64_t)n_links * 24)) != GVX_OK) return bail(s);

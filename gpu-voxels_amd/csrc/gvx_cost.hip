@@ -20,7 +20,7 @@
 // What bounds it: the samples.  8192 random waypoints of 7 x 64 spheres on 512^3 miss L2
 // 4.8 M times, 52 lines per ns, at a VALU load of a third; costs, gradient or both take the
 // same 92-95 us.  So the costs and their gradient come from one pass where both are wanted
-// (gvx_cost_forward_grad: an optimiser's step 265 -> 160 us).  Loads past the L1
+// (gvx_cost_forward_grad: an optimiser's step 341 -> 213 us with the host work of torch).  Loads past the L1
 // (non-temporal) lose the lines that neighbouring spheres share: 129 us.
 //
 // Whole waves per link and a block per waypoint (as this file had it) left lanes idle and one
@@ -282,7 +282,8 @@ __global__ void __launch_bounds__(64 * CMAXW) k_cost_bwd(const CostArgs c, const
         }
         if (dxo) {
           float* o = dxo + ((tw0 + p) * ns + ks) * 3;
-          o[0] = ax * up; o[1] = ay * up; o[2] = az * up;
+          const bool on = h > 0.f;  // an idle sphere's zero stays one whatever the factor
+          o[0] = on ? ax * up : 0.f; o[1] = on ? ay * up : 0.f; o[2] = on ? az * up : 0.f;
         }
         const float rx = x - m[3], ry = y - m[7], rz = z - m[11];
         c6[0] += ax; c6[1] += ay; c6[2] += az;
@@ -328,7 +329,8 @@ __global__ void __launch_bounds__(64 * CMAXW) k_cost_bwd(const CostArgs c, const
       }
       r = zx * cx + zy * cy + zz * cz;
     }
-    dq[tw0 * c.nl + e] = upstream ? r * upstream[(uint32_t)(tw0 + e / c.nl) / c.nwp] : r;
+    // zero without contact, also where the factor is infinite (the root of a cost of zero)
+    dq[tw0 * c.nl + e] = upstream && r != 0.f ? r * upstream[(uint32_t)(tw0 + e / c.nl) / c.nwp] : r;
   }
   if (partial && threadIdx.x < nw) {
     float s = 0.f;

@@ -31,7 +31,8 @@ class ClearanceCostFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         _, dq = ctx.saved_tensors
-        return dq * grad_out.detach().float()[:, None, None], None
+        # zero without contact, also where grad_out is infinite (the root of a cost of zero)
+        return torch.where(dq == 0, dq, dq * grad_out.detach().float()[:, None, None]), None
 
 
 def clearance_cost(q, cost: Cost):

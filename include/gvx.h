@@ -284,7 +284,7 @@ int gvx_cost_backward(gvx_cost c, const float* q_dev, uint32_t n_traj, uint32_t 
                       const float* upstream_dev, float* dq_out_dev, float* dx_out_dev);
 /* both in one pass over the grid: cost_out as gvx_cost_forward writes it, dq_out as
    gvx_cost_backward does for an upstream of ones.  The upstream factor is the last one applied
-   (dq = upstream * dq_out, the same bits as gvx_cost_backward). */
+   (dq = upstream * dq_out where dq_out is not zero, the same bits as gvx_cost_backward). */
 int gvx_cost_forward_grad(gvx_cost c, const float* q_dev, uint32_t n_traj, uint32_t n_wp, float* cost_out_dev,
                           float* dq_out_dev);
 

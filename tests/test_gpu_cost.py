@@ -375,3 +375,38 @@ def test_cost_layouts(gvx_lib, nl, spl, ntraj, nwp, dims):
     assert np.all(err <= 3e-5 * size)
     # a joint's term: |dc/dx| times a lever of at most the arm's reach
     assert np.all(np.abs(dq.cpu().numpy() - odq) <= 3e-5 * 0.5 * size.sum(axis=(2, 3))[:, :, None])
+
+
+def test_cost_infinite_upstream(gvx_lib):
+    """The gradient of a trajectory (or waypoint) without contact is zero whatever its upstream factor,
+    as in sqrt(cost) at a cost of zero; one in contact takes the factor."""
+    import torch
+    from gvx.torch_cost import clearance_cost
+    gvx = gvx_lib
+    d, side = (32, 32, 32), 0.1
+    k = torch.arange(32, device="cuda", dtype=torch.float32)
+    grid = (k[:, None, None] * 0.1).expand(32, 32, 32).reshape(-1).contiguous()  # distance grows with z
+    dh = np.array([[0, 0.3, 0, 0, 1], [0, 0.1, 0.1, 0, 0]], np.float32)
+    sph = np.zeros((2, 20, 4), np.float32)
+    sph[1, :, 0] = np.linspace(0, 0.1, 20)
+    sph[:, :, 3] = 0.1
+    base = np.array([1, 0, 0, 1.6, 0, 1, 0, 1.6, 0, 0, 1, 0.0], np.float32)
+    cost = gvx.Cost(grid, d, side, dh, sph[:, :, :], 0.6, 1.0, base)
+    cost_free = gvx.Cost(grid, d, side, dh, sph[:, :, :], -0.1, 1.0, base)
+    q = torch.zeros((3, 4, 2), device="cuda")
+    q[1, :, 0] = 2.0                     # link 1 high above; link 0 stays in contact
+    q[2, 0, 1] = 0.5
+    inf = torch.tensor([float("inf"), float("nan"), 2.0], device="cuda")
+    dq, dx = torch.empty_like(q), torch.empty((3, 4, 2, 20, 3), device="cuda")
+    torch.cuda.synchronize()
+    cost_free.backward(q, dq, dx, inf)
+    c = torch.empty(3, device="cuda")
+    cost_free.forward(q, c)
+    assert torch.equal(c, torch.zeros_like(c)) and torch.equal(dq, torch.zeros_like(dq))
+    assert torch.equal(dx, torch.zeros_like(dx))
+    p = q.clone().requires_grad_(True)
+    clearance_cost(p, cost_free).sqrt().sum().backward()
+    assert torch.equal(p.grad, torch.zeros_like(q))
+    cost.backward(q, dq, dx, inf)        # link 1 of trajectory 0 hangs in the field: dc/dq_0 != 0
+    assert torch.isinf(dq[0, :, 0]).all() and torch.isfinite(dq[2]).all() and (dq[2, :, 0] != 0).all()
+    assert torch.isinf(dx[0, :, 1, :, 2]).all() and torch.equal(dq[1], torch.zeros_like(dq[1]))
