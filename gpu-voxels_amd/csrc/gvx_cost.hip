@@ -257,7 +257,6 @@ __global__ void __launch_bounds__(64 * CMAXW) k_cost_bwd(const CostArgs c, const
   block_fk<WB>(c, tw0, nw, A, T);
   const uint32_t ns = c.nl * c.spl;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-#pragma unroll 2
   for (uint32_t p = 0; p < nw; ++p) {
     const float up = upstream && dxo ? upstream[(uint32_t)(tw0 + p) / c.nwp] : 1.0f;  // n < 2^31
     float acc = 0.f;

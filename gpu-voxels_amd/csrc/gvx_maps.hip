@@ -646,7 +646,7 @@ __global__ void __launch_bounds__(256) k_sensor_untag(uint32_t* __restrict__ hit
 // a block walks a brick's pairs with the 4096 counters in LDS and updates the brick's
 // voxels itself.  Bricks near the sensor hold most rays: their pairs are cut into chunks of
 // SB_CHUNK, whose counters meet in memory (hits, zero at rest) before the voxels are
-// updated.  That frame: count 23, place 6, pairs 41, cells 50, split 10 us; all of them
+// updated.  That frame: count 23, place 6, pairs 39, cells 48, split 10 us; all of them
 // half bound by instruction issue, half by latency.  Chunks of 1024 pairs, 512 threads
 // each and 16 blocks per CU end more evenly than 2048, 256 and 8: cells 69 + split 6 us
 // then (4096: 94 + 5; 1024 with 1024 threads 56).
@@ -754,7 +754,7 @@ struct SensorRay {
 
 // The entries of a block's rays, one thread each: the rays' targets and the prefix of
 // their entry counts in LDS.  (A thread per ray, face after face, took as long as the
-// longest ray: 43 + 77 us for the two kernels below, against 24 + 41 us.)
+// longest ray: 43 + 77 us for the two kernels below, against 23 + 39 us.)
 struct SensorCut {
   uint32_t t[3][SR_RAYS], pre[SR_RAYS + 1];
 };
@@ -786,20 +786,25 @@ __device__ __forceinline__ void sensor_cut(const SensorGeom& g, const uint64_t* 
   if (r >= 64 && r < SR_RAYS) c.pre[r + 1] += first;
   __syncthreads();
 }
-// entry i of the block: f(ray of the block, its SensorRay, steps at the entry)
-template <typename F>
-__device__ __forceinline__ void sensor_entry(const SensorGeom& g, const SensorCut& c, uint32_t i, F&& f)
+// the rays of the block's entries [i0, i0 + SP_BATCH), written by 8 threads per ray (a binary
+// search of the prefix per entry instead: pairs 41 us, 39 now)
+constexpr uint32_t SP_HELD = 4, SP_BATCH = SP_HELD * SR_THREADS;  // entries per thread and per block at a time
+__device__ __forceinline__ void sensor_owners(const SensorCut& c, uint32_t i0, uint8_t* own)
 {
-  uint32_t lo = 0, hi = SR_RAYS;  // the last ray whose prefix is at most i (rays without entries come last)
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (c.pre[mid] <= i) lo = mid; else hi = mid;
-  }
-  const uint32_t t[3] = {c.t[0][lo], c.t[1][lo], c.t[2][lo]};
+  static_assert(SR_THREADS == 8 * SR_RAYS && SR_RAYS <= 256, "8 threads per ray, a byte per entry");
+  const uint32_t r = threadIdx.x / 8, end = min(c.pre[r + 1], i0 + SP_BATCH);
+  for (uint32_t i = max(c.pre[r], i0) + threadIdx.x % 8; i < end; i += 8) own[i - i0] = (uint8_t)r;
+  __syncthreads();
+}
+// entry i of the block's ray r: f(its SensorRay, steps at the entry)
+template <typename F>
+__device__ __forceinline__ void sensor_entry(const SensorGeom& g, const SensorCut& c, uint32_t r, uint32_t i, F&& f)
+{
+  const uint32_t t[3] = {c.t[0][r], c.t[1][r], c.t[2][r]};
   const SensorRay ray(g, t);
   uint32_t k[3];
-  ray.entry(i - c.pre[lo], ray.faces(0), ray.faces(1), k);
-  f(lo, ray, k);
+  ray.entry(i - c.pre[r], ray.faces(0), ray.faces(1), k);
+  f(ray, k);
 }
 
 // a block's bricks with their pairs: slot of brick b, or SH_NONE when the table is full
@@ -825,6 +830,7 @@ __global__ void __launch_bounds__(SR_THREADS) k_sensor_count(const SensorGeom g,
                                                              uint32_t* __restrict__ hits, uint32_t* __restrict__ cnt)
 {
   __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
+  __shared__ uint8_t own[SP_BATCH];
   __shared__ SensorCut cut;
   const uint32_t m = st->targets;
   if (blockIdx.x * SR_RAYS >= m) return;  // uniform
@@ -834,15 +840,19 @@ __global__ void __launch_bounds__(SR_THREADS) k_sensor_count(const SensorGeom g,
   }
   if (threadIdx.x < SR_RAYS && blockIdx.x * SR_RAYS + threadIdx.x < m) hits[list[blockIdx.x * SR_RAYS + threadIdx.x]] = 0u;
   sensor_cut(g, list, m, cut);
-  for (uint32_t i = threadIdx.x; i < cut.pre[SR_RAYS]; i += SR_THREADS)
-    sensor_entry(g, cut, i, [&](uint32_t, const SensorRay& ray, const uint32_t (&k)[3]) {
-      uint32_t b, at;
-      ray.cell(g, k, b, at);
-      const uint32_t h = sensor_slot(keys, b);
-      if (h != SH_NONE) atomicAdd(&num[h], 1u);
-      else atomicAdd(cnt + b, 1u);
-    });
-  __syncthreads();
+  const uint32_t total = cut.pre[SR_RAYS];
+  for (uint32_t i0 = 0; i0 < total; i0 += SP_BATCH) {  // uniform
+    sensor_owners(cut, i0, own);
+    for (uint32_t i = i0 + threadIdx.x; i < min(total, i0 + SP_BATCH); i += SR_THREADS)
+      sensor_entry(g, cut, own[i - i0], i, [&](const SensorRay& ray, const uint32_t (&k)[3]) {
+        uint32_t b, at;
+        ray.cell(g, k, b, at);
+        const uint32_t h = sensor_slot(keys, b);
+        if (h != SH_NONE) atomicAdd(&num[h], 1u);
+        else atomicAdd(cnt + b, 1u);
+      });
+    __syncthreads();
+  }
   for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
     if (num[i]) atomicAdd(cnt + keys[i], num[i]);
 }
@@ -891,31 +901,32 @@ __global__ void __launch_bounds__(1024) k_sensor_place(uint32_t nb, SensorState*
 // the pairs (ray; entry cell and number of cells), sorted by brick: a block takes SP_HELD
 // entries per thread at a time, counts them per brick, takes a stretch per brick and fills
 // it.  An entry's pair and place wait in registers for the stretch (cut twice instead: 60 us,
-// 41 now; 512 threads 50).
-constexpr uint32_t SP_HELD = 4;
+// 39 now; 512 threads 50).
 __global__ void __launch_bounds__(SR_THREADS) k_sensor_pairs(const SensorGeom g, const SensorState* __restrict__ st,
                                                              const uint64_t* __restrict__ list,
                                                              uint32_t* __restrict__ cursor, uint2* __restrict__ pairs)
 {
   __shared__ uint32_t keys[SH_SLOTS], num[SH_SLOTS];
+  __shared__ uint8_t own[SP_BATCH];
   __shared__ SensorCut cut;
   const uint32_t m = st->targets;
   if (blockIdx.x * SR_RAYS >= m) return;  // uniform
   sensor_cut(g, list, m, cut);
   const uint32_t total = cut.pre[SR_RAYS];
-  for (uint32_t i0 = 0; i0 < total; i0 += SP_HELD * SR_THREADS) {  // uniform
+  for (uint32_t i0 = 0; i0 < total; i0 += SP_BATCH) {  // uniform
     for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS) {
       keys[i] = SH_NONE;
       num[i] = 0u;
     }
-    __syncthreads();
+    sensor_owners(cut, i0, own);
     uint32_t what[SP_HELD], slot[SP_HELD], nth[SP_HELD];
 #pragma unroll
     for (uint32_t j = 0; j < SP_HELD; ++j) {
       const uint32_t i = i0 + j * SR_THREADS + threadIdx.x;
       slot[j] = SH_NONE;
-      if (i < total)
-        sensor_entry(g, cut, i, [&](uint32_t r, const SensorRay& ray, const uint32_t (&k)[3]) {
+      if (i < total) {
+        const uint32_t r = own[i - i0];
+        sensor_entry(g, cut, r, i, [&](const SensorRay& ray, const uint32_t (&k)[3]) {
           uint32_t b, at;
           ray.cell(g, k, b, at);
           what[j] = at | ray.stretch(k) << 12 | r << 18;  // at most 46 cells
@@ -923,6 +934,7 @@ __global__ void __launch_bounds__(SR_THREADS) k_sensor_pairs(const SensorGeom g,
           if (slot[j] != SH_NONE) nth[j] = atomicAdd(&num[slot[j]], 1u);
           else pairs[atomicAdd(cursor + b, 1u)] = make_uint2(blockIdx.x * SR_RAYS + r, what[j] & 0x3FFFFu);
         });
+      }
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < SH_SLOTS; i += SR_THREADS)
