@@ -21,7 +21,7 @@
 //           entries' first positions, whole row segments written).
 // Small maps take one kernel each for y and x (k_pba_y_chunk, k_pba_x_chunk), which
 // search outwards over chunks of a line whatever the field.
-// All bisector tests are exact integer comparisons.
+// All bisector tests compare whole numbers exactly.
 #include "gvx_internal.hpp"
 
 namespace gvx {
@@ -182,12 +182,13 @@ __global__ void __launch_bounds__(256) k_pba_z_long(const uint32_t* __restrict__
 // each lane walks only the positions of a tile that hold a site (a bit mask), so
 // empty stretches of a line cost nothing.
 //
-// Bisector tests are exact integer arithmetic.  For sites a < b on the line
-// (positions pa, pb; squared off-line costs ca, cb), a is at least as close as b
-// at position p exactly when p * D <= N with N = (pb^2 - pa^2) + cb - ca and
-// D = 2 (pb - pa) > 0.  Positions are < 1024 and costs < 2^21, so N < 2^23 and
-// p * D < 2^21 fit int32; phase 2's comparison N_ab * D_bc >= N_bc * D_ab (pop b,
-// also on equality) has products < 2^34 (middle_empty).
+// Bisector tests are exact.  For sites a < b on the line (positions pa, pb; squared
+// off-line costs ca, cb), a is at least as close as b at position p exactly when
+// 2 p D <= N with N = (pb^2 - pa^2) + cb - ca and D = pb - pa > 0; phase 2's comparison
+// is N_ab * D_bc >= N_bc * D_ab (pop b, also on equality).  Positions are below 1024 and
+// z below 4094, so costs reach 1023^2 + 4093^2 > 2^24: the numbers are floats where a
+// whole diagonal stays below 2^24 (any map of up to 3832 layers) and integers beyond
+// (bis_floats).
 #ifndef GVX_PBA_TYR
 #define GVX_PBA_TYR 32
 #endif
@@ -223,10 +224,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t slice_rsrc(const void* base, u
                                            __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
 }
 
-// bisector of sites a < b: a is at least as close as b at p  <=>  2 p D <= N.  Whole numbers
-// below 2^24 in floats, each step exact.
-struct Bis {
-  float N, D;
+// Do costs, and with a line's squared positions every N, stay below 2^24?  Then they are
+// floats (T of the kernels below), else integers.
+static inline bool bis_floats(uint32_t dx, uint32_t dy, uint32_t dz)
+{
+  return (uint64_t)(dx - 1) * (dx - 1) + (uint64_t)(dy - 1) * (dy - 1) + (uint64_t)(dz - 1) * (dz - 1) < (1u << 24);
+}
+// bisector of sites a < b: a is at least as close as b at p  <=>  2 p D <= N
+template <typename T>
+struct Bis;
+// whole numbers below 2^24 in floats, each step exact
+template <>
+struct Bis<float> {
+  float N = 0.f, D = 1.f;
   __device__ __forceinline__ void set(float pa, float ca, float pb, float cb)
   {
     D = pb - pa;
@@ -234,15 +244,30 @@ struct Bis {
   }
   __device__ __forceinline__ bool a_wins(float p) const { return 2.0f * p * D <= N; }
 };
+// N below 2^25
+template <>
+struct Bis<int32_t> {
+  int32_t N = 0, D = 1;
+  __device__ __forceinline__ void set(int32_t pa, int32_t ca, int32_t pb, int32_t cb)
+  {
+    D = pb - pa;
+    N = __mul24(D, pb + pa) + (cb - ca);
+  }
+  __device__ __forceinline__ bool a_wins(int32_t p) const { return 2 * __mul24(p, D) <= N; }
+};
 // b (the middle of a < b < c) owns no position: bisector(a, b) >= bisector(b, c), N_ab D_bc >=
 // N_bc D_ab.  With p the rounded right side, its error is a whole number below 2^9 and a
 // float, and the left side less p is a whole number that rounds only above 2^24: the two
 // compare as the products do.  (In double precision the stack kernels of a 512^3 room took
 // 313 and 112 us, this way 309 and 106: the chain of a line and its LDS round trips are longer.)
-__device__ __forceinline__ bool middle_empty(const Bis& ab, const Bis& bc)
+__device__ __forceinline__ bool middle_empty(const Bis<float>& ab, const Bis<float>& bc)
 {
   const float p = bc.N * ab.D;
   return fmaf(ab.N, bc.D, -p) >= fmaf(bc.N, ab.D, -p);
+}
+__device__ __forceinline__ bool middle_empty(const Bis<int32_t>& ab, const Bis<int32_t>& bc)
+{
+  return (double)ab.N * (double)bc.D >= (double)bc.N * (double)ab.D;  // products below 2^35
 }
 
 // Per-lane stack of 32-bit entries: ring[depth % RK][lane] holds depths [lo, n);
@@ -292,6 +317,7 @@ struct LineStack {
 // Row tiles whose 64 x 32 block of columns holds no obstacle (tflags, from the z
 // pass) are neither loaded nor walked: they hold no site.  xflags[z] gets bit
 // x / TX for every line (x, z) left with a site, for the x pass.
+template <typename T>
 __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, uint32_t* __restrict__ out,
                                               uint32_t* __restrict__ stk, const uint32_t* __restrict__ tflags,
                                               const uint32_t* __restrict__ colm,
@@ -325,10 +351,10 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
   LineStack st{ring, stk + ((uint64_t)z * dx + x) * dy, lane, 0, 0};
   // top, second and third of the stack (entries; positions and costs of the first two);
   // bst = bisector(second, top)
-  float ty = 0.f, tc = 0.f, sy = 0.f, sc = 0.f;
+  T ty = 0, tc = 0, sy = 0, sc = 0;
   uint32_t te = 0, se = 0, e3 = 0;
-  Bis bst{0.f, 1.f};
-  auto cost = [&](int32_t s) -> float { const float d = (float)(s - zi); return d * d; };
+  Bis<T> bst;
+  auto cost = [&](int32_t s) -> T { const T d = (T)(s - zi); return d * d; };
   // pop the top: second and third move up, the new third is fetched (when fewer
   // than two entries remain the moved values are never read)
   auto pop_y = [&]() {
@@ -337,7 +363,7 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
     tc = sc;
     te = se;
     se = e3;
-    sy = (float)(e3 & 0x3FFu);
+    sy = (T)(e3 & 0x3FFu);
     sc = cost((int32_t)(e3 >> 10));
     bst.set(sy, sc, ty, tc);
     e3 = st.at3(st.n >= 3 ? st.n - 3 : 0);
@@ -384,9 +410,9 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
       m &= m - 1u;
       const uint32_t rn = m ? (uint32_t)__builtin_ctz(m) : r;
       const int32_t sn = ztile[rn][lane];
-      const float y = (float)(y0 + r), c = cost(s);
+      const T y = (T)(y0 + r), c = cost(s);
       if (st.n >= 1) {
-        Bis btn;
+        Bis<T> btn;
         btn.set(ty, tc, y, c);
         while (st.n >= 2 && middle_empty(bst, btn)) {
           pop_y();
@@ -426,7 +452,7 @@ __global__ void __launch_bounds__(TB) k_pba_y(const uint16_t* __restrict__ zs, u
     return;
   }
   for (int32_t yy = (int32_t)dy - 1; yy >= 0; --yy) {
-    while (st.n >= 2 && bst.a_wins((float)yy)) {
+    while (st.n >= 2 && bst.a_wins((T)yy)) {
       pop_y();
     }
     __builtin_amdgcn_raw_buffer_store_b32(x | te << 10, orr, (int)(x * 4),
@@ -948,6 +974,7 @@ __global__ void __launch_bounds__(TB * XN_WAVES) k_pba_x_chunk(const uint32_t* _
 // contiguous row segments.
 // Tiles of TX positions whose y lines of this slice kept no site (xflags, from the
 // y pass) hold only uninitialised voxels: they are neither loaded nor walked.
+template <typename T>
 __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, const uint16_t* __restrict__ yr,
                                               const uint32_t* __restrict__ yfs, uint32_t* __restrict__ stk,
                                               uint32_t* __restrict__ cnt,
@@ -969,16 +996,16 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
   const uint32_t lane = threadIdx.x, y = y0 + lane;
   const bool active = y < dy;
   const int32_t yi = (int32_t)y, zi = (int32_t)z;
-  auto cost = [&](uint32_t e) -> float {
-    return (float)(sq24((int32_t)((e >> 10) & 0x3FFu) - yi) + sq24((int32_t)(e >> 20) - zi));
+  auto cost = [&](uint32_t e) -> T {
+    return (T)(sq24((int32_t)((e >> 10) & 0x3FFu) - yi) + sq24((int32_t)(e >> 20) - zi));
   };
   // loader mapping: pass k covers rows LPR k + lane / TX, column lane % TX
   const uint32_t lr = lane / TX, lc = lane % TX;
   const uint32_t ntiles = (dx + TX - 1) / TX;
   LineStack st{ring, stk + ((uint64_t)z * dy + (active ? y : 0)) * dx, lane, 0, 0};
-  float tx = 0.f, tc = 0.f, sx = 0.f, sc = 0.f;
+  T tx = 0, tc = 0, sx = 0, sc = 0;
   uint32_t te = 0, se = 0, e3 = 0;  // top, second, third entry of the stack
-  Bis bst{0.f, 1.f};
+  Bis<T> bst;
   uint32_t pre[NLD];
   const uint32_t* __restrict__ slice = map + (uint64_t)z * dy * dx;
   const uint16_t* __restrict__ rslice = yr + (uint64_t)z * dy * dx;
@@ -1038,9 +1065,9 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
         m &= m - 1u;
         const uint32_t lxn = m ? (uint32_t)__builtin_ctz(m) : lx;
         const uint32_t en = tile[lane][lxn];
-        const float x = (float)(x0 + lx), c = cost(e);
+        const T x = (T)(x0 + lx), c = cost(e);
         if (st.n >= 1) {
-          Bis btn;
+          Bis<T> btn;
           btn.set(tx, tc, x, c);
           while (st.n >= 2 && middle_empty(bst, btn)) {
             // pop the top: second and third move up, the new third is fetched
@@ -1049,7 +1076,7 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
             tc = sc;
             te = se;
             se = e3;
-            sx = (float)(e3 & 0x3FFu);
+            sx = (T)(e3 & 0x3FFu);
             sc = cost(e3);
             bst.set(sx, sc, tx, tc);
             e3 = st.at3(st.n >= 3 ? st.n - 3 : 0);
@@ -1077,8 +1104,9 @@ __global__ void __launch_bounds__(TB) k_pba_x(const uint32_t* __restrict__ map, 
   }
 }
 
-// floor(N / D) for D > 0 and |N| < 2^22: the float quotient is within 1 of N / D,
-// and one integer step corrects its floor
+// floor(N / D) for D > 0: a float quotient below 2^12 is within 1 of N / D (N and the
+// division round to 2^-24 of it), and one integer step corrects its floor.  Larger ones
+// (|N| up to 2^25) may be further off, but stay outside the line, which is all that counts.
 __device__ __forceinline__ int32_t floor_div(int32_t N, int32_t D)
 {
   int32_t q = (int32_t)floorf((float)N / (float)D);
@@ -1685,7 +1713,7 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
   uint32_t* ycut = yfmt + dz;  // slices with positions beyond the y window
   uint32_t* xfb = ycut + dz;   // x groups left to the stack kernels
   uint32_t* xcnt = xfb + xgroups;  // per x range: obstacles, empty cells (+ 16); smallest window radius (+ 32)
-  const bool chunks = pba_chunk_suits(m->dims);
+  const bool chunks = pba_chunk_suits(m->dims), floats = bis_floats(dx, dy, dz);
   const uint32_t nxr = (dx + TB - 1) / TB;
   const uint64_t cols = (uint64_t)dx * dy;
   const uint32_t u = m->uninit;
@@ -1732,8 +1760,9 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
     return pba_launched("k_pba_x_chunk");
   }
   auto y_stack = [&](bool redo) {
-    hipLaunchKernelGGL(k_pba_y, dim3((unsigned)ygroups), dim3(TB), 0, s, zs, yb, st, tflags, colm, xflags, yfs, dx, dy,
-                       dz, u, redo);
+    const auto k = floats ? k_pba_y<float> : k_pba_y<int32_t>;
+    hipLaunchKernelGGL(k, dim3((unsigned)ygroups), dim3(TB), 0, s, zs, yb, st, tflags, colm, xflags, yfs, dx, dy, dz, u,
+                       redo);
     return pba_launched("k_pba_y");
   };
   {
@@ -1760,8 +1789,8 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
 #undef XL
     GVX_CHECK(pba_launched("k_pba_x_win"));
     GVX_CHECK(y_stack(true));
-    hipLaunchKernelGGL(k_pba_x, dim3((unsigned)xgroups), dim3(TB), 0, s, yb, yr, yfs, st, cnt, xflags, xfb, dx, dy, dz,
-                       u);
+    const auto kx = floats ? k_pba_x<float> : k_pba_x<int32_t>;
+    hipLaunchKernelGGL(kx, dim3((unsigned)xgroups), dim3(TB), 0, s, yb, yr, yfs, st, cnt, xflags, xfb, dx, dy, dz, u);
     GVX_CHECK(pba_launched("k_pba_x"));
     const uint64_t clines = (uint64_t)XC_LINES * XC_LPW, units = (lines + clines - 1) / clines;
     const uint64_t cgrid = std::max<uint64_t>((units + 63) / 64, std::min<uint64_t>(units, 4096));

@@ -64,3 +64,40 @@ def test_uneven_fields(gvx_lib, what):
     else:
         occ &= (x + y + z > 60)
     _check(gvx_lib, d, occ.reshape(-1))
+
+
+# z axes above 1024: the z pass in two sweeps, every x range to the stack kernels; (8, 1024, 3960)
+# and (8, 1024, 3970) are the two sides of their number format (a diagonal of 2^24)
+@pytest.mark.parametrize("d", [(70, 40, 1026), (33, 20, 4094), (3, 1024, 1100), (130, 2, 2000), (8, 1024, 3960),
+                               (8, 1024, 3970)])
+def test_deep_maps(gvx_lib, d):
+    rng = np.random.default_rng(sum(d))
+    n = int(np.prod(d))
+    for k in (1, 4, n // 3000, n // 20):
+        occ = np.zeros(n, bool)
+        occ[rng.integers(0, n, k)] = True
+        _check(gvx_lib, d, occ)
+
+
+def test_deep_map_squared_distances_above_24_bits(gvx_lib):
+    # row (238, 4093): costs 16784681, 16784744, 16784681 at x = 0, 8, 16, so the site at x = 8 is
+    # voxel 8's nearest by one; rounded to 24 bits it owns no voxel
+    d = (17, 239, 4094)
+    occ = np.zeros(d[::-1], bool)
+    for x, y, z in ((0, 18, 2), (8, 0, 3), (16, 18, 2)):
+        occ[z, y, x] = True
+    _check(gvx_lib, d, occ.reshape(-1))
+
+
+def test_deepest_map(gvx_lib):
+    # the far corner's row: (49, 11, 19) is voxel 48's nearest by one, 17621621 against 17621622
+    d = (128, 1024, 4094)
+    sites = np.array([(3, 12, 19), (20, 16, 17), (49, 11, 19), (56, 12, 18), (93, 12, 19), (115, 11, 17)], np.int64)
+    g = gvx_lib.Map(O.DIST_MAP, d, 0.01)
+    g.insert_coords(sites.astype(np.uint32), gvx_lib.eBVM_OCCUPIED)
+    g.pba()
+    row = np.stack([np.arange(d[0]), np.full(d[0], d[1] - 1), np.full(d[0], d[2] - 1)], 1)
+    want = ((row[:, None] - sites[None]) ** 2).sum(-1).min(1)
+    idx = (row[:, 2] * d[1] + row[:, 1]) * d[0] + row[:, 0]
+    assert want[48] == 17621621
+    assert np.array_equal(g.squared_distances(idx.astype(np.uint32)), want)
