@@ -1631,7 +1631,7 @@ static uint64_t pba_flag_words(uint32_t dx, uint32_t dy, uint32_t dz)
   const uint64_t cwords = (uint64_t)((dy + 31) / 32) * ((dx + 63) / 64);
   const uint64_t xgroups = (uint64_t)((dy + TB - 1) / TB) * dz;
   const uint64_t ygroups = (uint64_t)((dx + TB - 1) / TB) * dz;
-  return 64 + 2 * (uint64_t)dz + cwords + dz + ygroups + dz + dz + xgroups + 64;
+  return 64 + 2 * (uint64_t)dz + cwords + dz + ygroups + dz + dz + xgroups + 64;  // the last 64: 2 + 33 used
 }
 
 static int pba_launch(MapS* m, const PbaBufs& sc, bool timed);
@@ -1704,7 +1704,8 @@ static int pba_launch(MapS* m, const PbaBufs& sc, bool timed)
   uint32_t* st = (uint32_t*)sc.node;
   uint32_t* tflags = (uint32_t*)sc.flags;
   unsigned long long* xflags = (unsigned long long*)((uint32_t*)sc.flags + 64);
-  uint32_t* colm = (uint32_t*)sc.flags + 64 + 2 * (uint64_t)dz;
+  // 16-byte aligned for fill_u32, also where dz is odd (pba_flag_words' last 64 words have room)
+  uint32_t* colm = (uint32_t*)sc.flags + 64 + 2 * ((uint64_t)dz + dz % 2);
   // y lines of the stack kernel: yfs[z] per slice (second run, see k_pba_y), then
   // yfs[dz + group] per 64-column group (ranges too sparse for the window), then per
   // slice the format of its y output (set by the first run for the x pass)

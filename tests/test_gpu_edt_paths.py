@@ -79,6 +79,11 @@ def test_deep_maps(gvx_lib, d):
         _check(gvx_lib, d, occ)
 
 
+@pytest.mark.parametrize("d", [(70, 40, 1025), (1, 33, 4093)])
+def test_deep_maps_of_odd_depth(gvx_lib, d):
+    test_deep_maps(gvx_lib, d)
+
+
 def test_deep_map_squared_distances_above_24_bits(gvx_lib):
     # row (238, 4093): costs 16784681, 16784744, 16784681 at x = 0, 8, 16, so the site at x = 8 is
     # voxel 8's nearest by one; rounded to 24 bits it owns no voxel
