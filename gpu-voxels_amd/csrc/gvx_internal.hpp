@@ -42,6 +42,7 @@ struct Runtime {
   void* host_small = nullptr;
   void* dev_small = nullptr;
   uint32_t flag_seq = 0;  // see OutsideFlag
+  bool results_open = false;  // results_dev without its results_fetch: the counters may not be zero
   bool profiling = false;
 };
 Runtime& rt();
@@ -75,12 +76,14 @@ int scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* total_dev)
 // Results that a call waits for.  Device counters (a 64-bit count, 8 mask words) are
 // zero between calls: results_fetch launches one wave that copies them to pinned host
 // memory and zeroes them again, then waits (a fill before the kernel and a copy after it
-// cost two more dependent launches: 19 us for a call on a tiny map, 16 us this way).
+// cost two more dependent launches: 19 us for a call on a tiny map, 16 us this way).  A call
+// that ends between the two (a pending error of another library is enough) leaves counts
+// behind; the next results_dev clears them.
 struct ResultDev {
   unsigned long long* count;
   uint32_t* mask;
 };
-ResultDev results_dev();
+int results_dev(ResultDev* out);
 void result_word(uint32_t** dev, uint32_t** host);  // one more word, written by a kernel to both
 int results_fetch(uint64_t* count, uint8_t* mask);  // mask (32 bytes) may be null
 

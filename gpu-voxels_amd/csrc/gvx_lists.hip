@@ -1273,7 +1273,8 @@ int gvx_list_collide_map(gvx_list self, gvx_map map, float threshold, const int3
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
   uint32_t tm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (typemask) memcpy(tm, typemask, 32);
-  const ResultDev res = results_dev();
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
   if (self->n) {
     ProfScope ps("list_collide_map");
     unsigned g = grid_for(self->n, 256, 8192);
@@ -1302,7 +1303,8 @@ int gvx_list_collide_list(gvx_list self, gvx_list other, uint64_t* count, uint8_
   std::unique_lock<std::recursive_mutex> g1(self->mu, std::defer_lock), g2(other->mu, std::defer_lock);
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
-  const ResultDev res = results_dev();
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
   if (self->n && other->n) {
     hipLaunchKernelGGL(k_list_collide_list, dim3(grid_for(self->n, 256, 8192)), dim3(256), 0, rt().stream, self->ids,
                        self->bits, self->n, other->ids, other->bits, other->n, res.count, res.mask);
@@ -1329,7 +1331,9 @@ int gvx_list_collide_bitcheck(gvx_list self, gvx_list other, uint32_t margin, ui
   std::unique_lock<std::recursive_mutex> g1(self->mu, std::defer_lock), g2(other->mu, std::defer_lock);
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
-  unsigned long long* dcount = results_dev().count;
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
+  unsigned long long* dcount = res.count;
   if (self->n && other->n) {
     hipLaunchKernelGGL(k_list_bitcheck, dim3(grid_for(self->n, 256, 8192)), dim3(256), 0, rt().stream, self->ids,
                        self->bits, self->n, other->ids, other->bits, other->n, margin, dcount);

@@ -1705,7 +1705,9 @@ int gvx_map_collide(gvx_map self, gvx_map other, float threshold, const int32_t 
     *count = 0;
     return GVX_OK;
   }
-  unsigned long long* dcount = results_dev().count;
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
+  unsigned long long* dcount = res.count;
   {
     hipStream_t s = rt().stream;
     uint8_t* a = (uint8_t*)self->data;
@@ -1742,7 +1744,8 @@ int gvx_map_collide_types(gvx_map self, gvx_map other, float threshold, uint64_t
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
   const int thr = sv_float_to_probability(threshold);
-  const ResultDev res = results_dev();
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
   {
     ProfScope ps("collide_types");
     if (other->type == TBIT)
@@ -1772,7 +1775,8 @@ int gvx_map_collide_sv(gvx_map self, gvx_map other, float threshold, uint32_t wi
   std::unique_lock<std::recursive_mutex> g1(self->mu, std::defer_lock), g2(other->mu, std::defer_lock);
   if (self == other) g1.lock(); else std::lock(g1, g2);
   std::lock_guard<std::recursive_mutex> g3(rt().mu);
-  const ResultDev res = results_dev();
+  ResultDev res;
+  GVX_CHECK(results_dev(&res));
   {
     ProfScope ps("collide_sv");
     hipLaunchKernelGGL(k_collide_sv, dim3(stream_grid(self->n)), dim3(256), 0, rt().stream, (uint8_t*)self->data,

@@ -188,7 +188,7 @@ int fill_bytes(void* dst, uint8_t value, uint64_t n_bytes)
 
 // ---------------------------------------------------------------- results of a call
 // dev_small: [0, 1024) free scratch of the entry points, [1024, 1088) result counters
-// (zero between calls), [1088, 1092) the outside flag's device word, [1092, 1096)
+// (zero between calls, unless results_open), [1088, 1092) the outside flag's device word, [1092, 1096)
 // result_word.  host_small: the same on the host.
 constexpr size_t RES_AT = 1024, FLAG_AT = 1088, WORD_AT = 1092;
 
@@ -199,10 +199,14 @@ __global__ void k_results(uint32_t* __restrict__ dev, uint32_t* __restrict__ hos
   dev[threadIdx.x] = 0u;
 }
 
-ResultDev results_dev()
+int results_dev(ResultDev* out)
 {
-  char* d = (char*)rt().dev_small + RES_AT;
-  return ResultDev{(unsigned long long*)d, (uint32_t*)(d + 8)};
+  Runtime& r = rt();
+  char* d = (char*)r.dev_small + RES_AT;
+  if (r.results_open) GVX_CHECK(fill_u32(d, 0u, 10));
+  r.results_open = true;
+  *out = ResultDev{(unsigned long long*)d, (uint32_t*)(d + 8)};
+  return GVX_OK;
 }
 
 int results_fetch(uint64_t* count, uint8_t* mask)
@@ -212,6 +216,7 @@ int results_fetch(uint64_t* count, uint8_t* mask)
                      (uint32_t*)h);
   GVX_HIP(hipGetLastError());
   GVX_CHECK(sync());
+  rt().results_open = false;
   memcpy(count, h, 8);
   if (mask) memcpy(mask, h + 8, 32);
   return GVX_OK;

@@ -78,3 +78,40 @@ def test_results_of_one_call_stay_out_of_the_next(gvx_lib):
         lst.insert_points(inside, 5)
         assert lst.collide_map(full, mode=1)[0] == 1
         assert lst.collide_map(empty, mode=1)[0] == 0
+
+
+def pending_error(gvx):
+    """An error of another user of the HIP runtime: no call of this library, left to be collected."""
+    assert gvx.lib().hipSetDevice(1 << 20) != 0
+
+
+def test_results_after_a_call_that_ended_early(gvx_lib):
+    # a pending error ends a collision between its kernel and the read of its counters: what it
+    # counted must not show up in the next call's result
+    gvx = gvx_lib
+    d = (24, 20, 9)
+    n = int(np.prod(d))
+    _, _, a, b = _pair(gvx, d, O.BITVECTOR_MAP, O.BITVECTOR_MAP, 0.5, 1)
+    _, _, _, p = _pair(gvx, d, O.BITVECTOR_MAP, O.PROB_MAP, 0.5, 2)
+    empty = gvx.Map(O.BITVECTOR_MAP, d, 0.01)
+    la, lb, none = (gvx.VoxelList(d, 0.01) for _ in range(3))
+    xyz = np.stack(np.unravel_index(np.arange(0, n, 3), d), 1).astype(np.uint32)
+    la.insert_coords(xyz, 7)
+    lb.insert_coords(xyz, 9)
+    for early in (lambda: a.collide(b), lambda: a.collide(p, 0.3), lambda: a.collide_types(b),
+                  lambda: a.collide_types(p, 0.3), lambda: a.collide_sv(b, window=3),
+                  lambda: la.collide_map(a, mode=1), lambda: la.collide_list(lb), lambda: la.collide_bitcheck(la)):
+        for after in (lambda: empty.collide(b), lambda: empty.collide_types(b)[0], lambda: none.collide_map(a)[0],
+                      lambda: la.collide_list(none)[0]):
+            pending_error(gvx)
+            try:
+                early()
+            except gvx.GvxError:
+                pass
+            assert after() == 0
+        pending_error(gvx)
+        try:
+            early()
+        except gvx.GvxError:
+            pass
+        assert not empty.collide_types(b)[1].any()
