@@ -609,6 +609,7 @@ struct LuBuffers {
   unsigned long long *bm = nullptr, *wcopy = nullptr;
   uint32_t *wpre = nullptr, *sums = nullptr, *offs = nullptr;
 };
+static bool lu_open = false;  // a call that marked and did not reach its end: the bitmap may hold its ids
 static int lu_buffers(uint64_t map_words, LuBuffers* out)
 {
   static LuBuffers b;
@@ -626,7 +627,10 @@ static int lu_buffers(uint64_t map_words, LuBuffers* out)
     GVX_CHECK(dalloc((void**)&b.offs, tiles * 4));
     GVX_CHECK(fill_u32(b.bm, 0u, words * 2));
     cap = words;
+  } else if (lu_open) {
+    GVX_CHECK(fill_u32(b.bm, 0u, cap * 2));
   }
+  lu_open = true;
   *out = b;
   return GVX_OK;
 }
@@ -680,6 +684,7 @@ static int lu_unique(ListS* L, LuSource& src)
                        L->ids, L->coords, L->bits);
   GVX_HIP(hipGetLastError());
   GVX_CHECK(sync());
+  lu_open = false;
   L->n = *static_cast<volatile uint32_t*>(count_host);
   return GVX_OK;
 }

@@ -259,3 +259,27 @@ def test_bitmap_unique_edges(gvx_lib, d, clouds):
         assert np.array_equal(got_ids, np.array(sorted(want), np.uint32))
         assert np.array_equal(got_coords @ np.array([1, d[0], d[0] * d[1]]), got_ids)
         assert [int.from_bytes(b.tobytes(), "little") for b in got_bits] == [want[k] for k in sorted(want)]
+
+
+def test_insert_after_a_call_that_ended_early(gvx_lib):
+    """A pending error of another user of the HIP runtime ends an insert after it has marked its voxels:
+    the next list holds its own only."""
+    gvx = gvx_lib
+    d = (61, 40, 33)
+    rng = np.random.default_rng(3)
+    for clouds in (1, 20):
+        for first, second in ((5000, 10), (10, 5000)):
+            a, b = gvx.VoxelList(d, 0.01), gvx.VoxelList(d, 0.01)
+            xyz = [rng.integers(0, d, (n, 3)).astype(np.uint32) for n in (first, second)]
+            pts = [((c + 0.5) * 0.01).astype(np.float32) for c in xyz]
+            size = np.full(clouds, first // clouds, np.uint32)
+            size[0] += first - size.sum()
+            assert gvx.lib().hipSetDevice(1 << 20) != 0  # left to be collected
+            try:
+                a.insert_points(pts[0], sizes=size, meanings=np.full(clouds, 9, np.uint32))
+            except gvx.GvxError:
+                pass
+            b.insert_points(pts[1], meaning=8)
+            ids, _, bits = b.read()
+            assert np.array_equal(ids, np.unique(xyz[1] @ np.array([1, d[0], d[0] * d[1]])))
+            assert (bits[:, 1] == 1).all() and not bits[:, [0] + list(range(2, 32))].any()
