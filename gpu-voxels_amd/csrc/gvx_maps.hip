@@ -1224,7 +1224,9 @@ __global__ void __launch_bounds__(256) k_shift_sv(uint8_t* __restrict__ v, uint6
 }
 
 // per-voxel words of insertSensorData (tags, then ray counters): allocated zeroed once
-// per size and left zeroed by every scan
+// per size and left zeroed by every scan, as are the bricks' counts below.  Open: taken by
+// a scan that did not reach its end, and cleared before the next use.
+static bool sensor_hits_open = false, sensor_bricks_open = false;
 static int sensor_hits_buffer(uint64_t n, uint32_t** out)
 {
   static uint32_t* buf = nullptr;
@@ -1237,7 +1239,10 @@ static int sensor_hits_buffer(uint64_t n, uint32_t** out)
     GVX_CHECK(dalloc((void**)&buf, ((n + 3) / 4) * 16));
     GVX_CHECK(fill_u32(buf, 0u, ((n + 3) / 4) * 4));
     cap = n;
+  } else if (sensor_hits_open) {
+    GVX_CHECK(fill_u32(buf, 0u, ((cap + 3) / 4) * 4));
   }
+  sensor_hits_open = true;
   *out = buf;
   return GVX_OK;
 }
@@ -1296,7 +1301,10 @@ static int sensor_bricks_buffers(uint64_t nb, uint64_t pairs, SensorBricks* out)
     GVX_CHECK(fill_u32(b.cnt, 0u, nb));
     cap_b = nb;
     cap_p = pairs;
+  } else if (sensor_bricks_open) {
+    GVX_CHECK(fill_u32(b.cnt, 0u, cap_b));
   }
+  sensor_bricks_open = true;
   *out = b;
   return GVX_OK;
 }
@@ -1595,7 +1603,10 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
                        P.weight, P.st);
     GVX_HIP(hipGetLastError());
   }
-  return sync();
+  GVX_CHECK(sync());
+  sensor_hits_open = false;
+  if (enable_raycasting && bricks) sensor_bricks_open = false;
+  return GVX_OK;
 }
 
 int gvx_map_insert_coords(gvx_map m, const uint32_t* xyz, uint64_t n, uint32_t meaning, int mem, int* points_outside)

@@ -131,3 +131,26 @@ def test_sensor_long_rays(gvx_lib, dims):
         o = O.new_map(O.PROB_MAP, dims)
         O.prob_insert_sensor(o, dims, side, sensor, pts)
         assert np.array_equal(g.read(), o)
+
+
+def test_scan_after_a_scan_that_ended_early(gvx_lib):
+    """A pending error of another user of the HIP runtime ends a scan after it has tagged its target
+    voxels: the next scan's tags, rays and counts are its own."""
+    gvx = gvx_lib
+    rng = np.random.default_rng(12)
+    dims, side = (61, 47, 33), 0.02
+    sensor = np.array([0.6, 0.5, 0.3], np.float32)
+    pts = _scan(rng, 6000, dims, side, sensor)
+    for early, ray in ((True, True), (True, False), (False, True)):
+        g = gvx.Map(gvx.PROBAB_VOXELMAP, dims, side)
+        assert gvx.lib().hipSetDevice(1 << 20) != 0  # left to be collected
+        try:
+            g.insert_sensor_data(pts, sensor, raycast=early)
+        except gvx.GvxError:
+            g.clear()
+        for few in (pts[:700], pts):
+            g = gvx.Map(gvx.PROBAB_VOXELMAP, dims, side)
+            o = O.new_map(O.PROB_MAP, dims)
+            g.insert_sensor_data(few, sensor, raycast=ray)
+            O.prob_insert_sensor(o, dims, side, sensor, few, raycast=ray)
+            assert np.array_equal(g.read(), o)
