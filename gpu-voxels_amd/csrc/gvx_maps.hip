@@ -1054,9 +1054,9 @@ __global__ void __launch_bounds__(1024) k_sensor_split(const SensorGeom g, const
 }
 
 // pass 1 without bricks, for maps with an edge above SB_EDGE and for scans whose pairs
-// would pass SB_PAIR_BYTES: one lane per distinct target voxel walks the line from the
-// sensor voxel to the target and adds the target's weight to the 32-bit counter of every cell it visits
-// (atomics without a return value: the walk never waits).  Rays of neighbouring
+// would pass SB_PAIR_BYTES or find no memory: one lane per distinct target voxel walks the
+// line from the sensor voxel to the target and adds the target's weight to the 32-bit
+// counter of every cell it visits (atomics without a return value: the walk never waits).  Rays of neighbouring
 // targets (consecutive lanes) share many cells, so at every step each run of
 // consecutive lanes on one cell adds its summed weight once (a 640 x 480 depth
 // image into a 512^3 map: 21.4 M atomics for 50.7 M cells walked).
@@ -1274,8 +1274,9 @@ static int sensor_points(uint64_t n, SensorPoints* out)
   return GVX_OK;
 }
 
-// bricks and pairs of one scan: n rays enter at most nb_edges bricks each (the sum of the
-// brick counts along the axes); counts are zero between scans
+// bricks and pairs of one scan: n rays enter at most bx + by + bz bricks each (236 MB for a
+// 640 x 480 frame in 512^3); counts are zero between scans.  Without the memory for them
+// (GVX_ERR_OOM) nothing is kept, and the scan goes without bricks.
 constexpr uint64_t SB_PAIR_BYTES = 2ull << 30;
 struct SensorBricks {
   uint32_t *cnt = nullptr, *cursor = nullptr, *split = nullptr;
@@ -1288,16 +1289,29 @@ static int sensor_bricks_buffers(uint64_t nb, uint64_t pairs, SensorBricks* out)
   static uint64_t cap_b = 0, cap_p = 0;
   if (cap_b < nb || cap_p < pairs) {
     GVX_CHECK(sync());
-    dfree(b.cnt); dfree(b.cursor); dfree(b.split); dfree(b.chunks); dfree(b.pairs);
-    b = SensorBricks();
+    const auto drop = [] {
+      dfree(b.cnt); dfree(b.cursor); dfree(b.split); dfree(b.chunks); dfree(b.pairs);
+      b = SensorBricks();
+      cap_b = cap_p = 0;
+    };
+    const uint64_t need_b = nb, need_p = pairs;
     nb = std::max(nb, cap_b);
     pairs = std::max(pairs, cap_p);
-    cap_b = cap_p = 0;
-    GVX_CHECK(dalloc((void**)&b.cnt, nb * 4));
-    GVX_CHECK(dalloc((void**)&b.cursor, nb * 4));
-    GVX_CHECK(dalloc((void**)&b.split, nb * 4));
-    GVX_CHECK(dalloc((void**)&b.chunks, (nb + pairs / SB_CHUNK + 1) * 16));
-    GVX_CHECK(dalloc((void**)&b.pairs, pairs * 8));
+    int s;
+    for (;;) {
+      drop();
+      if ((s = dalloc((void**)&b.cnt, nb * 4)) == GVX_OK && (s = dalloc((void**)&b.cursor, nb * 4)) == GVX_OK &&
+          (s = dalloc((void**)&b.split, nb * 4)) == GVX_OK &&
+          (s = dalloc((void**)&b.chunks, (nb + pairs / SB_CHUNK + 1) * 16)) == GVX_OK &&
+          (s = dalloc((void**)&b.pairs, pairs * 8)) == GVX_OK)
+        break;
+      if (nb == need_b && pairs == need_p) {
+        drop();
+        return s;
+      }
+      nb = need_b;  // not the room of earlier scans too
+      pairs = need_p;
+    }
     GVX_CHECK(fill_u32(b.cnt, 0u, nb));
     cap_b = nb;
     cap_p = pairs;
@@ -1554,9 +1568,13 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
   const uint32_t dx = m->dims[0], dy = m->dims[1], dz = m->dims[2];
   const uint32_t bx = (dx + SB - 1) / SB, by = (dy + SB - 1) / SB, bz = (dz + SB - 1) / SB;
   const uint64_t nb = (uint64_t)bx * by * bz, pairs = n * (uint64_t)(bx + by + bz);
-  const bool bricks = std::max(dx, std::max(dy, dz)) <= SB_EDGE && pairs * 8 <= SB_PAIR_BYTES;
+  bool bricks = enable_raycasting && std::max(dx, std::max(dy, dz)) <= SB_EDGE && pairs * 8 <= SB_PAIR_BYTES;
   SensorBricks B;
-  if (enable_raycasting && bricks) GVX_CHECK(sensor_bricks_buffers(nb, pairs, &B));
+  if (bricks) {
+    const int e = sensor_bricks_buffers(nb, pairs, &B);
+    if (e != GVX_OK && e != GVX_ERR_OOM) return e;
+    bricks = e == GVX_OK;
+  }
   const SensorGeom geom = {{sx, sy, sz}, udiv(dx), udiv(dy), bx, by};
   const unsigned gp = grid_for(n, 256, 1u << 14);
   {
@@ -1569,10 +1587,10 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
                        side, sin, pts, n, robot, robot_meaning, P.st, P.pos, P.list, P.weight);
     hipLaunchKernelGGL(k_sensor_weigh, dim3(gp), dim3(256), 0, s, hits, dx, dy, dz, side, sin, pts, n, robot,
                        robot_meaning, P.pos, P.weight);
-    if (!(enable_raycasting && bricks)) hipLaunchKernelGGL(k_sensor_untag, dim3(gp), dim3(256), 0, s, hits, P.list, P.st);
+    if (!bricks) hipLaunchKernelGGL(k_sensor_untag, dim3(gp), dim3(256), 0, s, hits, P.list, P.st);
     GVX_HIP(hipGetLastError());
   }
-  if (enable_raycasting && bricks) {
+  if (bricks) {
     ProfScope ps("sensor_rays");
     const unsigned gr = (unsigned)((n + SR_RAYS - 1) / SR_RAYS);
     hipLaunchKernelGGL(k_sensor_count, dim3(gr), dim3(SR_THREADS), 0, s, geom, P.st, P.list, hits, B.cnt);
@@ -1605,7 +1623,7 @@ int gvx_map_insert_sensor(gvx_map m, const float* xyz, uint64_t n, const float s
   }
   GVX_CHECK(sync());
   sensor_hits_open = false;
-  if (enable_raycasting && bricks) sensor_bricks_open = false;
+  if (bricks) sensor_bricks_open = false;
   return GVX_OK;
 }
 

@@ -154,3 +154,42 @@ def test_scan_after_a_scan_that_ended_early(gvx_lib):
             g.insert_sensor_data(few, sensor, raycast=ray)
             O.prob_insert_sensor(o, dims, side, sensor, few, raycast=ray)
             assert np.array_equal(g.read(), o)
+
+
+def test_scan_without_memory_for_bricks(gvx_lib):
+    """A scan that finds no memory for its (ray, brick) pairs (768 MB here) goes without them."""
+    import ctypes
+    gvx, hip = gvx_lib, gvx_lib.lib()
+    dims, side = (256, 256, 256), 0.01
+    rng = np.random.default_rng(5)
+    pts = rng.uniform(0, 2.56, (2000000, 3)).astype(np.float32)
+    sensor = np.array([1.3, 0.1, 1.2], np.float32)
+    full, want = gvx.Map(gvx.PROBAB_VOXELMAP, dims, side), gvx.Map(gvx.PROBAB_VOXELMAP, dims, side)
+    full.insert_sensor_data(pts, sensor, raycast=False)  # the points' own arrays are there before
+    full.clear()
+    held = []
+
+    def free():
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    try:
+        block = 16 << 30
+        while block >= 32 << 20:
+            p = ctypes.c_void_p()
+            if free() < block + (160 << 20):
+                block >>= 1
+            elif hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(block)) == 0:
+                held.append(p)
+            else:
+                hip.hipGetLastError()
+                block >>= 1
+        assert free() < 300 << 20
+        full.insert_sensor_data(pts, sensor)
+    finally:
+        for p in held:
+            hip.hipFree(p)
+    want.insert_sensor_data(pts, sensor)
+    got = full.read()
+    assert np.array_equal(got, want.read()) and int((got == -127).sum()) > 10000
