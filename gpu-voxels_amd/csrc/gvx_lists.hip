@@ -1007,6 +1007,8 @@ static int list_insert(ListS* l, const float* dp, uint64_t n, const uint32_t* en
   return make_unique(l);
 }
 
+std::recursive_mutex& list_mutex(void* lv) { return static_cast<ListS*>(static_cast<gvx_list_s*>(lv))->mu; }
+
 int list_insert_device(void* lv, const float* dp, uint64_t n, const uint32_t* ends, uint32_t ncl,
                        const uint32_t* meanings, uint32_t meaning)
 {

@@ -7,6 +7,7 @@
 
 namespace gvx {
 
+std::recursive_mutex& list_mutex(void* list);
 int list_insert_device(void* list, const float* pts_dev, uint64_t n, const uint32_t* ends_dev, uint32_t ncl,
                        const uint32_t* meanings_dev, uint32_t meaning);
 
@@ -258,6 +259,7 @@ int gvx_list_insert_robot(gvx_list list, const float* link_pts, const uint32_t* 
   GVX_CHECK(ensure_init());
   if (!list) return fail(GVX_ERR_BAD_ARG, "null list");
   if (n_links == 0 || !link_sizes || !dh || !q) return fail(GVX_ERR_BAD_ARG, "null argument");
+  std::lock_guard<std::recursive_mutex> g(list_mutex(list));  // an object's lock before the runtime's, as everywhere
   std::lock_guard<std::recursive_mutex> g2(rt().mu);
   RobotStage S;
   uint64_t n = 0;

@@ -283,3 +283,43 @@ def test_insert_after_a_call_that_ended_early(gvx_lib):
             ids, _, bits = b.read()
             assert np.array_equal(ids, np.unique(xyz[1] @ np.array([1, d[0], d[0] * d[1]])))
             assert (bits[:, 1] == 1).all() and not bits[:, [0] + list(range(2, 32))].any()
+
+
+def test_two_threads_on_one_list(gvx_lib):
+    """insert_points and list_insert_robot on one list from two threads take their locks in one order."""
+    import threading
+    gvx = gvx_lib
+    rng = np.random.default_rng(8)
+    d, side = (64, 64, 64), 0.02
+    pts = rng.uniform(0, 1.2, (500, 3)).astype(np.float32)
+    links = rng.uniform(-0.1, 0.1, (300, 3)).astype(np.float32)
+    sizes = np.array([100, 200], np.uint32)
+    dh = np.array([[0, 0.1, 0.2, 1.5707964, 0], [0, 0.15, 0.1, 0, 0]], np.float32)
+    base = np.array([1, 0, 0, 0.6, 0, 1, 0, 0.6, 0, 0, 1, 0.6], np.float32)
+    qs = rng.uniform(-3, 3, (200, 2)).astype(np.float32)
+    lst, want = gvx.VoxelList(d, side), gvx.VoxelList(d, side)
+    errors = []
+
+    def run(f):
+        try:
+            f()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    def points(to):
+        for k in range(200):
+            to.insert_points(pts[: 100 + 2 * k], meaning=5)
+
+    def robot(to):
+        for q in qs:
+            gvx.list_insert_robot(to, links, sizes, dh, q, base, meaning=6)
+
+    threads = [threading.Thread(target=run, args=(lambda f=f: f(lst),), daemon=True) for f in (points, robot)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not any(t.is_alive() for t in threads) and not errors
+    points(want)
+    robot(want)
+    assert all(np.array_equal(a, b) for a, b in zip(lst.read(), want.read()))
