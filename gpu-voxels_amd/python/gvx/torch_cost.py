@@ -16,10 +16,11 @@ def _sync():
 
 class ClearanceCostFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, cost):
+    def forward(ctx, q, cost, taped=True):
         q = q.detach().contiguous().float()
         out = torch.empty(q.shape[0], device=q.device, dtype=torch.float32)
-        if not ctx.needs_input_grad[0]:
+        # needs_input_grad does not know of torch.no_grad(): taped does
+        if not (taped and ctx.needs_input_grad[0]):
             _sync()
             return cost.forward(q, out)
         dq = torch.empty_like(q)
@@ -32,9 +33,9 @@ class ClearanceCostFn(torch.autograd.Function):
     def backward(ctx, grad_out):
         _, dq = ctx.saved_tensors
         # zero without contact, also where grad_out is infinite (the root of a cost of zero)
-        return torch.where(dq == 0, dq, dq * grad_out.detach().float()[:, None, None]), None
+        return torch.where(dq == 0, dq, dq * grad_out.detach().float()[:, None, None]), None, None
 
 
 def clearance_cost(q, cost: Cost):
     """q: (T, W, L) float32 CUDA tensor of joint values -> (T,) cost per trajectory."""
-    return ClearanceCostFn.apply(q, cost)
+    return ClearanceCostFn.apply(q, cost, torch.is_grad_enabled())
