@@ -379,10 +379,15 @@ static int cost_run(CostS* c, const float* q, uint32_t ntraj, uint32_t nwp, floa
                     float* dxo)
 {
   const uint64_t n = (uint64_t)ntraj * nwp;
-  if (n == 0) return GVX_OK;
   if (n > 0x7FFFFFFFull) return fail(GVX_ERR_BAD_ARG, "too many (trajectory, waypoint) pairs");
   std::lock_guard<std::recursive_mutex> g(c->mu);
   std::lock_guard<std::recursive_mutex> g2(rt().mu);
+  if (n == 0) {  // a trajectory without waypoints costs nothing
+    if (!out || ntraj == 0) return GVX_OK;
+    hipLaunchKernelGGL(k_cost_sum, dim3((ntraj + 3) / 4), dim3(256), 0, rt().stream, c->partial, ntraj, nwp, out);
+    GVX_HIP(hipGetLastError());
+    return sync();
+  }
   if (out) GVX_CHECK(cost_reserve(c, n));
   float* partial = out ? c->partial : nullptr;
   hipStream_t s = rt().stream;

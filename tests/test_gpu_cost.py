@@ -410,3 +410,21 @@ def test_cost_infinite_upstream(gvx_lib):
     cost.backward(q, dq, dx, inf)        # link 1 of trajectory 0 hangs in the field: dc/dq_0 != 0
     assert torch.isinf(dq[0, :, 0]).all() and torch.isfinite(dq[2]).all() and (dq[2, :, 0] != 0).all()
     assert torch.isinf(dx[0, :, 1, :, 2]).all() and torch.equal(dq[1], torch.zeros_like(dq[1]))
+
+
+def test_cost_of_trajectories_without_waypoints(gvx_lib):
+    """No waypoints: costs of zero, written by every entry point that writes costs."""
+    import torch
+    gvx = gvx_lib
+    grid = torch.ones(8 ** 3, device="cuda")
+    cost = gvx.Cost(grid, (8, 8, 8), 0.1, np.zeros((2, 5), np.float32), np.zeros((2, 3, 4), np.float32), 5.0)
+    q, dq = torch.zeros(16, device="cuda"), torch.full((16,), 7.0, device="cuda")
+    for n in (1, 5, 300):
+        for both in (False, True):
+            out = torch.full((n + 1,), 7.0, device="cuda")
+            torch.cuda.synchronize()
+            args = (cost.h, gvx._p(q), n, 0, gvx._p(out))
+            gvx.check(gvx.lib().gvx_cost_forward_grad(*args, gvx._p(dq)) if both else gvx.lib().gvx_cost_forward(*args))
+            assert not out[:n].any() and out[n] == 7.0 and (dq == 7.0).all()
+    gvx.check(gvx.lib().gvx_cost_backward(cost.h, gvx._p(q), 5, 0, None, gvx._p(dq), None))
+    assert (dq == 7.0).all()
