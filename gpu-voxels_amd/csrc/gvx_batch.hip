@@ -79,7 +79,8 @@ struct BatchS {
   uint64_t* bcell = nullptr;    // per brick: a bit per 2x2x2-voxel cell that holds an occupied voxel
   uint32_t* wrank = nullptr;    // per brick word: rank of its first occupied voxel (bprefix + earlier words)
   uint32_t* bsat = nullptr;     // summed-area table of occupied bricks, (bxn+1) x (byn+1) x (bzn+1)
-  uint32_t n_occ = 0;
+  uint32_t n_occ = 0;          // occupied voxels and
+  uint32_t n_occ_bricks = 0;   // bricks that hold one
   // robot
   uint32_t n_links = 0;
   uint64_t n_pts = 0;
@@ -693,11 +694,11 @@ struct PoseArgs {
 // poses before: 64 poses of 40k points from host memory 66 -> 33 us, the 1024 poses 103 ->
 // 90, an environment with a tenth of all voxels occupied 1274 -> 514 (96 poses 375 -> 122); the
 // first call on new buffers 286 -> 86.  Four chunks at a time with 1024 threads, a block per
-// CU; three with 512, three blocks in 80 registers (1024 poses of 150k points 83 us, with four
-// and two blocks 88).  Tried: a bit per occupied voxel in LDS, a line per occupied brick
-// instead of the whole bitmap (both the same), a second box test against single voxels
-// (10 % fewer chunks, no faster), two chunks at a time in 64 registers (a tenth slower, they
-// spill).
+// CU; three with 512, three blocks in 80 registers (1024 poses of 150k points with 512 threads
+// 83 us, with four and two blocks 88).  Tried: a bit per occupied voxel in LDS, a line per
+// occupied brick instead of the whole bitmap (both the same), a second box test against
+// single voxels (10 % fewer chunks, no faster), two chunks at a time in 64 registers (a tenth
+// slower, they spill).
 constexpr uint32_t PB_RUNS = 64;    // runs per round of broad and narrow phase
 constexpr uint32_t PB_HASH = 4096;  // slots
 constexpr uint32_t PB_PROBES = 16;
@@ -1005,9 +1006,13 @@ static int batch_rebuild_env(BatchS* b)
   hipLaunchKernelGGL(k_word_rank, dim3((unsigned)((b->nbricks + 255) / 256)), dim3(256), 0, s, b->bricks, b->bprefix,
                      b->nbricks, b->wrank, b->bcell);
   GVX_HIP(hipGetLastError());
-  GVX_HIP(hipMemcpyAsync(rt().host_small, b->bprefix + b->nbricks, 4, hipMemcpyDeviceToHost, s));
+  uint32_t* host = (uint32_t*)rt().host_small;
+  const uint64_t sat_last = (uint64_t)(b->bxn + 1) * (b->byn + 1) * (b->bzn + 1) - 1;
+  GVX_HIP(hipMemcpyAsync(host, b->bprefix + b->nbricks, 4, hipMemcpyDeviceToHost, s));
+  GVX_HIP(hipMemcpyAsync(host + 1, b->bsat + sat_last, 4, hipMemcpyDeviceToHost, s));
   GVX_CHECK(sync());
-  b->n_occ = *(uint32_t*)rt().host_small;
+  b->n_occ = host[0];
+  b->n_occ_bricks = host[1];
   const uint64_t words = (b->max_poses + 31) / 32;
   const uint64_t need = (uint64_t)(b->n_occ ? b->n_occ : 1) * words;
   // captured graphs hold the hit-matrix size of the previous environment
@@ -1102,20 +1107,38 @@ static bool pose_blocks_suit(const BatchS* b)
 
 // The kernel a schedule takes for n poses.  Schedule 0 takes a block per pose unless the poses
 // are few for their points: one CU then walks what 128-point chunks spread over the chip.
-// Call times, device memory, pose blocks against 128-point chunks, links of 150k points in
-// 512^3: 4 poses 34 / 26 us, 16: 39 / 37, 64: 38 / 43, 256: 45 / 63, 1024: 83 / 106;
-// 60k points in 256^3: 4: 28 / 26, 16: 31 / 34, 64: 30 / 43, 1024: 58 / 135; 20k points: 4: 23 / 23,
-// 64: 23 / 33, 1024: 39 / 89.  A pose takes 1024 threads while a CU has at most three poses
-// (150k points, 64 poses: 38 us, with 512 47; 512 poses 62 and 65), and 512 beyond, where
-// three blocks share a CU (1024 poses of 40k points in eight scenes: 44 to 61 us with 1024, 35
-// to 52 with 512) -- but not for many points, whose longest pose then lasts longest (150k
-// points: 61 to 107 us with 1024, 55 to 112 with 512).
-static int kernel_schedule(const BatchS* b, uint32_t n, int ks)
+// Call times, pose blocks against 128-point chunks, links of 150k points in a 512^3 room: 4
+// poses 34 / 26 us, 16: 39 / 37, 64: 38 / 43, 256: 45 / 63; 60k points in 256^3: 4: 28 / 26,
+// 16: 31 / 34, 64: 30 / 43, 1024: 58 / 135; 20k points: 4: 23 / 23, 64: 23 / 33, 1024: 39 / 89.
+//
+// A pose takes 1024 threads while a CU has at most three poses (150k points, 64 poses: 38 us,
+// with 512 47; 512 poses 62 and 65), and 512 beyond, where three blocks share a CU (1024 poses
+// of 40k points in eight scenes: 44 to 61 us with 1024, 35 to 52 with 512).
+//
+// Robots of more than 2^17 points, back-to-back calls on 512^3 maps in us (chunks, 512
+// threads, 1024 threads):
+//   rooms                  1024 poses, 8 scenes  45-185  41-98   49-93    2048, 3 scenes  127-288  108-130  126-168
+//   the slowest such room  1024 poses  75 98 72,  1280  87 98 94,  1536  101 105 120
+//   one depth image, six   300 poses   15-32  17-32  13-25                800   19-50   17-34   20-37
+//                          1024        21-64  17-40  23-50                4096  48-188  38-90   71-142
+//   the benchmark's (one of the six)  512 poses 20 30 28, 800: 23 30 28, 1024: 27 30 34
+// A few long poses decide 512 against 1024 threads in the rooms until there are more than four
+// poses per CU.  A depth image leaves few bricks occupied (below 1.4 % of them; rooms above
+// 3.3 %) and poses short (3 to 73 chunks of 64 points; rooms 80 to 320): between one and 3.5
+// poses per CU chunks are as fast as either on average, and the steadier ones.
+// At 2^17 points the rooms' longest poses no longer tell (128k points, four scenes: 39-86
+// with 512 threads, 49-74 with 1024, chunks 44-76).
+// pinned: joint values and results in pinned host memory, which only pose blocks use: chunks
+// take three copies (the benchmark's image, 512 poses from host memory: 59 us, pose blocks 45).
+static int kernel_schedule(const BatchS* b, uint32_t n, int ks, bool pinned)
 {
   const uint32_t cus = (uint32_t)(rt().num_cus > 0 ? rt().num_cus : 256);
   if (ks == 0 && b->n_pts > 4096ull * n) return 1;
   if (kSchedules[ks].chunk == 0 && !pose_blocks_suit(b)) return 1;
-  return ks == 0 ? (n > 3 * cus && b->n_pts <= 1u << 17 ? 6 : 7) : ks;
+  if (ks != 0) return ks;
+  if (b->n_pts <= 1u << 17) return n > 3 * cus ? 6 : 7;
+  if (64ull * b->n_occ_bricks < b->nbricks) return 2ull * n > 7ull * cus ? 6 : n > cus && !pinned ? 1 : 7;
+  return n > 4 * cus ? 6 : 7;
 }
 
 // chunks of `block` consecutive points of one link (the last one of a link may be
@@ -1230,7 +1253,7 @@ static int batch_enqueue(BatchS* b, uint32_t n, int sched, const float* q, uint3
 static int batch_run(BatchS* b, uint32_t n, int sched, const float* q, uint32_t* counts, uint32_t* masks)
 {
   hipStream_t s = rt().stream;
-  const int ks = kernel_schedule(b, n, sched % kKernelSchedules);
+  const int ks = kernel_schedule(b, n, sched % kKernelSchedules, b->io && q == reinterpret_cast<const float*>(b->io));
   const ChunkTab* ct = nullptr;
   if (kSchedules[ks].chunk) GVX_CHECK(chunk_table(b, kSchedules[ks].chunk, &ct));  // built before any capture
   if (ct) {
@@ -1455,7 +1478,7 @@ static int batch_collide_impl(gvx_batch b, const float* q, uint32_t n, int mem, 
     return sync();
   }
   if (b->io && mem == GVX_MEM_HOST && out_mem == GVX_MEM_HOST &&
-      kSchedules[kernel_schedule(b, n, sched % kKernelSchedules)].chunk == 0) {
+      kSchedules[kernel_schedule(b, n, sched % kKernelSchedules, true)].chunk == 0) {
     // a pose block reads its joint values once and writes 36 bytes: over the bus, instead of
     // three copies (64 poses of 40k points: 59 -> 33 us)
     uint32_t *io_masks = b->io + (uint64_t)b->max_poses * b->n_links, *io_counts = io_masks + (uint64_t)b->max_poses * 8;

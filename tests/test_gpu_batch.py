@@ -329,3 +329,40 @@ def test_batch_pose_blocks(gvx_lib, case):
     assert 0 <= b.autotune(n) < 16
     c, m = b.collide(q[:7])
     assert np.array_equal(c, oc[:7]) and np.array_equal(m, om[:7])
+
+
+@pytest.mark.parametrize("sparse", [True, False])
+def test_default_schedule_of_many_points(gvx_lib, sparse):
+    """Above 2^17 points schedule 0 chooses by poses per CU and by how many bricks are occupied: its
+    results are the chunk kernels' on both sides of every line, from device and host memory."""
+    import torch
+    gvx = gvx_lib
+    rng = np.random.default_rng(31)
+    d, side = (128, 128, 128), 0.02
+    env = gvx.Map(O.BITVECTOR_MAP, d, side)
+    spots = rng.uniform(0.4, 2.1, (30 if sparse else 3000, 3)).astype(np.float32)  # of 4096 bricks
+    env.insert_points(spots, 1)
+    sizes = np.array([30001, 1, 60000, 44999], np.uint32)
+    dh, pts = _robot(rng, 4, sizes)
+    base = np.array([1, 0, 0, 1.2, 0, 1, 0, 1.2, 0, 0, 1, 1.0], np.float32)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    q = rng.uniform(-np.pi, np.pi, (4 * cus + 1, 4)).astype(np.float32)
+    b = gvx.Batch(env, pts, sizes, dh, base, max_poses=len(q))
+    qd = torch.from_numpy(q).cuda()
+    torch.cuda.synchronize()
+    for n in (32, 33, cus, cus + 1, 3 * cus, 3 * cus + 1, 7 * cus // 2, 7 * cus // 2 + 1, 4 * cus, 4 * cus + 1):
+        b.set_schedule(2)
+        want = b.collide(q[:n])
+        assert want[0].sum() > 0
+        for s in (0, 8):
+            b.set_schedule(s)
+            c = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+            m = torch.full((n, 32), 9, dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            b.collide(qd[:n], c, m)
+            assert np.array_equal(c.cpu().numpy(), want[0].astype(np.int32)), (s, n)
+            assert np.array_equal(m.cpu().numpy(), want[1].reshape(n, 32)), (s, n)
+            chunk = 128 if n <= 32 or (sparse and cus < n <= 7 * cus // 2) else 64
+            assert b.last_stats()[0] == n * int(np.ceil(sizes / chunk).sum()), (s, n)
+            got = b.collide(q[:n])
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (s, n)
