@@ -129,7 +129,6 @@ struct CostArgs {
 // link frames of the block's waypoints into LDS: T[wp * nl + l] = base * A_0 ... A_{l-1}
 // (KinematicChain::setConfiguration, robot/dh_robot/KinematicChain.cu:93-126).  The chain is
 // serial: the block's waypoints walk theirs side by side, one lane each.
-template <uint32_t WB>
 __device__ __forceinline__ void block_fk(const CostArgs& c, uint64_t tw0, uint32_t nw, float (*A)[12], float (*T)[12])
 {
   for (uint32_t j = threadIdx.x; j < nw * c.nl; j += blockDim.x)  // rows of q are consecutive
@@ -189,7 +188,7 @@ __global__ void __launch_bounds__(64 * CMAXW) k_cost_fwd(const CostArgs c, float
   __shared__ float wsum[CMAXW][WB];
   const uint64_t tw0 = (uint64_t)blockIdx.x * WB;
   const uint32_t nw = c.n - tw0 < WB ? (uint32_t)(c.n - tw0) : WB;
-  block_fk<WB>(c, tw0, nw, A, T);
+  block_fk(c, tw0, nw, A, T);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   float acc[WB];
 #pragma unroll
@@ -254,7 +253,7 @@ __global__ void __launch_bounds__(64 * CMAXW) k_cost_bwd(const CostArgs c, const
   __shared__ float wsum[CMAXW][WB];
   const uint64_t tw0 = (uint64_t)blockIdx.x * WB;
   const uint32_t nw = c.n - tw0 < WB ? (uint32_t)(c.n - tw0) : WB;
-  block_fk<WB>(c, tw0, nw, A, T);
+  block_fk(c, tw0, nw, A, T);
   const uint32_t ns = c.nl * c.spl;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   for (uint32_t p = 0; p < nw; ++p) {
