@@ -11,9 +11,10 @@
 //     chunk of consecutive points covers a small patch with a tight bounding box;
 //   * forward kinematics runs per pose on the GPU (deterministic sin/cos);
 //   * as a rule a block evaluates a whole pose (k_batch_pose), with the voxels that it has
-//     counted in LDS.  Few poses of many points, and maps that its 32-bit keys do not
-//     reach, take (chunk, group of poses) work items instead (k_batch_collide), and the
-//     rest of this list is about those;
+//     counted in LDS.  Few poses of many points, some numbers of them in sparse
+//     environments (kernel_schedule), and maps that its 32-bit keys do not reach, take
+//     (chunk, group of poses) work items instead (k_batch_collide), and the rest of this
+//     list is about those;
 //   * one thread per pose first poses the chunk's box and drops the poses whose box
 //     reaches no occupied cell (a conservative test, so no colliding point is ever
 //     dropped), then the chunk's points, one per thread, are tested against the

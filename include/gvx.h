@@ -259,9 +259,9 @@ int gvx_batch_last_stats(gvx_batch b, uint64_t* tests, uint64_t* live_pairs, uin
 int gvx_sync(void);
 /* choose and cache the fastest launch schedule for n_poses, timed on the joint values of
    the last gvx_batch_collide call with a host-memory q.  Schedules 0-7, launched directly:
-   0 chooses by the sizes, 1-5 differ in chunk size, block size and poses per thread, 6 and 7
-   give a pose a block of 512 or 1024 threads; 8-15: the same kernels replayed from a HIP
-   graph captured per (n_poses, buffers). */
+   0 chooses by the sizes and the environment's occupied bricks, 1-5 differ in chunk size,
+   block size and poses per thread, 6 and 7 give a pose a block of 512 or 1024 threads; 8-15:
+   the same kernels replayed from a HIP graph captured per (n_poses, buffers). */
 int gvx_batch_autotune(gvx_batch b, uint32_t n_poses, int* schedule_out);
 int gvx_batch_set_schedule(gvx_batch b, int schedule);
 /* per-pose reference path on the GPU: clear a robot map, transform and insert
